@@ -43,7 +43,6 @@ constexpr int NL = 11;
 constexpr int LCIN[NL] = {8, 32, 32, 64, 64, 128, 192, 64, 96, 32, 32};
 constexpr int LCOUT[NL] = {32, 32, 64, 64, 128, 128, 64, 64, 32, 32, 3};
 constexpr int LEVEL[NL] = {1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 1};
-constexpr int WCHUNK = 2048;   // points per weight-gradient chunk
 
 int pad32(int k) { return (k + 31) / 32 * 32; }
 
@@ -70,7 +69,7 @@ struct gm_unet {
     bf16_t *g11 = nullptr, *g10 = nullptr, *g9 = nullptr, *dcat1 = nullptr, *g8 = nullptr, *g7 = nullptr;
     bf16_t *dcat2 = nullptr, *g6 = nullptr, *g5 = nullptr, *dp3 = nullptr, *g4 = nullptr, *g3 = nullptr;
     bf16_t *dp2 = nullptr, *g2 = nullptr, *g1 = nullptr;
-    float *part = nullptr, *bpart = nullptr, *tgt = nullptr;
+    float *part = nullptr, *tgt = nullptr;
     double *dpart = nullptr, *dacc = nullptr;   // 1024 + 4 doubles
     bf16_t *ds_feat = nullptr;   // [cap][P1][8]
     float *ds_tgt = nullptr;     // [cap][P1][3]
@@ -91,8 +90,6 @@ int ualloc(gm_unet *u, T **p, size_t n)
     (void)hipMemset(*p, 0, n * sizeof(T));
     return GM_OK;
 }
-
-long long nchunks(long long P) { return (P + WCHUNK - 1) / WCHUNK; }
 
 void conv(gm_unet *u, int l, const bf16_t *in, long long ldi, bf16_t *out, long long ldo, float *outf = nullptr,
           long long ldf = 0)
@@ -130,18 +127,13 @@ void wgrad(gm_unet *u, int l, const bf16_t *in, long long ldi, const bf16_t *g)
 {
     const ULayer &L = u->L[l];
     const int *n = u->n[LEVEL[l]];
-    const long long P = u->P[LEVEL[l]];
     gmu::WgradArgs a;
     a.in = in; a.ldi = ldi;
     a.g = g; a.ldg = L.coutp;
     a.nx = n[0]; a.ny = n[1]; a.nz = n[2];
     a.cin = L.cin; a.cout = L.coutp;
-    a.chunk = WCHUNK;
-    a.nchunks = (int)nchunks(P);
     a.part = u->part;
-    gmu::launch_wgrad(u->stream, a);
-    gmu::launch_wgrad_reduce(u->stream, u->part, a.nchunks, L.coutp, L.cin, L.kpad, L.g, 1);
-    gmu::launch_bias_grad(u->stream, g, L.coutp, P, L.coutp, u->bpart, L.bg, 1);
+    gmu::launch_wgrad(u->stream, a, L.kpad, L.g, L.bg);
 }
 
 void forward(gm_unet *u, const bf16_t *x0)
@@ -290,7 +282,8 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
             (r = ualloc(u, &L.bv, L.coutp)) || (r = ualloc(u, &L.bg, L.coutp)) || (r = ualloc(u, &L.w16, nw)))
             return bail(r);
         if (l > 0 && (r = ualloc(u, &L.wT, (size_t)L.cin * L.kpadT))) return bail(r);
-        part_cap = std::max(part_cap, nchunks(u->P[LEVEL[l]]) * L.coutp * 27 * L.cin);
+        const int *n = u->n[LEVEL[l]];
+        part_cap = std::max(part_cap, gmu::wgrad_part_floats(n[0], n[1], n[2], L.cin, L.coutp));
     }
     const long long P1 = u->P[1], P2 = u->P[2], P3 = u->P[3];
     int r;
@@ -304,7 +297,7 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
         (r = ualloc(u, &u->g6, P3 * 128)) || (r = ualloc(u, &u->g5, P3 * 128)) || (r = ualloc(u, &u->dp3, P3 * 64)) ||
         (r = ualloc(u, &u->g4, P2 * 64)) || (r = ualloc(u, &u->g3, P2 * 64)) || (r = ualloc(u, &u->dp2, P2 * 32)) ||
         (r = ualloc(u, &u->g2, P1 * 32)) || (r = ualloc(u, &u->g1, P1 * 32)) || (r = ualloc(u, &u->part, part_cap)) ||
-        (r = ualloc(u, &u->bpart, (size_t)gmu::bias_grad_chunks(P1) * 128)) || (r = ualloc(u, &u->tgt, P1 * 3)) ||
+        (r = ualloc(u, &u->tgt, P1 * 3)) ||
         (r = ualloc(u, &u->dpart, 1024 + (size_t)gmu::loss_blocks(P1))) || (r = ualloc(u, &u->dacc, 4)))
         return bail(r);
     if (capacity > 0) {

@@ -41,27 +41,22 @@ struct ConvArgs {
 };
 void launch_conv(hipStream_t s, const ConvArgs &a);
 
-// Weight gradient partials: part[chunk][co][t][ci] = sum over the chunk's
-// points p of g[p][co] in[p + off(t)][ci].
+// Weight and bias gradients of a layer, added to grad[co][t*cin+ci] (pitch
+// kpad) and bgrad[co]: sums over the points p of g[p][co] in[p + off(t)][ci]
+// and of g[p][co], through partials of wgrad_part_floats() values summed in
+// a fixed order.
 struct WgradArgs {
     const bf16_t *in = nullptr;
     long long ldi = 0;
     const bf16_t *g = nullptr;
     long long ldg = 0;
     int nx = 0, ny = 0, nz = 0;
-    int cin = 0, cout = 0;    // cin multiple of 8, cout multiple of 16
-    int chunk = 0;            // points per chunk (multiple of 64)
-    int nchunks = 0;
+    int cin = 0, cout = 0;    // cin 8, 16 or a multiple of 32; cout 16 or a multiple of 32
+    int nwg = 0;              // workgroups along the points (set by launch_wgrad)
     float *part = nullptr;
 };
-void launch_wgrad(hipStream_t s, const WgradArgs &a);
-// grad[co][t*cin+ci] (pitch kpad) (+)= sum over chunks in order.
-void launch_wgrad_reduce(hipStream_t s, const float *part, int nchunks, int cout, int cin, int kpad, float *grad,
-                         int accumulate);
-// bgrad[c] (+)= sum_p g[p][c], through per-chunk partials (fixed order).
-void launch_bias_grad(hipStream_t s, const bf16_t *g, long long ldg, long long P, int c, float *part, float *bgrad,
-                      int accumulate);
-int bias_grad_chunks(long long P);
+void launch_wgrad(hipStream_t s, WgradArgs a, int kpad, float *grad, float *bgrad);
+long long wgrad_part_floats(int nx, int ny, int nz, int cin, int cout);
 
 // 3x3x3 average, stride 2, padding 1, divisor 27 (nx.. fine sizes).
 void launch_pool(hipStream_t s, const bf16_t *in, long long ldi, int nx, int ny, int nz, int c, bf16_t *out,

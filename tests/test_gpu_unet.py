@@ -73,6 +73,25 @@ def test_loss_and_gradient_match_oracle(g):
         off += n
 
 
+# box edges of the kernels (boxes of 8 x 4 points and 2, 4 or 8 planes): the
+# smallest grid, one point past a box on each axis in turn, and a grid whose
+# weight-gradient workgroups each take several boxes
+@pytest.mark.parametrize("shape", [(5, 5, 5), (9, 5, 13), (5, 9, 9), (17, 13, 17), (33, 5, 9), (65, 33, 33)])
+def test_gradient_at_box_edges(g, shape):
+    import oracle as o
+    params, feat, target = case(21, shape)
+    with g.UNet(shape[2], shape[1], shape[0]) as u:
+        u.set_params(params)
+        loss, grad = u.loss_grad(feat, target)
+    l_r, _, g_r = o.unet_loss(params, feat, target, round_bf16=True)
+    assert abs(loss - l_r) < 1e-3 * l_r
+    off = 0
+    for l, (cin, cout) in enumerate(o.UNET_LAYERS):
+        n = cout * 27 * cin + cout
+        assert relerr(grad[off:off + n], g_r[off:off + n]) < 3e-2, l
+        off += n
+
+
 def relaxed_braid(g, n, steps):
     """A braid on an (n, n, 2n-1) grid relaxed by `steps` attempts (F32K)."""
     p = small_braid(n, n, 2 * n - 1)
