@@ -50,8 +50,8 @@ struct ULayer {
     int cin = 0, cout = 0, coutp = 0, kpad = 0, kpadT = 0;
     float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;   // [coutp][kpad]
     float *b = nullptr, *bm = nullptr, *bv = nullptr, *bg = nullptr; // [coutp]
-    bf16_t *w16 = nullptr;   // [coutp][kpad]
-    bf16_t *wT = nullptr;    // [cin][kpadT]: flipped transpose (input gradient)
+    bf16_t *wf = nullptr;    // packed bf16 weights (coutp * kpad)
+    bf16_t *wb = nullptr;    // packed flipped transpose, the input gradient's (cin * kpadT)
 };
 
 }  // namespace
@@ -98,13 +98,12 @@ void conv(gm_unet *u, int l, const bf16_t *in, long long ldi, bf16_t *out, long 
     const int *n = u->n[LEVEL[l]];
     gmu::ConvArgs a;
     a.in = in; a.ldi = ldi;
-    a.w = L.w16; a.kpad = L.kpad;
+    a.w = L.wf;
     a.bias = L.b;
     a.out = out; a.ldo = ldo;
     a.outf = outf; a.ldf = ldf;
     a.nx = n[0]; a.ny = n[1]; a.nz = n[2];
-    a.cin = L.cin; a.coutp = L.coutp; a.cout = L.coutp;
-    a.relu = l != NL - 1;
+    a.cin = L.cin; a.coutp = L.coutp;
     gmu::launch_conv(u->stream, a);
 }
 
@@ -115,11 +114,11 @@ void conv_bwd(gm_unet *u, int l, const bf16_t *g, const bf16_t *mask, long long 
     const int *n = u->n[LEVEL[l]];
     gmu::ConvArgs a;
     a.in = g; a.ldi = L.coutp;
-    a.w = L.wT; a.kpad = L.kpadT;
+    a.w = L.wb;
     a.out = out; a.ldo = ldo;
     a.mask = mask; a.ldm = ldm;
     a.nx = n[0]; a.ny = n[1]; a.nz = n[2];
-    a.cin = L.coutp; a.coutp = L.cin; a.cout = L.cin;
+    a.cin = L.coutp; a.coutp = L.cin;
     gmu::launch_conv(u->stream, a);
 }
 
@@ -129,7 +128,7 @@ void wgrad(gm_unet *u, int l, const bf16_t *in, long long ldi, const bf16_t *g)
     const int *n = u->n[LEVEL[l]];
     gmu::WgradArgs a;
     a.in = in; a.ldi = ldi;
-    a.g = g; a.ldg = L.coutp;
+    a.g = g;
     a.nx = n[0]; a.ny = n[1]; a.nz = n[2];
     a.cin = L.cin; a.cout = L.coutp;
     a.part = u->part;
@@ -203,8 +202,7 @@ void refresh_bf16(gm_unet *u)
 {
     for (int l = 0; l < NL; ++l) {
         ULayer &L = u->L[l];
-        gmu::launch_f32_to_bf16(u->stream, L.w, (long long)L.coutp * L.kpad, L.w16);
-        if (L.wT) gmu::launch_flip(u->stream, L.w16, L.coutp, L.cin, L.kpad, L.wT, L.kpadT);
+        gmu::launch_pack(u->stream, L.w, L.coutp, L.cin, L.kpad, L.wf, L.wb, L.kpadT);
     }
 }
 
@@ -213,10 +211,10 @@ void adam(gm_unet *u, float lr, float gscale)
     ++u->step;
     for (auto &L : u->L) {
         gmu::launch_adam(u->stream, L.w, L.g, L.m, L.v, (long long)L.coutp * L.kpad, gscale, lr, 0.9f, 0.999f, 1e-8f,
-                         u->step, L.w16);
-        gmu::launch_adam(u->stream, L.b, L.bg, L.bm, L.bv, L.coutp, gscale, lr, 0.9f, 0.999f, 1e-8f, u->step, nullptr);
-        if (L.wT) gmu::launch_flip(u->stream, L.w16, L.coutp, L.cin, L.kpad, L.wT, L.kpadT);
+                         u->step);
+        gmu::launch_adam(u->stream, L.b, L.bg, L.bm, L.bv, L.coutp, gscale, lr, 0.9f, 0.999f, 1e-8f, u->step);
     }
+    refresh_bf16(u);
 }
 
 int upload_feat(gm_unet *u, const double *feat)
@@ -279,9 +277,9 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
         int r;
         if ((r = ualloc(u, &L.w, nw)) || (r = ualloc(u, &L.m, nw)) || (r = ualloc(u, &L.v, nw)) ||
             (r = ualloc(u, &L.g, nw)) || (r = ualloc(u, &L.b, L.coutp)) || (r = ualloc(u, &L.bm, L.coutp)) ||
-            (r = ualloc(u, &L.bv, L.coutp)) || (r = ualloc(u, &L.bg, L.coutp)) || (r = ualloc(u, &L.w16, nw)))
+            (r = ualloc(u, &L.bv, L.coutp)) || (r = ualloc(u, &L.bg, L.coutp)) || (r = ualloc(u, &L.wf, nw)))
             return bail(r);
-        if (l > 0 && (r = ualloc(u, &L.wT, (size_t)L.cin * L.kpadT))) return bail(r);
+        if (l > 0 && (r = ualloc(u, &L.wb, (size_t)L.cin * L.kpadT))) return bail(r);
         const int *n = u->n[LEVEL[l]];
         part_cap = std::max(part_cap, gmu::wgrad_part_floats(n[0], n[1], n[2], L.cin, L.coutp));
     }

@@ -15,17 +15,17 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ inline float bf2f(bf16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-// float -> bfloat16, round to nearest even (NaN stays NaN)
-__device__ inline bf16_t f2bf(float f)
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// two floats -> two bfloat16 in a word, round to nearest even (NaN stays NaN)
+__device__ inline uint32_t f2bf2(float lo, float hi)
 {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (bf16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
 __device__ inline u32x4 ld16(const bf16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
@@ -43,7 +43,7 @@ __device__ inline void unpack8(u32x4 v, float *f)
 __device__ inline u32x4 pack8(const float *f)
 {
     u32x4 v;
-    for (int e = 0; e < 4; ++e) v[e] = (uint32_t)f2bf(f[2 * e]) | ((uint32_t)f2bf(f[2 * e + 1]) << 16);
+    for (int e = 0; e < 4; ++e) v[e] = f2bf2(f[2 * e], f[2 * e + 1]);
     return v;
 }
 
@@ -64,243 +64,450 @@ __device__ inline int xcd_run(int b, int n)
 }
 
 // ------------------------------------------------------------------ conv
-// Workgroup: 4 waves x 32 output points; each wave keeps 2 x NF tiles of
-// 16 x 16 FP32 accumulators.  A comes straight from global memory (16 bytes
-// per lane: 8 channels of one neighbour point), B (weights) likewise; the
-// 27-fold reuse of activations and the reuse of weights across workgroups
-// are served by the caches.
-template <int NF>
-__global__ __launch_bounds__(256) void k_conv(ConvArgs a)
+// Workgroup: a box of 8 x 4 x BZ output points (BZ = MTW WM / 2) and
+// 16 NTW WN output channels; WM waves along the points, WN along the
+// channels, each with MTW x NTW tiles of 16 points x 16 channels in FP32
+// accumulators.  The box's input with a one-point halo, all CIN channels,
+// is staged in LDS once and serves the 27 taps by constant row offsets
+// (rows outside the grid hold zeros, so no test runs per tap).  A row is 16
+// bytes longer than its channels, an odd number of 16-byte words, and a y of
+// rows is rounded up to half a turn of the banks past a whole number of
+// them: the sixteen points of a tile, eight x of two y, lie on different
+// banks.  A thread's staged words differ only in z (and y in a few steps), so
+// the grid tests cost next to nothing.  The weights come in the order the lanes take them
+// (k_pack), 1 KB a tile and step, straight from memory (L1, L2) into a ring
+// of registers kRing steps ahead.  The weights are the first operand and
+// the points the second, so a lane ends up with four consecutive channels
+// of one point and stores them in 8 bytes.
+// K runs as (tap, channel) in steps of 32 whatever the layer, one
+// accumulator per output: every output is the same sum in the same order
+// for any box.
+// What bounds it: LDS and L1 reads against the matrix pipe, about even at 32
+// output channels (MTW LDS and NTW L1 reads of 1 KB for MTW NTW matrix
+// instructions a step); at the coarsest level the few hundred workgroups.
+// 65 x 65 x 193, all layers and input gradients of a sample: 5.0 -> 1.6 ms
+// against operands loaded straight from memory per tap, with a grid test per
+// tap and lane
+constexpr int CBX = 8, CBY = 4;                   // box, z planes by the variant
+constexpr int CPX = CBX + 2, CPY = CBY + 2;       // halo points per y, y per z
+// LDS layout, in 16-byte words: a point, a y and a z of the halo
+constexpr int conv_pw(int cin) { return cin == 8 ? 1 : cin / 8 + 1; }
+constexpr int conv_yw(int cin) { return (CPX * conv_pw(cin) + 7) / 16 * 16 + 8; }
+constexpr int conv_zw(int cin) { return CPY * conv_yw(cin); }
+
+// What becomes of a sum: bias and ReLU (a layer), the bias alone in FP32 (the
+// head), nothing or the ReLU's derivative of `mask` (input gradients)
+enum ConvEnd { kRelu, kHead, kPlain, kMask };
+
+template <int CIN, int NTW, int WN, int MTW, int WM, int END>
+__global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CIN == 128 ? 2 : 3))) void k_conv(ConvArgs a)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, r16 = lane & 15;
-    const long long P = (long long)a.nx * a.ny * a.nz;
-    const long long m0 = ((long long)blockIdx.x * 4 + wave) * 32;
-    int px[2], py[2], pz[2];
-    bool pv[2];
-    for (int r = 0; r < 2; ++r) {
-        const long long p = m0 + 16 * r + r16;
-        pv[r] = p < P;
-        decomp(pv[r] ? p : 0, a.nx, a.ny, px[r], py[r], pz[r]);
-    }
-    f32x4 acc[2][NF];
-    for (int r = 0; r < 2; ++r)
-        for (int f = 0; f < NF; ++f) acc[r][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    static_assert(MTW % 2 == 0, "two tiles of 16 points make one z plane of the box");
+    constexpr int NT = 64 * WN * WM, BZ = MTW * WM / 2, KS = (27 * CIN + 31) / 32, CW = CIN / 8;
+    constexpr int PW = conv_pw(CIN), YW = conv_yw(CIN), ZW = conv_zw(CIN), ZERO = ZW * (BZ + 2);
+    static_assert(YW >= CPX * PW && YW % 16 == 8);
+    extern __shared__ u32x4 Xs[];   // [BZ + 2][CPY][CPX][PW], then two words of zeros
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, r16 = lane & 15;
+    const int wn = wave % WN, wm = wave / WN;
+    const int nbx = (a.nx + CBX - 1) / CBX, nby = (a.ny + CBY - 1) / CBY;
+    const int box = xcd_run(blockIdx.x, gridDim.x);
+    const int x0 = box % nbx * CBX, y0 = box / nbx % nby * CBY, z0 = box / (nbx * nby) * BZ;
     const u32x4 zero = {0u, 0u, 0u, 0u};
-    const bf16_t *wl = a.w + (long long)r16 * a.kpad + 8 * g;
-    for (int k0 = 0; k0 < a.kpad; k0 += 32) {
-        const int k = k0 + 8 * g;
-        const int t = k / a.cin, ci = k - t * a.cin;
-        u32x4 A[2] = {zero, zero};
-        if (t < 27) {
-            const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-            for (int r = 0; r < 2; ++r) {
-                const int qx = px[r] + dx, qy = py[r] + dy, qz = pz[r] + dz;
-                if (pv[r] && qx >= 0 && qx < a.nx && qy >= 0 && qy < a.ny && qz >= 0 && qz < a.nz)
-                    A[r] = ld16(a.in + (qx + (long long)a.nx * (qy + (long long)a.ny * qz)) * a.ldi + ci);
+
+    // this wave's weights: tile nt of step s at ((s * tiles + nt) * 64 + lane) * 8
+    const int nt0 = (blockIdx.y * WN + wn) * NTW;
+    const long long wstep = (long long)(a.coutp / 16) * 512;
+    const bf16_t *wl = a.w + ((long long)nt0 * 64 + lane) * 8;
+    // steps ahead: nine (a z plane of taps) where a step is two tiles, three
+    // where it is more; all of the few steps of 8 and 16 channels
+    constexpr int kRing = CIN < 32 ? KS : NTW <= 2 ? 9 : 3;
+    // staging: LN lanes take one y of the halo, 16 bytes each, YR of them at a time
+    constexpr int LN = CPX * CW, Y1 = NT / LN, YR = Y1 >= CPY ? Y1 / CPY * CPY : Y1 >= 3 ? 3 : Y1;
+    constexpr int NS = (CPY * (BZ + 2) + YR - 1) / YR;
+    static_assert(YR > 0 && (CPY % YR == 0 || YR % CPY == 0), "a thread's y repeats");
+    // (every lane loads, from the array's start where its point lies outside: a
+    // branch per load would wait for each)
+    u32x4 v[NS];
+    const int sy = tid / LN, sx = tid % LN / CW, sc = tid % CW, gx = x0 - 1 + sx;
+    const bool sok = sy < YR && gx >= 0 && gx < a.nx;
+    auto inside = [&](int yz) {
+        const int y = y0 - 1 + yz % CPY, z = z0 - 1 + yz / CPY;
+        return sok && yz < CPY * (BZ + 2) && y >= 0 && y < a.ny && z >= 0 && z < a.nz;
+    };
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int yz = s * YR + sy, y = y0 - 1 + yz % CPY, z = z0 - 1 + yz / CPY;
+        const long long p = gx + (long long)a.nx * (y + (long long)a.ny * z);
+        v[s] = ld16(a.in + (inside(yz) ? p * a.ldi + 8 * sc : 0));
+    }
+    // the lane's output points
+    const int ox = x0 + (r16 & 7), co = 16 * nt0 + 4 * g;
+    long long op[MTW];
+    bool ook[MTW];
+#pragma unroll
+    for (int m = 0; m < MTW; ++m) {
+        const int y = y0 + (r16 >> 3) + 2 * (m & 1), z = z0 + wm * (MTW / 2) + (m >> 1);
+        ook[m] = ox < a.nx && y < a.ny && z < a.nz;
+        op[m] = ook[m] ? ox + (long long)a.nx * (y + (long long)a.ny * z) : 0;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int yz = s * YR + sy;
+        if (sy < YR && yz < CPY * (BZ + 2)) Xs[yz * YW + sx * PW + sc] = inside(yz) ? v[s] : zero;
+    }
+    bf16x8 W[kRing][NTW];
+#pragma unroll
+    for (int s = 0; s < kRing; ++s)
+#pragma unroll
+        for (int n = 0; n < NTW; ++n) W[s][n] = as_bf(ld16(wl + s * wstep + 512 * n));
+    // the ReLU masks of the lane's outputs, ready when the sums are
+    u32x2 mask[END == kMask ? MTW : 1][NTW];
+    if constexpr (END == kMask)
+#pragma unroll
+        for (int m = 0; m < MTW; ++m)
+#pragma unroll
+            for (int n = 0; n < NTW; ++n)
+                mask[m][n] = *reinterpret_cast<const u32x2 *>(a.mask + op[m] * a.ldm + co + 16 * n);
+    if (CIN < 32 && tid < 2) Xs[ZERO + tid] = zero;
+    __syncthreads();
+
+    f32x4 acc[MTW][NTW];
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+        for (int n = 0; n < NTW; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // word of the lane's point in the wave's first tile; tile m lies two y (m & 1) and m >> 1 z on
+    const int lrow = PW * (r16 & 7) + YW * (r16 >> 3) + ZW * (wm * (MTW / 2));
+    auto mrow = [](int m) { return 2 * YW * (m & 1) + ZW * (m >> 1); };
+    if constexpr (CIN < 32) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const int t = CIN == 8 ? 4 * s + g : 2 * s + (g >> 1), c = CIN == 8 ? 0 : g & 1;
+            const int trow = PW * (t % 3) + YW * (t / 3 % 3) + ZW * (t / 9) + c;
+#pragma unroll
+            for (int m = 0; m < MTW; ++m) {
+                const bf16x8 X = as_bf(Xs[t < 27 ? lrow + mrow(m) + trow : ZERO + c]);
+#pragma unroll
+                for (int n = 0; n < NTW; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[s][n], X, acc[m][n], 0, 0, 0);
             }
         }
-        const bf16x8 A0 = as_bf(A[0]), A1 = as_bf(A[1]);
-        for (int f = 0; f < NF; ++f) {
-            const bf16x8 B = as_bf(ld16(wl + (long long)16 * f * a.kpad + k0));
-            acc[0][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A0, B, acc[0][f], 0, 0, 0);
-            acc[1][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1, B, acc[1][f], 0, 0, 0);
+    } else {
+        constexpr int CC = CIN / 32;
+        const u32x4 *xl = Xs + lrow + g;
+#pragma unroll 1
+        for (int tz = 0; tz < 3; ++tz, xl += ZW) {
+#pragma unroll
+            for (int q = 0; q < 9 * CC; ++q) {
+                const int t = q / CC, at = PW * (t % 3) + YW * (t / 3) + 4 * (q % CC);
+                bf16x8 X[MTW];
+#pragma unroll
+                for (int m = 0; m < MTW; ++m) X[m] = as_bf(xl[at + mrow(m)]);
+#pragma unroll
+                for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                    for (int n = 0; n < NTW; ++n)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[q % kRing][n], X[m], acc[m][n], 0, 0, 0);
+                const int sn = min(tz * 9 * CC + q + kRing, KS - 1);
+#pragma unroll
+                for (int n = 0; n < NTW; ++n) W[q % kRing][n] = as_bf(ld16(wl + sn * wstep + 512 * n));
+            }
         }
     }
-    for (int f = 0; f < NF; ++f) {
-        const int co = 16 * f + r16;
-        if (co >= a.cout) continue;
-        const float b = a.bias ? a.bias[co] : 0.f;
-        for (int r = 0; r < 2; ++r)
-            for (int i = 0; i < 4; ++i) {
-                const long long p = m0 + 16 * r + 4 * g + i;
-                if (p >= P) continue;
-                float v = acc[r][f][i] + b;
-                if (a.relu && !(v > 0.f)) v = 0.f;
-                if (a.mask && !(bf2f(a.mask[p * a.ldm + co]) > 0.f)) v = 0.f;
-                if (a.out) a.out[p * a.ldo + co] = f2bf(v);
-                if (a.outf) a.outf[p * a.ldf + co] = v;
+
+    f32x4 bias[NTW];
+    if constexpr (END == kRelu || END == kHead)
+#pragma unroll
+        for (int n = 0; n < NTW; ++n) bias[n] = *reinterpret_cast<const f32x4 *>(a.bias + co + 16 * n);
+#pragma unroll
+    for (int m = 0; m < MTW; ++m) {
+        if (!ook[m]) continue;
+#pragma unroll
+        for (int n = 0; n < NTW; ++n) {
+            f32x4 v = acc[m][n];
+            if constexpr (END == kRelu || END == kHead) v += bias[n];
+            if constexpr (END == kHead) {
+                *reinterpret_cast<f32x4 *>(a.outf + op[m] * a.ldf + co + 16 * n) = v;
+                continue;
             }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (END == kRelu) v[e] = v[e] > 0.f ? v[e] : 0.f;
+                if constexpr (END == kMask)
+                    v[e] = (e & 1 ? hi16(mask[m][n][e >> 1]) : lo16(mask[m][n][e >> 1])) > 0.f ? v[e] : 0.f;
+            }
+            *reinterpret_cast<u32x2 *>(a.out + op[m] * a.ldo + co + 16 * n) = u32x2{f2bf2(v[0], v[1]), f2bf2(v[2], v[3])};
+        }
     }
+}
+
+// Weights of a layer as k_conv's lanes take them, rounded to bfloat16: tile
+// nt of step s holds for lane l row 16 nt + (l & 15), k = 32 s + 8 (l >> 4)
+// .. + 7.  wf: rows co, k = t cin + ci.  wb, the input gradient's: rows ci,
+// k = t' coutp + co with the flipped tap 26 - t' (zero past 27 coutp).
+__global__ void k_pack(const float *w, int coutp, int cin, int kpad, bf16_t *wf, bf16_t *wb, int kpadT)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;   // one lane of one tile
+    const int nf = coutp * kpad / 8, nb = wb ? cin * kpadT / 8 : 0;
+    if (i >= nf + nb) return;
+    const bool fwd = i < nf;
+    const int j = fwd ? i : i - nf, tiles = (fwd ? coutp : cin) / 16;
+    const int l = j & 63, row = 16 * ((j >> 6) % tiles) + (l & 15), k = 32 * ((j >> 6) / tiles) + 8 * (l >> 4);
+    float v[8];
+    for (int e = 0; e < 8; ++e) {
+        if (fwd) {
+            v[e] = w[(long long)row * kpad + k + e];
+        } else {
+            const int t = (k + e) / coutp, co = (k + e) % coutp;
+            v[e] = t < 27 ? w[(long long)co * kpad + (26 - t) * cin + row] : 0.f;
+        }
+    }
+    st16((fwd ? wf : wb) + (long long)j * 8, pack8(v));
 }
 
 // ------------------------------------------------------------- weight grad
-// Workgroup: a run of 8 x 4 x 8 boxes of points and one block of 16 MCO
-// output by 16 NCI input channels; each of its four waves owns seven of the
-// 27 taps (the 28th is the bias gradient: the input replaced by ones) and
-// keeps their FP32 accumulators over the whole run, so a box's output
-// gradient and its input with a one-point halo are read from memory once
-// for all taps.  K runs over points: a step is the 32 points of one z plane
-// of the box.  Both operands lie in LDS point by point as in memory (16
-// channels, 32 bytes a row) and ds_read_b64_tr_b16 hands each lane four
-// consecutive points of its channel; a tap is a constant row offset, halo
-// rows outside the grid hold zeros, so there is no test per tap.  Rows of a
-// box row are 12 apart: the four rows a 16-lane group reads are 128
-// consecutive bytes and the groups' rows lie 384 bytes apart, so the reads
-// meet no bank conflict.  The next box's rows are loaded into registers
-// while the present one is multiplied.
-// What bounds it: the LDS reads (2 MCO + 14 NCI 512-byte reads for 7 MCO NCI
-// matrix instructions a step).  Weight and bias gradients of all eleven
-// layers of a 65 x 65 x 193 sample, reductions included: 13.2 -> 0.91 ms
-// against one workgroup per (2048 points, tap, 64 x 64 block), which read
-// both tensors once a tap and transposed them by 2-byte LDS stores, and
-// separate passes for the biases
-constexpr int WBX = 8, WBY = 4, WBZ = 8;           // box
-constexpr int WPX = 12;                            // rows from one y to the next
-constexpr int WHZ = WPX * (WBY + 2);               // halo rows from one z to the next
-constexpr int WXR = WHZ * (WBZ + 2), WGR = WPX * WBY * WBZ;
-constexpr int WXN = (WBX + 2) * (WBY + 2) * (WBZ + 2), WGN = WBX * WBY * WBZ;   // rows in use
+// Workgroup: one chunk of 2048 consecutive points, one z plane of nine taps
+// and one block of 16 MCO output by 16 NCI input channels; each of its three
+// waves owns the three taps of one y and keeps their FP32 accumulators over
+// the chunk, so both tensors are staged once for nine taps.  K runs over
+// points, 32 consecutive ones a step, and the chunks' partials are summed in
+// turn (k_wgrad_sum): the order of the sum depends on nothing but the grid.
+// Both operands lie in LDS point by point as in memory (16 channels, 32
+// bytes a row) and ds_read_b64_tr_b16 hands each lane four consecutive
+// points of its channel.  A wave stages the input rows of its y: those of
+// the tile's points in order, with one row of zeros from each grid row to
+// the next (x = -1 and x = nx share it) and zeros where y or z lies outside,
+// so a point's row is its index plus the grid rows begun since the tile's
+// first point, the three taps are constant row offsets, and no test runs per
+// tap.
+// What bounds it: the LDS reads (2 MCO + 6 NCI reads of 512 bytes for 3 MCO
+// NCI matrix instructions a step) beside the staging's address arithmetic
+// and latency, which the workgroups a CU holds cover.  Weight and bias
+// gradients of all eleven layers of a 65 x 65 x 193 sample, sums included:
+// 13.2 -> 1.4 ms against one workgroup per (chunk, tap, 64 x 64 block), which
+// read both tensors once a tap and transposed them by 2-byte LDS stores
+constexpr int WCHUNK = 2048;   // points a workgroup sums
+constexpr int WT = 96;         // points of a tile: 64 and 128 are 5 to 15% slower (latency; two waves a SIMD for registers)
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-// the K slice of one operand: points x 0..3 and 4..7 of the lane group's row
-__device__ inline bf16x8 ld_points(const bf16_t *p)
+__device__ inline s16x4 ld_points(const bf16_t *p)
 {
     typedef __attribute__((address_space(3))) s16x4 *lp;
-    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p));
-    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 4 * 16));
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p));
+}
+__device__ inline bf16x8 join(s16x4 a, s16x4 b)
+{
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int MCO, int NCI>
-__global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs a)
-{
-    extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
-    bf16_t *Xs = lds, *Gs = lds + NCI * WXR * 16;
-    constexpr int NX = (WXN * 2 * NCI + 255) / 256, NG = WGN * 2 * MCO / 256;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, r16 = lane & 15;
-    const int nciB = (a.cin + 16 * NCI - 1) / (16 * NCI);
-    const int co0 = (int)(blockIdx.y / nciB) * 16 * MCO, ci0 = (int)(blockIdx.y % nciB) * 16 * NCI;
-    const int nbx = (a.nx + WBX - 1) / WBX, nby = (a.ny + WBY - 1) / WBY, nbz = (a.nz + WBZ - 1) / WBZ;
-    const int nbox = nbx * nby * nbz;
-    const int wg = xcd_run(blockIdx.x, a.nwg);
-    const int beg = (int)((long long)wg * nbox / a.nwg), end = (int)((long long)(wg + 1) * nbox / a.nwg);
-    const u32x4 zero = {0u, 0u, 0u, 0u};
+// Input rows of a tile and y: the points, a row of zeros per grid row begun,
+// and one row on either side
+__host__ __device__ inline int wgrad_rows(int nx) { return WT + (WT - 1) / nx + 3; }
 
-    // the thread's slots, recomputed for each box: kept across the boxes their
-    // coordinates would take the registers of the accumulators
-    auto slot0 = [&]() {
-        int q = tid;
-        asm volatile("" : "+v"(q));
-        return q;
-    };
-    u32x4 xr[NX], gr[NG];
-    auto load = [&](int box) {
-        const int q0 = slot0();
-        const int x0 = box % nbx * WBX, y0 = box / nbx % nby * WBY, z0 = box / (nbx * nby) * WBZ;
+// floor(v / n) of 0 <= v < 2^16 with inv = 1 / n: v + 1/2 is at least 1/(2n)
+// away from a multiple of n, relative to the quotient more than the rounding
+__device__ inline int small_div(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
+
+template <int MCO, int NCI>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_wgrad(WgradArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) bf16_t lds[];   // [3][NCI][rows][16] input, [MCO][WT][16] gradient, [3][rows] int
+    const int rows = wgrad_rows(a.nx), xn = rows * 16;
+    constexpr int gn = WT * 16;
+    const int tid = threadIdx.x, lane = tid & 63, ty = tid >> 6, g = lane >> 4, r16 = lane & 15;
+    bf16_t *Xs = lds + ty * NCI * xn, *Gs = lds + 3 * NCI * xn;
+    const int tz = blockIdx.y % 3, blk = blockIdx.y / 3;
+    const int nciB = (a.cin + 16 * NCI - 1) / (16 * NCI);
+    const int co0 = blk / nciB * 16 * MCO, ci0 = blk % nciB * 16 * NCI;
+    const int P = a.nx * a.ny * a.nz;
+    const int chunk = xcd_run(blockIdx.x, gridDim.x);
+    const int pbeg = chunk * WCHUNK, pend = min(pbeg + WCHUNK, P);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    const float invx = 1.f / (float)(a.nx + 1), invx0 = 1.f / (float)a.nx, invy = 1.f / (float)a.ny;
+
+    f32x4 acc[3][MCO][NCI];
 #pragma unroll
-        for (int j = 0; j < NX; ++j) {
-            const int q = q0 + 256 * j, row = q / (2 * NCI), ci = ci0 + 8 * (q % (2 * NCI));
-            const int x = x0 - 1 + row % (WBX + 2), y = y0 - 1 + row / (WBX + 2) % (WBY + 2);
-            const int z = z0 - 1 + row / ((WBX + 2) * (WBY + 2));
-            xr[j] = zero;
-            if (row < WXN && ci < a.cin && x >= 0 && x < a.nx && y >= 0 && y < a.ny && z >= 0 && z < a.nz)
-                xr[j] = ld16(a.in + (x + (long long)a.nx * (y + (long long)a.ny * z)) * a.ldi + ci);
+    for (int j = 0; j < 3; ++j)
+        for (int m = 0; m < MCO; ++m)
+            for (int n = 0; n < NCI; ++n) acc[j][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int lch = 4 * (r16 & 3), lpt = 8 * g + (r16 >> 2);
+    const int sc = lane % (2 * NCI), sr = lane / (2 * NCI);   // staging: 8-channel group and first row
+    const bool cok = ci0 + 8 * sc < a.cin;
+    const bf16_t *src = a.in + ci0 + 8 * sc;
+    bf16_t *xst = Xs + (sc >> 1) * xn + 8 * (sc & 1);
+    constexpr int RS = 32 / NCI;                              // rows a wave stages at a time
+    // a tile's words on their way to LDS: loaded while the tile before is multiplied
+    constexpr int NX = (WT + (WT - 1) / 5 + 3 + RS - 1) / RS, NG = (WT * 2 * MCO + 191) / 192;   // grids have nx >= 5
+    u32x4 xv[NX], gv[NG];
+    int *const tab = reinterpret_cast<int *>(lds + (3 * NCI * xn + MCO * gn)) + ty * rows;   // the wave's
+    auto load = [&](int pb) {
+        // the grid points of the rows (-1: zeros), one row a lane: worked out by
+        // every lane for the rows it loads, this arithmetic took longer than the
+        // matrix instructions
+        const int rb = pb / a.nx, xb = pb - rb * a.nx, yb = rb % a.ny;   // first point: grid row, x and y
+        for (int r = lane; r < rows; r += 64) {
+            // row r is x = xb - 1 + r, counted on over rows of nx + 1
+            const int X = xb + a.nx + r, q = small_div(X, invx), x = X - q * (a.nx + 1);
+            const int Y = yb + q - 1 + a.ny, y = Y - small_div(Y, invy) * a.ny + ty - 1;   // q - 1 >= -1
+            const int p = x + a.nx * (rb + q - 1 + ty - 1 + (tz - 1) * a.ny);
+            tab[r] = x < a.nx && y >= 0 && y < a.ny && p >= 0 && p < P ? p : -1;
+        }
+        int p[NX];
+#pragma unroll
+        for (int u = 0; u < NX; ++u) p[u] = tab[min(sr + u * RS, rows - 1)];
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            xv[u] = zero;
+            if (cok && p[u] >= 0) xv[u] = ld16(src + p[u] * a.ldi);
         }
 #pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            const int q = q0 + 256 * j, row = q / (2 * MCO), co = co0 + 8 * (q % (2 * MCO));
-            const int x = x0 + row % WBX, y = y0 + row / WBX % WBY, z = z0 + row / (WBX * WBY);
-            gr[j] = zero;
-            if (x < a.nx && y < a.ny && z < a.nz)
-                gr[j] = ld16(a.g + (x + (long long)a.nx * (y + (long long)a.ny * z)) * a.ldg + co);
+        for (int u = 0; u < NG; ++u) {
+            const int q = tid + 192 * u, i = q / (2 * MCO), c = q % (2 * MCO), p = pb + i;
+            gv[u] = zero;
+            if (i < WT && p < pend) gv[u] = ld16(a.g + (long long)p * a.cout + co0 + 8 * c);
         }
     };
     auto store = [&]() {
-        const int q0 = slot0();
 #pragma unroll
-        for (int j = 0; j < NX; ++j) {
-            const int q = q0 + 256 * j, row = q / (2 * NCI), c = q % (2 * NCI);
-            const int at = row % (WBX + 2) + WPX * (row / (WBX + 2) % (WBY + 2)) + WHZ * (row / ((WBX + 2) * (WBY + 2)));
-            if (row < WXN) st16(Xs + ((c >> 1) * WXR + at) * 16 + 8 * (c & 1), xr[j]);
-        }
+        for (int u = 0; u < NX; ++u)
+            if (sr + u * RS < rows) st16(xst + (sr + u * RS) * 16, xv[u]);
 #pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            const int q = q0 + 256 * j, row = q / (2 * MCO), c = q % (2 * MCO);
-            const int at = row % WBX + WPX * (row / WBX);
-            st16(Gs + ((c >> 1) * WGR + at) * 16 + 8 * (c & 1), gr[j]);
+        for (int u = 0; u < NG; ++u) {
+            const int q = tid + 192 * u, i = q / (2 * MCO), c = q % (2 * MCO);
+            if (i < WT) st16(Gs + (c >> 1) * gn + i * 16 + 8 * (c & 1), gv[u]);
         }
     };
-
-    int toff[7];   // LDS element offset of the wave's taps
-#pragma unroll
-    for (int j = 0; j < 7; ++j) {
-        const int t = min(7 * wave + j, 26);
-        toff[j] = 16 * (t % 3 + WPX * (t / 3 % 3) + WHZ * (t / 9));
-    }
-    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-    f32x4 acc[7][MCO][NCI];
-#pragma unroll
-    for (int j = 0; j < 7; ++j)
-        for (int m = 0; m < MCO; ++m)
-            for (int n = 0; n < NCI; ++n) acc[j][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int lrow = 16 * ((r16 >> 2) + WPX * g) + 4 * (r16 & 3);
-    if (beg < end) load(beg);
-    for (int box = beg; box < end; ++box) {
+    load(pbeg);
+    for (int pb = pbeg; pb < pend; pb += WT) {
+        const int xb = pb % a.nx;
         __syncthreads();
         store();
         __syncthreads();
-        if (box + 1 < end) load(box + 1);
-#pragma unroll 1
-        for (int kz = 0; kz < WBZ; ++kz) {
+        if (pb + WT < pend) load(pb + WT);
+        auto step = [&](int s) {
+            const int i = 32 * s + lpt;   // the lane's points i, i + 4
+            const bf16_t *x1 = Xs + lch + 16 * (i + small_div(xb + i, invx0));
+            const bf16_t *x2 = Xs + lch + 16 * (i + 4 + small_div(xb + i + 4, invx0));
+            const bf16_t *gp = Gs + lch + 16 * i;
             bf16x8 A[MCO];
 #pragma unroll
-            for (int m = 0; m < MCO; ++m) A[m] = ld_points(Gs + m * WGR * 16 + 16 * WPX * WBY * kz + lrow);
+            for (int m = 0; m < MCO; ++m) A[m] = join(ld_points(gp + m * gn), ld_points(gp + m * gn + 64));
 #pragma unroll
-            for (int j = 0; j < 7; ++j) {
+            for (int n = 0; n < NCI; ++n) {
 #pragma unroll
-                for (int n = 0; n < NCI; ++n) {
-                    bf16x8 B = ld_points(Xs + n * WXR * 16 + 16 * WHZ * kz + lrow + toff[j]);
-                    if (j == 6 && wave == 3) B = ones;
+                for (int j = 0; j < 3; ++j) {
+                    const bf16x8 B = join(ld_points(x1 + n * xn + 16 * j), ld_points(x2 + n * xn + 16 * j));
 #pragma unroll
                     for (int m = 0; m < MCO; ++m)
                         acc[j][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], B, acc[j][m][n], 0, 0, 0);
                 }
             }
-        }
+        };
+        const int steps = (min(WT, pend - pb) + 31) / 32;
+#pragma unroll 1
+        for (int s = 0; s < steps; ++s) step(s);
     }
-    float *part = a.part + ((long long)blockIdx.y * a.nwg + wg) * (28 * MCO * NCI * 256);
+    float *part = a.part + ((long long)blk * gridDim.x + chunk) * (27 * MCO * NCI * 256);
 #pragma unroll
-    for (int j = 0; j < 7; ++j)
+    for (int j = 0; j < 3; ++j)
 #pragma unroll
         for (int m = 0; m < MCO; ++m)
 #pragma unroll
             for (int n = 0; n < NCI; ++n)
-                *reinterpret_cast<f32x4 *>(part + (((7 * wave + j) * MCO + m) * NCI + n) * 256 + 4 * lane) = acc[j][m][n];
+                *reinterpret_cast<f32x4 *>(part + (((9 * tz + 3 * ty + j) * MCO + m) * NCI + n) * 256 + 4 * lane) = acc[j][m][n];
 }
 
-// Sum of the workgroups' partials in a fixed order, added to the layer's
-// weight and bias gradients: 32 groups of four values a workgroup, eight
-// threads along the partials of each (one thread a value walked up to 400
-// partials by itself before)
-template <int MCO, int NCI>
-__global__ __launch_bounds__(256) void k_wgrad_reduce(WgradArgs a, int kpad, float *grad, float *bgrad)
+// Bias gradient partials of 4096 points, ph = 256 / c threads a channel:
+// thread k sums the points k, k + ph, ... in turn, and the ph sums are added
+// in turn.  A workgroup takes 32 channels and stages 512 points of them in
+// LDS at a time, 16 bytes a lane: one chain of 2-byte loads a thread had
+// taken 224 us a layer on average at 65 x 65 x 193
+constexpr int BG_CHUNK = 4096, BG_PTS = 512, BG_CH = 32;
+
+__global__ __launch_bounds__(256) void k_bias_part(const bf16_t *g, int P, int c, float *part)
 {
-    __shared__ f32x4 red[8][32];
-    constexpr int N4 = 28 * MCO * NCI * 64;
-    const int col = threadIdx.x & 31, sl = threadIdx.x >> 5;
-    const int i = blockIdx.x * 32 + col;
-    const float *p = a.part + (long long)blockIdx.y * a.nwg * (4 * N4) + 4 * i;
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    __shared__ __attribute__((aligned(16))) bf16_t st[BG_PTS * BG_CH];
+    __shared__ float red[256];
+    const int w = c < BG_CH ? c : BG_CH, ph = 256 / c, ch = threadIdx.x % w, k = threadIdx.x / w, c0 = blockIdx.y * BG_CH;
+    const int p0 = blockIdx.x * BG_CHUNK, p1 = min(p0 + BG_CHUNK, P);
+    float s = 0.f;
+    for (int pb = p0; pb < p1; pb += BG_PTS) {
+        const int n = min(BG_PTS, p1 - pb);
+        __syncthreads();
 #pragma unroll 8
-    for (int w = sl; w < a.nwg; w += 8) s += *reinterpret_cast<const f32x4 *>(p + (long long)w * (4 * N4));
-    red[sl][col] = s;
-    __syncthreads();
-    if (sl) return;
+        for (int q = threadIdx.x; q < n * (w / 8); q += 256) {
+            const int i = q / (w / 8), e = q % (w / 8);
+            st16(st + 8 * q, ld16(g + (long long)(pb + i) * c + c0 + 8 * e));
+        }
+        __syncthreads();
+        if (k < ph) {
+            int i = k;
+            for (; i + 15 * ph < n; i += 16 * ph) {
+                bf16_t v[16];
 #pragma unroll
-    for (int q = 1; q < 8; ++q) s += red[q][col];
-    const int lane = i & 63, n = (i >> 6) % NCI, m = (i >> 6) / NCI % MCO, t = (i >> 6) / (NCI * MCO);
-    const int nciB = (a.cin + 16 * NCI - 1) / (16 * NCI);
-    const int co = ((int)(blockIdx.y / nciB) * MCO + m) * 16 + 4 * (lane >> 4);
-    const int ci = ((int)(blockIdx.y % nciB) * NCI + n) * 16 + (lane & 15);
-    if (t < 27) {
-        if (ci < a.cin)
+                for (int u = 0; u < 16; ++u) v[u] = st[(i + u * ph) * w + ch];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) grad[(long long)(co + e) * kpad + t * a.cin + ci] += s[e];
-    } else if (ci == 0) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bgrad[co + e] += s[e];
+                for (int u = 0; u < 16; ++u) s += bf2f(v[u]);
+            }
+            for (; i < n; i += ph) s += bf2f(st[i * w + ch]);
+        }
     }
+    if (k < ph) red[threadIdx.x] = s;
+    __syncthreads();
+    if (k == 0) {
+        for (int j = 1; j < ph; ++j) s += red[j * w + ch];
+        part[(long long)blockIdx.x * c + c0 + ch] = s;
+    }
+}
+
+// Sums of partials in turn, added to the layer's weight gradient, and (the
+// last workgroups of the grid) to its bias gradient: 64 values a workgroup;
+// its 256 threads load 64 partials of each into LDS, and one wave adds them
+// in order while the next 64 are on their way
+template <int MCO, int NCI>
+__global__ __launch_bounds__(256) void k_wgrad_sum(WgradArgs a, int nchunks, int kpad, float *grad, const float *bpart,
+                                                   int nbparts, float *bgrad)
+{
+    __shared__ float st[2][64][64];
+    constexpr int N = 27 * MCO * NCI * 256;
+    const int col = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const bool bias = blockIdx.x == N / 64;
+    const int i = blockIdx.x * 64 + col, bi = blockIdx.y * 64 + col;
+    if (bias && (int)blockIdx.y * 64 >= a.cout) return;
+    const int n = bias ? nbparts : nchunks;
+    const long long ld = bias ? a.cout : N;
+    const bool live = !bias || bi < a.cout;
+    const float *p = bias ? bpart + bi : a.part + (long long)blockIdx.y * nchunks * N + i;
+    float v[16], s = 0.f;
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int c = c0 + 4 * u + q;
+            v[u] = live && c < n ? p[c * ld] : 0.f;
+        }
+    };
+    load(0);
+    for (int c0 = 0, b = 0; c0 < n; c0 += 64, b ^= 1) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) st[b][4 * u + q][col] = v[u];
+        __syncthreads();
+        if (c0 + 64 < n) load(c0 + 64);
+        if (q == 0) {
+            const int m = min(64, n - c0);
+#pragma unroll 16
+            for (int c = 0; c < m; ++c) s += st[b][c][col];
+        }
+    }
+    if (q || !live) return;
+    if (bias) {
+        bgrad[bi] += s;
+        return;
+    }
+    const int e = i & 3, lane = i >> 2 & 63, m = (i >> 8) / NCI % MCO, nn = (i >> 8) % NCI, t = (i >> 8) / (NCI * MCO);
+    const int nciB = (a.cin + 16 * NCI - 1) / (16 * NCI);
+    const int co = ((int)(blockIdx.y / nciB) * MCO + m) * 16 + 4 * (lane >> 4) + e;
+    const int ci = ((int)(blockIdx.y % nciB) * NCI + nn) * 16 + (lane & 15);
+    if (ci < a.cin) grad[(long long)co * kpad + t * a.cin + ci] += s;
 }
 
 // ------------------------------------------------------------ pool / up
@@ -458,7 +665,7 @@ __global__ void k_loss_final(const double *part, int n, long long P, double *acc
 }
 
 __global__ void k_adam(float *w, const float *g, float *m, float *v, long long n, float gscale, float lr, float b1,
-                       float b2, float eps, float c1, float c2, bf16_t *w16)
+                       float b2, float eps, float c1, float c2)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -467,26 +674,13 @@ __global__ void k_adam(float *w, const float *g, float *m, float *v, long long n
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    const float wi = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-    w[i] = wi;
-    if (w16) w16[i] = f2bf(wi);
-}
-
-__global__ void k_flip(const bf16_t *w16, int coutp, int cin, int kpad, bf16_t *wT, int kpadT)
-{
-    const long long n = (long long)cin * 27 * coutp;
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int co = (int)(i % coutp);
-    const int tp = (int)((i / coutp) % 27);
-    const int ci = (int)(i / (27LL * coutp));
-    wT[(long long)ci * kpadT + tp * coutp + co] = w16[(long long)co * kpad + (26 - tp) * cin + ci];
+    w[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
 __global__ void k_f2b(const float *in, long long n, bf16_t *out)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = f2bf(in[i]);
+    if (i < n) out[i] = (bf16_t)f2bf2(in[i], 0.f);
 }
 
 // ------------------------------------------------- context <-> network
@@ -638,33 +832,53 @@ inline unsigned nblk(long long n, int t = 256) { return (unsigned)((n + t - 1) /
 
 }  // namespace
 
-void launch_conv(hipStream_t s, const ConvArgs &a)
+namespace {
+template <int CIN, int NTW, int WN, int MTW, int WM, int END>
+void launch_conv_k(hipStream_t s, const ConvArgs &a)
 {
-    const long long P = (long long)a.nx * a.ny * a.nz;
-    const unsigned grid = (unsigned)((P + 127) / 128);
-    switch (a.coutp) {
-    case 16: k_conv<1><<<grid, 256, 0, s>>>(a); break;
-    case 32: k_conv<2><<<grid, 256, 0, s>>>(a); break;
-    case 64: k_conv<4><<<grid, 256, 0, s>>>(a); break;
-    case 96: k_conv<6><<<grid, 256, 0, s>>>(a); break;
-    case 128: k_conv<8><<<grid, 256, 0, s>>>(a); break;
-    case 192: k_conv<12><<<grid, 256, 0, s>>>(a); break;
-    default: break;   // the host validates coutp
+    constexpr int BZ = MTW * WM / 2, lds = 16 * (conv_zw(CIN) * (BZ + 2) + 2);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k_conv<CIN, NTW, WN, MTW, WM, END>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)attr;
+    const int boxes = ((a.nx + CBX - 1) / CBX) * ((a.ny + CBY - 1) / CBY) * ((a.nz + BZ - 1) / BZ);
+    k_conv<CIN, NTW, WN, MTW, WM, END><<<dim3(boxes, a.coutp / (16 * NTW * WN)), 64 * WN * WM, lds, s>>>(a);
+}
+}  // namespace
+
+// The network's layers and their input gradients: boxes of eight planes
+// while the halo fits three workgroups a CU (32 channels, 54 KB of 160), of
+// four or two above that; channels split over two waves, or two workgroups,
+// where the box has few tiles of points
+int launch_conv(hipStream_t s, const ConvArgs &a)
+{
+    const bool fwd = a.bias != nullptr;
+    switch (a.cin * 1000 + a.coutp) {
+    case 8032: launch_conv_k<8, 2, 1, 4, 4, kRelu>(s, a); return 0;
+    case 16032: launch_conv_k<16, 2, 1, 4, 4, kMask>(s, a); return 0;
+    case 32016: launch_conv_k<32, 1, 1, 4, 4, kHead>(s, a); return 0;
+    case 32032:
+        fwd ? launch_conv_k<32, 2, 1, 4, 4, kRelu>(s, a) : launch_conv_k<32, 2, 1, 4, 4, kMask>(s, a);
+        return 0;
+    case 32064: launch_conv_k<32, 4, 1, 4, 4, kRelu>(s, a); return 0;
+    case 32096: launch_conv_k<32, 3, 2, 4, 2, kPlain>(s, a); return 0;
+    case 64032: launch_conv_k<64, 2, 1, 2, 4, kPlain>(s, a); return 0;
+    case 64064:
+        fwd ? launch_conv_k<64, 2, 2, 4, 2, kRelu>(s, a) : launch_conv_k<64, 2, 2, 4, 2, kMask>(s, a);
+        return 0;
+    case 64128: launch_conv_k<64, 2, 2, 4, 2, kRelu>(s, a); return 0;
+    case 64192: launch_conv_k<64, 3, 2, 4, 2, kPlain>(s, a); return 0;
+    case 96032: launch_conv_k<96, 2, 1, 2, 4, kRelu>(s, a); return 0;
+    case 128064: launch_conv_k<128, 2, 2, 2, 2, kPlain>(s, a); return 0;
+    case 128128:
+        fwd ? launch_conv_k<128, 2, 2, 2, 2, kRelu>(s, a) : launch_conv_k<128, 2, 2, 2, 2, kMask>(s, a);
+        return 0;
+    case 192064: launch_conv_k<192, 2, 2, 2, 4, kRelu>(s, a); return 0;
     }
+    return -1;   // no layer of the network
 }
 
 namespace {
-template <int MCO, int NCI>
-void launch_wgrad_k(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad)
-{
-    constexpr int lds = (NCI * WXR + MCO * WGR) * 16 * (int)sizeof(bf16_t);
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_wgrad<MCO, NCI>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)attr;
-    const int blocks = (a.cout / (16 * MCO)) * ((a.cin + 16 * NCI - 1) / (16 * NCI));
-    k_wgrad<MCO, NCI><<<dim3(a.nwg, blocks), 256, lds, s>>>(a);
-    k_wgrad_reduce<MCO, NCI><<<dim3(28 * MCO * NCI * 2, blocks), 256, 0, s>>>(a, kpad, grad, bgrad);
-}
+int wgrad_chunks(long long P) { return (int)((P + WCHUNK - 1) / WCHUNK); }
 // channel blocks: 32 x 32, 16 wide where the layer has no more
 int wgrad_mco(int cout) { return cout % 32 ? 1 : 2; }
 int wgrad_nci(int cin) { return cin <= 16 ? 1 : 2; }
@@ -673,25 +887,29 @@ int wgrad_blocks(int cin, int cout)
     const int nci = 16 * wgrad_nci(cin);
     return cout / (16 * wgrad_mco(cout)) * ((cin + nci - 1) / nci);
 }
-}  // namespace
-
-// Workgroups along the points: about 512 for all channel blocks (two a CU by
-// their LDS), at most one a box
-int wgrad_groups(int nx, int ny, int nz, int cin, int cout)
+template <int MCO, int NCI>
+void launch_wgrad_k(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad)
 {
-    const int nbox = ((nx + WBX - 1) / WBX) * ((ny + WBY - 1) / WBY) * ((nz + WBZ - 1) / WBZ);
-    return std::max(1, std::min(nbox, 512 / wgrad_blocks(cin, cout)));
+    const int lds = (3 * NCI * wgrad_rows(a.nx) + MCO * WT) * 32 + 3 * wgrad_rows(a.nx) * 4;   // at most 40 KB
+    const long long P = (long long)a.nx * a.ny * a.nz;
+    const int nch = wgrad_chunks(P), blocks = wgrad_blocks(a.cin, a.cout), nb = (int)((P + BG_CHUNK - 1) / BG_CHUNK);
+    float *bpart = a.part + (long long)nch * blocks * 27 * MCO * NCI * 256;
+    k_wgrad<MCO, NCI><<<dim3(nch, 3 * blocks), 192, lds, s>>>(a);
+    k_bias_part<<<dim3(nb, (a.cout + BG_CH - 1) / BG_CH), 256, 0, s>>>(a.g, (int)P, a.cout, bpart);
+    k_wgrad_sum<MCO, NCI><<<dim3(27 * MCO * NCI * 4 + 1, blocks), 256, 0, s>>>(
+        a, nch, kpad, grad, bpart, nb, bgrad);
 }
+}  // namespace
 
 long long wgrad_part_floats(int nx, int ny, int nz, int cin, int cout)
 {
-    return (long long)wgrad_groups(nx, ny, nz, cin, cout) * wgrad_blocks(cin, cout) * 28 * wgrad_mco(cout) *
-           wgrad_nci(cin) * 256;
+    const long long P = (long long)nx * ny * nz;
+    return (long long)wgrad_chunks(P) * wgrad_blocks(cin, cout) * 27 * wgrad_mco(cout) * wgrad_nci(cin) * 256 +
+           (P + BG_CHUNK - 1) / BG_CHUNK * cout;
 }
 
-void launch_wgrad(hipStream_t s, WgradArgs a, int kpad, float *grad, float *bgrad)
+void launch_wgrad(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad)
 {
-    a.nwg = wgrad_groups(a.nx, a.ny, a.nz, a.cin, a.cout);
     if (wgrad_mco(a.cout) == 1) {
         if (wgrad_nci(a.cin) == 1) launch_wgrad_k<1, 1>(s, a, kpad, grad, bgrad);
         else launch_wgrad_k<1, 2>(s, a, kpad, grad, bgrad);
@@ -740,16 +958,17 @@ void launch_loss(hipStream_t s, const float *y, const float *target, float inv_s
 }
 
 void launch_adam(hipStream_t s, float *w, const float *g, float *m, float *v, long long n, float gscale, float lr,
-                 float b1, float b2, float eps, int step, bf16_t *w16)
+                 float b1, float b2, float eps, int step)
 {
     const float c1 = (float)(1.0 / (1.0 - std::pow((double)b1, step)));
     const float c2 = (float)(1.0 / (1.0 - std::pow((double)b2, step)));
-    k_adam<<<nblk(n), 256, 0, s>>>(w, g, m, v, n, gscale, lr, b1, b2, eps, c1, c2, w16);
+    k_adam<<<nblk(n), 256, 0, s>>>(w, g, m, v, n, gscale, lr, b1, b2, eps, c1, c2);
 }
 
-void launch_flip(hipStream_t s, const bf16_t *w16, int coutp, int cin, int kpad, bf16_t *wT, int kpadT)
+void launch_pack(hipStream_t s, const float *w, int coutp, int cin, int kpad, bf16_t *wf, bf16_t *wb, int kpadT)
 {
-    k_flip<<<nblk((long long)cin * 27 * coutp), 256, 0, s>>>(w16, coutp, cin, kpad, wT, kpadT);
+    k_pack<<<nblk(((long long)coutp * kpad + (wb ? (long long)cin * kpadT : 0)) / 8), 256, 0, s>>>(w, coutp, cin, kpad,
+                                                                                              wf, wb, kpadT);
 }
 
 void launch_f32_to_bf16(hipStream_t s, const float *in, long long n, bf16_t *out)

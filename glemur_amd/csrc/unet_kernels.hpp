@@ -17,15 +17,15 @@ namespace gmu {
 using bf16_t = uint16_t;
 
 // out[p][co] = bias[co] + sum_k in[p + off(t)][ci] W[co][k] (zero padding),
-// then optional ReLU, optional mask (value kept where mask[p][co] > 0),
-// stored as bf16 (out) or fp32 (outf); channels co >= cout are not stored.
+// for a layer (with a bias) then the ReLU, for an input gradient the mask if
+// there is one (value kept where mask[p][co] > 0), stored as bf16 (out); the
+// head (16 rows) stores the sum and bias as fp32 (outf).
 // With W the flipped transpose of a layer's weights this is the layer's
 // input gradient.
 struct ConvArgs {
     const bf16_t *in = nullptr;
     long long ldi = 0;
-    const bf16_t *w = nullptr;
-    int kpad = 0;
+    const bf16_t *w = nullptr;   // packed by launch_pack
     const float *bias = nullptr;
     bf16_t *out = nullptr;
     long long ldo = 0;
@@ -35,11 +35,11 @@ struct ConvArgs {
     long long ldm = 0;
     int nx = 0, ny = 0, nz = 0;
     int cin = 0;      // multiple of 8
-    int coutp = 0;    // rows of W: 16, 32, 64, 96, 128 or 192
-    int cout = 0;     // channels stored (<= coutp)
-    int relu = 0;
+    int coutp = 0;    // rows of W, all stored
 };
-void launch_conv(hipStream_t s, const ConvArgs &a);
+// 0, or -1 when (cin, coutp) is neither a layer of the network nor the
+// input gradient of one
+int launch_conv(hipStream_t s, const ConvArgs &a);
 
 // Weight and bias gradients of a layer, added to grad[co][t*cin+ci] (pitch
 // kpad) and bgrad[co]: sums over the points p of g[p][co] in[p + off(t)][ci]
@@ -48,14 +48,12 @@ void launch_conv(hipStream_t s, const ConvArgs &a);
 struct WgradArgs {
     const bf16_t *in = nullptr;
     long long ldi = 0;
-    const bf16_t *g = nullptr;
-    long long ldg = 0;
+    const bf16_t *g = nullptr;   // [P][cout]
     int nx = 0, ny = 0, nz = 0;
     int cin = 0, cout = 0;    // cin 8, 16 or a multiple of 32; cout 16 or a multiple of 32
-    int nwg = 0;              // workgroups along the points (set by launch_wgrad)
     float *part = nullptr;
 };
-void launch_wgrad(hipStream_t s, WgradArgs a, int kpad, float *grad, float *bgrad);
+void launch_wgrad(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad);
 long long wgrad_part_floats(int nx, int ny, int nz, int cin, int cout);
 
 // 3x3x3 average, stride 2, padding 1, divisor 27 (nx.. fine sizes).
@@ -80,11 +78,14 @@ int loss_blocks(long long P);
 
 // Adam (Kingma & Ba 2015) on n master weights: m = b1 m + (1-b1) g',
 // v = b2 v + (1-b2) g'^2, w -= lr mhat / (sqrt(vhat) + eps), with
-// g' = g * gscale; w16 = bf16(w) when w16 != null.
+// g' = g * gscale.
 void launch_adam(hipStream_t s, float *w, const float *g, float *m, float *v, long long n, float gscale, float lr,
-                 float b1, float b2, float eps, int step, bf16_t *w16);
-// wT[ci][t'*coutp + co] = w16[co][(26 - t')*cin + ci] (pitch kpadT).
-void launch_flip(hipStream_t s, const bf16_t *w16, int coutp, int cin, int kpad, bf16_t *wT, int kpadT);
+                 float b1, float b2, float eps, int step);
+// A layer's weights rounded to bf16 in the order of the convolution's lanes:
+// wf (coutp * kpad values) for the layer, wb (cin * kpadT, or null) for its
+// input gradient, the flipped transpose W[co][(26 - t') cin + ci] at row ci,
+// k = t' coutp + co.
+void launch_pack(hipStream_t s, const float *w, int coutp, int cin, int kpad, bf16_t *wf, bf16_t *wb, int kpadT);
 void launch_f32_to_bf16(hipStream_t s, const float *in, long long n, bf16_t *out);
 void launch_zero(hipStream_t s, void *p, long long bytes);
 
