@@ -75,5 +75,69 @@ __device__ __forceinline__ void ghost_b(const Geo &g, const GhostPt &G, int face
     else ghost_b_f<2>(g, G, side, xin, B, det);
 }
 
+// floor(v / n) of 0 <= v < 4096, n <= 64 with inv = 1 / n to a few ulp: v + 1/2
+// is 1/(2n) away from a multiple of n, the product's error below 2e-5
+__device__ __forceinline__ int small_div(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
+
+// The points of a block launch a thread computes: output point and face
+// neighbour of a bw x bh x bd block, in box coordinates (the block starts at
+// 2); threads without one repeat the last.
+struct BlockRole {
+    bool own, ring;
+    int oc, orr, oz, rc, rr, rz;
+};
+__device__ __forceinline__ BlockRole block_role(int t, int bw, int bh, int bd)
+{
+    BlockRole b;
+    const float iw = __builtin_amdgcn_rcpf((float)bw), ih = __builtin_amdgcn_rcpf((float)bh);
+    const int np = bw * bh * bd, fx = bh * bd, fy = bw * bd, fz = bw * bh, nr = 2 * (fx + fy + fz);
+    b.own = t < np;
+    b.ring = t < nr;
+    const int v = min(t, np - 1), vy = small_div(v, iw), vz = small_div(vy, ih);
+    b.oc = 2 + v - vy * bw;
+    b.orr = 2 + vy - vz * bh;
+    b.oz = 2 + vz;
+    // faces x- x+ y- y+ z- z+
+    int u = min(t, nr - 1);
+    const int axis = u < 2 * fx ? 0 : u < 2 * (fx + fy) ? 1 : 2;
+    u -= axis == 0 ? 0 : axis == 1 ? 2 * fx : 2 * (fx + fy);
+    const int f = axis == 0 ? fx : axis == 1 ? fy : fz, s = u >= f;
+    u -= s * f;
+    const int q = small_div(u, axis == 0 ? ih : iw), p = u - q * (axis == 0 ? bh : bw);   // first and second tangent
+    b.rc = axis == 0 ? (s ? bw + 2 : 1) : 2 + p;
+    b.rr = axis == 1 ? (s ? bh + 2 : 1) : 2 + (axis == 0 ? p : q);
+    b.rz = axis == 2 ? (s ? bd + 2 : 1) : 2 + q;
+    return b;
+}
+
+// Wave reductions by lane shifts within the vector registers (rows of 16,
+// then across rows); the result is in lane 63.  Values >= 0 for the maxima.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp0(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp0(float v) { return __builtin_bit_cast(float, dpp0<CTRL, ROWS>(__builtin_bit_cast(int, v))); }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp0(double v)
+{
+    const long long b = __builtin_bit_cast(long long, v);
+    const unsigned lo = dpp0<CTRL, ROWS>((int)b), hi = dpp0<CTRL, ROWS>((int)(b >> 32));
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+template <class R, class F>
+__device__ __forceinline__ R wave_reduce63(R v, F f)
+{
+    v = f(v, dpp0<0x111, 0xf>(v));   // row_shr 1, 2, 4, 8
+    v = f(v, dpp0<0x112, 0xf>(v));
+    v = f(v, dpp0<0x114, 0xf>(v));
+    v = f(v, dpp0<0x118, 0xf>(v));
+    v = f(v, dpp0<0x142, 0xa>(v));   // row_bcast 15 into rows 1 and 3
+    v = f(v, dpp0<0x143, 0xc>(v));   // row_bcast 31 into rows 2 and 3
+    return v;
+}
+template <class R>
+__device__ __forceinline__ R wave_max63(R v) { return wave_reduce63(v, [](R a, R b) { return b > a ? b : a; }); }
+template <class R>
+__device__ __forceinline__ R wave_sum63(R v) { return wave_reduce63(v, [](R a, R b) { return a + b; }); }
+
 }  // namespace
 }  // namespace gmd

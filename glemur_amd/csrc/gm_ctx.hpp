@@ -115,6 +115,10 @@ struct gm_ctx {
     // rect and z chunking that suit its own workgroup size and occupancy
     int TX[7] = {}, TY[7] = {}, tiles_x[7] = {}, tiles_y[7] = {};
     int CZ[7] = {}, nchunks[7] = {}, nblocks[7] = {};
+    // stage kernels that compute blocks at once instead of marching their
+    // tile (small grids; off once a caller sets tiles)
+    bool block[6] = {};
+    int BX = 0, BY = 0, BZ = 0;   // the block
     int ncu = 256;
     EvTimer tm;                   // kernel timing (gm_timing_*)
     // graph of one batch

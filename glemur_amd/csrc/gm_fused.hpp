@@ -30,6 +30,7 @@ struct FusedArgs {
     int emit, diag, check_done;
     int face_table;                   // 1: every ghost face from the precomputed constants
                                       // (initial boundary distortion); 0: x/y faces direct (F32K)
+    int block;                        // 1: TX x TY x CZ points a workgroup at once (small grids), no march
     int rev;                          // F32K: march z downwards (plane q stored at nz + 1 - q)
     int rev_alt;                      // F32K: odd z chunks march the other way
     // F64 buffers
@@ -62,6 +63,10 @@ struct CtlArgs {
     int log_cap;
 };
 
+// Block launches (FusedArgs::block): threads a workgroup, at least the points
+// of the block and the face neighbours of the block, and the LDS a box may take.
+constexpr int kBlockThreads = 512;
+constexpr int kBlockLds = 160 * 1024 - 1024;
 // Largest rect (TX+4)(TY+4) a workgroup holds: one point per thread.
 int fused_max_points(int f32k);
 void set_tableau(const TableauF &t);

@@ -875,6 +875,406 @@ k_stage32_batch(const FusedArgs *__restrict__ args, const int *__restrict__ star
     stage32_body<NT, STAGE, PRESS, ALT, false>(args[lo], L - start[lo]);
 }
 
+// ================================================================ blocks
+// Stage kernel of small grids: a workgroup computes a block of up to NT
+// points at once, one output point a thread, instead of marching a column
+// of planes.  A plane step of the march takes about 0.75 us however few
+// columns a workgroup holds (its LDS reads, FP64 determinant and barrier
+// follow one another), so a chunk of two planes, which needs eight or nine
+// steps to fill the pipeline, takes 8 us; a block goes through the same
+// chain once, behind one exposure of the loads' latency.  The price is the
+// halo: the stage positions of the block and of every point within two
+// steps of it along the axes are formed here (2.7 points an output point for
+// 8 x 8 x 8), B at the block and its face neighbours (at most NT of them, one a
+// thread).  Every point takes the operations of the march in their order,
+// so the results are its bit for bit; the energy is summed in another order.
+// What bounds it: at 33 x 33 x 97 (225 blocks, one a CU) the chain itself,
+// 4.5 us a stage beside the march's 21 to 27; from a few blocks a CU on the
+// vector instructions (about half of them for halo and face neighbours) and
+// the two blocks a CU that LDS holds: 49 x 49 x 145 stages 1 to 4 26 to 29 ->
+// 14 to 16 us (events around the launches), an attempt 166 -> 93 us.
+template <int NT, int STAGE, bool PRESS, bool PERI>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_block32(FusedArgs A)
+{
+#pragma clang fp contract(fast)
+    constexpr bool FINAL = STAGE == 5;
+    constexpr int n = STAGE;             // slopes entering the stage position
+    constexpr bool DIAG = STAGE == 0;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ double red[7][NT / 64];
+    const Geo &g = A.g;
+    Ctl *ctl = A.ctl;
+    if (A.check_done && ctl->done) return;
+    const int cur = ctl->cur;
+    const float dt = (float)ctl->dt;
+    const long long P3 = 3 * g.P;
+
+    const int lb = xcd_remap(blockIdx.x, A.nblocks);
+    const int tx = lb % A.tiles_x, ty = (lb / A.tiles_x) % A.tiles_y, ch = lb / (A.tiles_x * A.tiles_y);
+    const int ix0 = tx * A.TX, iy0 = ty * A.TY, iz0 = ch * A.CZ;
+    const int bw = min(A.TX, g.nx - ix0), bh = min(A.TY, g.ny - iy0), bd = min(A.CZ, g.nz - iz0);
+    // box of positions, two points beyond the block on every side; box
+    // coordinate (c, r, z) is padded point (ix0 - 1 + c, iy0 - 1 + r, iz0 - 1 + z)
+    const int W = A.TX + 4, H = A.TY + 4, D = A.CZ + 4, WH = W * H, Wb = W - 2, WHb = Wb * (H - 2);
+    float4 *xa = reinterpret_cast<float4 *>(smem);          // hi x, y, z, small x
+    float4 *bl = xa + W * H * D;                            // B, one point beyond the block
+    float2 *xb = reinterpret_cast<float2 *>(bl + WHb * (D - 2));   // small y, z
+    auto xi = [&](int c, int r, int z) { return c + W * r + WH * z; };
+    auto bi = [&](int c, int r, int z) { return (c - 1) + Wb * (r - 1) + WHb * (z - 1); };
+    auto ldx = [&](int i, Pt3 &o) {
+        const float4 a = xa[i];
+        const float2 b = xb[i];
+        o.h[0] = a.x; o.h[1] = a.y; o.h[2] = a.z;
+        o.s[0] = a.w; o.s[1] = b.x; o.s[2] = b.y;
+    };
+    auto ldb = [&](int i, float o[3]) {
+        const float4 a = bl[i];
+        o[0] = a.x; o[1] = a.y; o[2] = a.z;
+    };
+
+    const bool px = PERI && g.xPeri, py = PERI && g.yPeri, pz = PERI && g.zPeri;
+    // the periods a point beyond a periodic axis is away from its source, and
+    // byte offsets of a point's source and of the point itself
+    auto sg = [](bool on, int i, int nn) { return on ? (i <= 0 ? -1 : i >= nn + 1 ? 1 : 0) : 0; };
+    auto src12 = [&](int gi, int gj, int gk) {
+        const int i = px ? gi - sg(true, gi, g.nx) * g.nx : min(max(gi, 0), g.nx + 1);
+        const int j = py ? gj - sg(true, gj, g.ny) * g.ny : min(max(gj, 0), g.ny + 1);
+        const int k = pz ? gk - sg(true, gk, g.nz) * g.nz : min(max(gk, 0), g.nz + 1);
+        return 12 * (int)(i + g.sx * (long long)j + g.sxy * (long long)k);
+    };
+    const BufF bXh = buf_of(A.Xh[cur], P3), bXl = buf_of(A.Xl[cur], P3), bB0 = buf_of(A.B0_32, P3);
+    BufF bK[5];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) bK[m] = buf_of(A.K32 + m * P3, P3);
+
+    // ---- this thread's output point and its face neighbour of the block
+    const int t = threadIdx.x;
+    const BlockRole role = block_role(t, bw, bh, bd);
+    const bool own = role.own, ring = role.ring;
+    const int oc = role.oc, orr = role.orr, oz = role.oz, rc = role.rc, rr = role.rr, rz = role.rz;
+    const int ogi = ix0 - 1 + oc, ogj = iy0 - 1 + orr, ogk = iz0 - 1 + oz;
+    const int o12 = src12(ogi, ogj, ogk);
+    const int rgi = ix0 - 1 + rc, rgj = iy0 - 1 + rr, rgk = iz0 - 1 + rz;
+    float b0o[3], b0r[3];
+    bB0.ld3(o12, b0o);
+    bB0.ld3(src12(rgi, rgj, rgk), b0r);
+    float fg0[3] = {0.f, 0.f, 0.f}, fe0[3] = {0.f, 0.f, 0.f};
+    if constexpr (FINAL) {
+        // sum (c - b5) k and sum (c - c*) k of the output point
+        float k[5][3];
+#pragma unroll
+        for (int m = 0; m < 5; ++m) bK[m].ld3(o12, k[m]);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            float a1 = 0, a2 = 0;
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                a1 += (float)(c_tab32.c[m] - c_tab32.b[5 * 6 + m]) * k[m][l];
+                a2 += (float)c_tab32.ce[m] * k[m][l];
+            }
+            fg0[l] = a1;
+            fe0[l] = a2;
+        }
+    }
+    (void)fg0; (void)fe0;
+
+    // ---- (1) stage positions of the box: a thread takes one column, groups
+    // of W H threads its planes in turn
+    {
+        const float iWH = __builtin_amdgcn_rcpf((float)WH);
+        const int groups = small_div(NT, iWH), grp = small_div(t, iWH), col0 = t - grp * WH;
+        const int r = small_div(col0, __builtin_amdgcn_rcpf((float)W)), c = col0 - r * W;
+        const int gi = ix0 - 1 + c, gj = iy0 - 1 + r;
+        const bool col = gi >= (px ? -1 : 0) && gi <= g.nx + (px ? 2 : 1) && gj >= (py ? -1 : 0) && gj <= g.ny + (py ? 2 : 1);
+        // virtual columns: the outer ghost of a line-tied x or y face
+        const int vx = !px && gj >= 0 && gj <= g.ny + 1 ? (gi == -1 ? -1 : gi == g.nx + 2 ? 1 : 0) : 0;
+        const int vy = !py && gi >= 0 && gi <= g.nx + 1 ? (gj == -1 ? -1 : gj == g.ny + 2 ? 1 : 0) : 0;
+        const bool ldc = grp < groups && (col || (!A.face_table && (vx != 0 || vy != 0)));
+        // points within two steps of the block along the axes
+        const int far = max(max(2 - c, c - 1 - bw), 0) + max(max(2 - r, r - 1 - bh), 0);
+        const int v0 = src12(gi, gj, 0) - (pz ? 12 * (int)(g.sxy * g.nz) : 0);   // the column's plane 0
+        const int sgx = sg(px, gi, g.nx), sgy = sg(py, gj, g.ny);
+        constexpr int U = n >= 4 ? 2 : n >= 2 ? 3 : 4;   // planes loaded at a time
+        for (int z0 = grp; z0 < bd + 4; z0 += U * groups) {
+            struct In {
+                float x[3], lo[3], k[5][3];
+            } in[U];
+            bool ok[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int z = z0 + u * groups, gk = iz0 - 1 + z;
+                ok[u] = ldc && z < bd + 4 && far + max(max(2 - z, z - 1 - bd), 0) <= 2 && gk >= (pz ? -1 : 0) &&
+                        gk <= g.nz + (pz ? 2 : 1);
+                if (ok[u]) {
+                    const int v = v0 + 12 * (int)g.sxy * (gk - (pz ? sg(true, gk, g.nz) * g.nz : 0));
+                    bXh.ld3(v, in[u].x);
+                    bXl.ld3(v, in[u].lo);
+#pragma unroll
+                    for (int m = 0; m < 5; ++m)
+                        if (m < n) bK[m].ld3(v, in[u].k[m]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (!ok[u]) continue;
+                const int z = z0 + u * groups;
+                Pt3 xn;
+#pragma unroll
+                for (int l = 0; l < 3; ++l) {
+                    float s = in[u].lo[l];
+#pragma unroll
+                    for (int m = 0; m < 5; ++m)
+                        if (m < n) s += (float)c_tab32.b[n * 6 + m] * in[u].k[m][l];
+                    xn.h[l] = in[u].x[l];
+                    xn.s[l] = s;
+                }
+                if (vx) xn.s[0] += (float)vx * (float)g.dx;
+                if (vy) xn.s[1] += (float)vy * (float)g.dy;
+                if constexpr (PERI) {
+                    const int sh[3] = {sgx, sgy, sg(pz, iz0 - 1 + z, g.nz)};
+                    const double per[3] = {g.Lx + g.dx, g.Ly + g.dy, g.Lz + g.dz};
+#pragma unroll
+                    for (int l = 0; l < 3; ++l) {
+                        if (sh[l]) {
+                            const float ph = (float)per[l], pl = (float)(per[l] - (double)ph);
+                            float hs, e;
+                            two_sum(xn.h[l], (float)sh[l] * ph, hs, e);
+                            xn.h[l] = hs;
+                            xn.s[l] += e + (float)sh[l] * pl;
+                        }
+                    }
+                }
+                const int i = col0 + WH * z;
+                xa[i] = make_float4(xn.h[0], xn.h[1], xn.h[2], xn.s[0]);
+                xb[i] = make_float2(xn.s[1], xn.s[2]);
+            }
+        }
+    }
+    __syncthreads();
+
+    // ---- (2) B at the block and its face neighbours
+    const float hx = 0.5f * (float)g.dx1, hy = 0.5f * (float)g.dy1, hz = 0.5f * (float)g.dz1;
+    auto interior = [&](int i, const float b0[3], float drn[3][3], float Bv[3]) {
+        Pt3 a, b;
+        ldx(i + 1, a);
+        ldx(i - 1, b);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) drn[0][l] = dif(a, b, l);
+        ldx(i + W, a);
+        ldx(i - W, b);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) drn[1][l] = dif(a, b, l);
+        ldx(i + WH, a);
+        ldx(i - WH, b);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) drn[2][l] = dif(a, b, l);
+        const double detv = det32(drn) * ((double)hx * (double)hy * (double)hz);
+        const float rd = __builtin_amdgcn_rcpf((float)detv);
+        const float bs[3] = {b0[0] * hx, b0[1] * hy, b0[2] * hz};
+#pragma unroll
+        for (int l = 0; l < 3; ++l) Bv[l] = (drn[0][l] * bs[0] + drn[1][l] * bs[1] + drn[2][l] * bs[2]) * rd;
+        return detv;
+    };
+    const int xo = xi(oc, orr, oz);
+    float dr[3][3], Bc[3];
+    const double dq0 = interior(xo, b0o, dr, Bc);
+    if (own) bl[bi(oc, orr, oz)] = make_float4(Bc[0], Bc[1], Bc[2], 0.f);
+    if (ring) {
+        const bool gx = rgi == 0 || rgi == g.nx + 1, gy = rgj == 0 || rgj == g.ny + 1;
+        const bool lx = gx && !px, ly = gy && !py, lz = !pz && (rgk == 0 || rgk == g.nz + 1);
+        const int i = xi(rc, rr, rz);
+        float Bv[3];
+        if (!lz && !(A.face_table && (lx || ly))) {
+            float drn[3][3];
+            (void)interior(i, b0r, drn, Bv);
+            if (lx) Bv[0] = b0r[0];
+            if (ly) Bv[1] = b0r[1];
+        } else {
+            const int face = lz ? 2 : lx ? 0 : 1;
+            const int side = lz ? rgk != 0 : lx ? rgi != 0 : rgj != 0;
+            const int u = lz ? rgi - 1 : lx ? rgj - 1 : rgi - 1, v = lz ? rgj - 1 : rgk - 1;
+            const int st = lz ? WH : lx ? 1 : W;
+            Pt3 pin;
+            ldx(side ? i - st : i + st, pin);
+            double xin[3], Bd[3], detv;
+#pragma unroll
+            for (int l = 0; l < 3; ++l) xin[l] = (double)pin.h[l] + (double)pin.s[l];
+            const GhostPt &G = A.ghost[A.ghost_off[face * 2 + side] + u + (long long)nface(g, face) * v];
+            ghost_b(g, G, face, side, xin, Bd, detv);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) Bv[l] = (float)Bd[l];
+        }
+        bl[bi(rc, rr, rz)] = make_float4(Bv[0], Bv[1], Bv[2], 0.f);
+    }
+    __syncthreads();
+
+    // ---- (3) J, force and slope at the output point
+    double dmax = 0, e_sum = 0;
+    float mx[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    (void)mx;
+    int nan_seen = 0;
+    if (own) {
+        const int ib = bi(oc, orr, oz);
+        float db[3][3], bp[3], bm[3];
+        ldb(ib + 1, bp);
+        ldb(ib - 1, bm);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) db[0][l] = bp[l] - bm[l];
+        ldb(ib + Wb, bp);
+        ldb(ib - Wb, bm);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) db[1][l] = bp[l] - bm[l];
+        ldb(ib + WHb, bp);
+        ldb(ib - WHb, bm);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) db[2][l] = bp[l] - bm[l];
+        float C[3][3];
+#pragma unroll
+        for (int a0 = 0; a0 < 3; ++a0) cross3(dr[(a0 + 1) % 3], dr[(a0 + 2) % 3], C[a0]);
+        float Jv[3] = {0.f, 0.f, 0.f}, kv[3];
+#pragma unroll
+        for (int a0 = 0; a0 < 3; ++a0) {
+            Jv[0] = fmaf(C[a0][1], db[a0][2], fmaf(-C[a0][2], db[a0][1], Jv[0]));
+            Jv[1] = fmaf(C[a0][2], db[a0][0], fmaf(-C[a0][0], db[a0][2], Jv[1]));
+            Jv[2] = fmaf(C[a0][0], db[a0][1], fmaf(-C[a0][1], db[a0][0], Jv[2]));
+        }
+        const float rD = __builtin_amdgcn_rcpf((float)(dq0 * (8.0 * g.dx * g.dy * g.dz)));
+#pragma unroll
+        for (int l = 0; l < 3; ++l) Jv[l] *= rD;
+        kv[0] = Jv[1] * Bc[2] - Jv[2] * Bc[1];
+        kv[1] = Jv[2] * Bc[0] - Jv[0] * Bc[2];
+        kv[2] = Jv[0] * Bc[1] - Jv[1] * Bc[0];
+        const int ii = ogi - 1, jj = ogj - 1, kk = ogk - 1;
+        float eps = 1.f;
+        if (g.epsilonProf) {
+            const float eps_xy = (float)(A.epsx[ii] * A.epsy[jj]);
+            eps = eps_xy * (float)A.epsz[kk];
+        }
+        float gv[3] = {0, 0, 0};
+        const double detv = dq0;
+        if constexpr (PRESS) {
+            // gradP in cofactor form, as the march forms it; the mixed second
+            // differences from the positions themselves
+            float dd[3][3], mxy[3], mxz[3], myz[3];
+            Pt3 xc, a, b;
+            ldx(xo, xc);
+#pragma unroll
+            for (int a2 = 0; a2 < 2; ++a2) {
+                Pt3 xp;
+                ldx(a2 == 0 ? xo + 1 : xo + W, xp);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) dd[a2][l] = fmaf(2.f, dif(xp, xc, l), -dr[a2][l]);
+            }
+            ldx(xo - WH, a);
+            ldx(xo + WH, b);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) dd[2][l] = dif(b, xc, l) - dif(xc, a, l);
+            auto mixed = [&](int sa, int sb, float m[3]) {   // dr_b(+a) - dr_b(-a)
+                Pt3 p, q;
+                float e[3];
+                ldx(xo + sa + sb, p);
+                ldx(xo + sa - sb, q);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) e[l] = dif(p, q, l);
+                ldx(xo - sa + sb, p);
+                ldx(xo - sa - sb, q);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) m[l] = e[l] - dif(p, q, l);
+            };
+            mixed(1, W, mxy);
+            mixed(1, WH, mxz);
+            mixed(W, WH, myz);
+            auto dot = [](const float u[3], const float v[3]) { return u[0] * v[0] + u[1] * v[1] + u[2] * v[2]; };
+            const float N0 = 4.f * dot(dd[0], C[0]) + dot(mxy, C[1]) + dot(mxz, C[2]);
+            const float N1 = 4.f * dot(dd[1], C[1]) + dot(mxy, C[0]) + dot(myz, C[2]);
+            const float N2 = 4.f * dot(dd[2], C[2]) + dot(mxz, C[0]) + dot(myz, C[1]);
+            const float f = -(float)g.beta * __builtin_amdgcn_rcpf((float)detv) * (rD * rD);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) gv[l] = (N0 * C[0][l] + N1 * C[1][l] + N2 * C[2][l]) * f;
+        }
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            kv[l] *= dt * eps;
+            if (PRESS) kv[l] += -dt * gv[l];
+        }
+        if (DIAG && A.diag) {
+            float jxb[3];
+            cross3(Jv, Bc, jxb);
+            const float b2 = fmaf(Bc[0], Bc[0], fmaf(Bc[1], Bc[1], Bc[2] * Bc[2]));
+            const float nc2 = fmaf(jxb[0], jxb[0], fmaf(jxb[1], jxb[1], jxb[2] * jxb[2]));
+            const float nj2 = fmaf(Jv[0], Jv[0], fmaf(Jv[1], Jv[1], Jv[2] * Jv[2]));
+            const float den2 = nj2 * b2;
+            const int bound = (ii == 0) + (jj == 0) + (kk == 0) + (ii == g.nx - 1) + (jj == g.ny - 1) +
+                              (kk == g.nz - 1);
+            const float wb = __builtin_bit_cast(float, (127 - bound) << 23);   // 2^-bound
+            e_sum = (double)(b2 * wb) * detv;
+            mx[0] = nb_maxf(0.f, nj2);   // squared, as the march keeps them
+            mx[1] = nb_maxf(0.f, nc2 * __builtin_amdgcn_rcpf(b2 * b2));
+            mx[2] = nb_maxf(0.f, den2 > 0.f ? nc2 * __builtin_amdgcn_rcpf(den2) : 0.f);
+            mx[3] = nb_maxf(0.f, nc2);
+            mx[4] = nb_maxf(0.f, den2);
+        }
+        if constexpr (!FINAL) {
+            bK[STAGE < 5 ? STAGE : 0].st3(kv, o12);
+        } else {
+            Pt3 xc;
+            ldx(xo, xc);
+            float hn[3], ln[3];
+#pragma unroll
+            for (int l = 0; l < 3; ++l) {
+                float hi = xc.h[l], lo;
+                if (l < 2 || g.zUpdate) {
+                    float d = xc.s[l] + (fg0[l] + (float)c_tab32.c[5] * kv[l]);
+                    float s, e;
+                    two_sum(hi, d, s, e);
+                    float hi2 = s + e;
+                    lo = e - (hi2 - s);
+                    hi = hi2;
+                    double dd = fabs((double)fe0[l] + c_tab32.ce[5] * (double)kv[l]);
+                    if (dd != dd) nan_seen = 1;
+                    dmax = nb_max(dmax, dd);
+                } else {
+                    lo = bXl.ld(o12 + 4 * l, 0);
+                }
+                hn[l] = hi;
+                ln[l] = lo;
+            }
+            buf_of(A.Xh[cur ^ 1], P3).st3(hn, o12);
+            buf_of(A.Xl[cur ^ 1], P3).st3(ln, o12);
+        }
+    }
+
+    // ---- block partials (fixed order: deterministic)
+    if (!FINAL && !(DIAG && A.diag)) return;
+    const int w = t >> 6, lane = t & 63;
+    if (FINAL) {
+        dmax = wave_max63(dmax);
+        if (lane == 63) red[0][w] = dmax;
+        if (nan_seen) atomicOr(&ctl->nan_seen, 1);
+    } else {
+        e_sum = wave_sum63(e_sum);
+        if (lane == 63) red[1][w] = e_sum;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+            mx[m] = wave_max63(mx[m]);
+            if (lane == 63) red[m + 2][w] = mx[m];
+        }
+    }
+    __syncthreads();
+    if (t >= 7) return;
+    // thread q combines one of the seven quantities
+    double v = red[t][0];
+    if (t == 1)
+        for (int q = 1; q < NT / 64; ++q) v += red[1][q];
+    else
+        for (int q = 1; q < NT / 64; ++q) v = nb_max(v, red[t][q]);
+    if (FINAL) {
+        if (t == 0) A.part_delta[lb] = v;
+    } else if (t >= 1) {
+        A.part_diag[(t - 1) * (long long)A.nblocks + lb] = t == 1 ? v : sqrt(v);
+    }
+}
+
 namespace {
 // chunk-alternating variants exist for stages 1-5 in 768- and 1024-thread
 // workgroups; other launches ignore A.rev_alt
@@ -931,6 +1331,32 @@ void launch_peri32(hipStream_t s, const FusedArgs &A)
     case 4: launch_k32<512, 4, PRESS, false, true>(s, A); break;
     case 5: launch_k32<512, 5, PRESS, false, true>(s, A); break;
     default: launch_k32<512, 6, PRESS, false, true>(s, A); break;
+    }
+}
+// LDS of a block's box: positions 24 bytes a point, B 16 bytes
+size_t block32_lds(const FusedArgs &A)
+{
+    return (size_t)24 * (A.TX + 4) * (A.TY + 4) * (A.CZ + 4) + (size_t)16 * (A.TX + 2) * (A.TY + 2) * (A.CZ + 2);
+}
+template <int STAGE, bool PRESS, bool PERI>
+void launch_b32(hipStream_t s, const FusedArgs &A)
+{
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k_block32<kBlockThreads, STAGE, PRESS, PERI>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBlockLds);
+    (void)attr;
+    hipLaunchKernelGGL((k_block32<kBlockThreads, STAGE, PRESS, PERI>), dim3(A.nblocks), dim3(kBlockThreads),
+                       block32_lds(A), s, A);
+}
+template <bool PRESS, bool PERI>
+void launch_block32(hipStream_t s, const FusedArgs &A)
+{
+    switch (A.stage) {
+    case 0: launch_b32<0, PRESS, PERI>(s, A); break;
+    case 1: launch_b32<1, PRESS, PERI>(s, A); break;
+    case 2: launch_b32<2, PRESS, PERI>(s, A); break;
+    case 3: launch_b32<3, PRESS, PERI>(s, A); break;
+    case 4: launch_b32<4, PRESS, PERI>(s, A); break;
+    default: launch_b32<5, PRESS, PERI>(s, A); break;
     }
 }
 // 1024 threads: stages 0-4 and the fields pass without pressure
@@ -1083,6 +1509,12 @@ void launch_fused32_batch(hipStream_t s, int stage, int press, int nt, const Fus
 
 void launch_fused32(hipStream_t s, const FusedArgs &A)
 {
+    if (A.block) {
+        const bool peri = A.g.xPeri || A.g.yPeri || A.g.zPeri;
+        if (A.g.pressure) peri ? launch_block32<true, true>(s, A) : launch_block32<true, false>(s, A);
+        else peri ? launch_block32<false, true>(s, A) : launch_block32<false, false>(s, A);
+        return;
+    }
     if (A.g.xPeri || A.g.yPeri || A.g.zPeri) {
         if (A.g.pressure) launch_peri32<true>(s, A);
         else launch_peri32<false>(s, A);

@@ -30,6 +30,8 @@
 #include "gm_fused.hpp"
 #include "fused_common.hpp"
 
+#include <type_traits>
+
 namespace gmd {
 
 __constant__ TableauF c_tab;
@@ -706,6 +708,442 @@ __global__ void __launch_bounds__(NT) k_stage64_batch(const FusedArgs *__restric
     stage64_body<NT, STAGE, PRESS, false, false>(args[lo], L - start[lo]);
 }
 
+// ================================================================ blocks
+// Stage kernel of small grids: a workgroup computes a block of up to NT
+// points at once, one output point a thread, instead of marching a column
+// of planes (2 to 3 us a plane step however few columns, 3 steps to fill the
+// pipeline).  The stage positions of the block and of every point within two
+// steps of it along the axes are formed, B at the block and at its face
+// neighbours (at most NT, one a thread), then J and the slope: one pass
+// through the march's chain, behind one exposure of the loads' latency.
+// Every point takes the march's operations in their order (the reference's),
+// so the results are the same bit for bit; the energy is summed in another
+// order.  Points beyond a periodic face hold their source's position
+// unshifted and readers shift, as in the march.
+// It needs half the march's registers (122 to 138, no queues along z), so
+// two blocks share a CU.  An attempt at 33 x 33 x 97 285 -> 72 us, at 65 x 65
+// x 193 372 -> 328 us; bound by the FP64 instructions of the block, its ring
+// and its halo there.
+template <int NT, int STAGE, bool PRESS, bool PERI>
+__global__ void __launch_bounds__(NT) k_block64(FusedArgs A)
+{
+    constexpr bool FINAL = STAGE == 5, DIAG = STAGE == 0;
+    constexpr int n = STAGE;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ double red[7][NT / 64];
+    const Geo &g = A.g;
+    Ctl *ctl = A.ctl;
+    if (A.check_done && ctl->done) return;
+    const int cur = ctl->cur;
+    const double dt = ctl->dt;
+    const long long P = g.P, P3 = 3 * P;
+
+    const int lb = xcd_remap(blockIdx.x, A.nblocks);
+    const int tx = lb % A.tiles_x, ty = (lb / A.tiles_x) % A.tiles_y, ch = lb / (A.tiles_x * A.tiles_y);
+    const int ix0 = tx * A.TX, iy0 = ty * A.TY, iz0 = ch * A.CZ;
+    const int bw = min(A.TX, g.nx - ix0), bh = min(A.TY, g.ny - iy0), bd = min(A.CZ, g.nz - iz0);
+    // box of positions, two points beyond the block on every side; box
+    // coordinate (c, r, z) is padded point (ix0 - 1 + c, iy0 - 1 + r, iz0 - 1 + z)
+    const int W = A.TX + 4, H = A.TY + 4, D = A.CZ + 4, WH = W * H, nbox = WH * D;
+    const int Wb = W - 2, WHb = Wb * (H - 2), nb = WHb * (D - 2);
+    double *xs = reinterpret_cast<double *>(smem), *bs = xs + 3 * nbox;
+    auto ldx = [&](int i, Pos &o) {
+#pragma unroll
+        for (int l = 0; l < 3; ++l) o.x[l] = xs[l * nbox + i];
+    };
+    auto ldb = [&](int i, double o[3]) {
+#pragma unroll
+        for (int l = 0; l < 3; ++l) o[l] = bs[l * nb + i];
+    };
+    auto stb = [&](int i, const double v[3]) {
+#pragma unroll
+        for (int l = 0; l < 3; ++l) bs[l * nb + i] = v[l];
+    };
+    auto bi = [&](int c, int r, int z) { return (c - 1) + Wb * (r - 1) + WHb * (z - 1); };
+
+    const bool px = PERI && g.xPeri, py = PERI && g.yPeri, pz = PERI && g.zPeri;
+    // the point the reference copies into one beyond a periodic face
+    auto wrap = [](bool on, int i, int nn) { return on ? (i <= 0 ? i + nn : i >= nn + 1 ? i - nn : i) : i; };
+    auto shift = [&](Pos &v, int axis, int sgn) {
+        if (PERI && sgn != 0) {
+            const double Lp = axis == 0 ? g.Lx : axis == 1 ? g.Ly : g.Lz;
+            const double h = axis == 0 ? g.dx : axis == 1 ? g.dy : g.dz;
+            v.x[axis] = sgn < 0 ? (v.x[axis] - Lp) - h : (v.x[axis] + Lp) + h;
+        }
+    };
+    (void)shift;
+    const double *X0 = A.X64[cur], *K = A.K64;
+
+    // ---- this thread's output point and its face neighbour of the block
+    const int t = threadIdx.x;
+    const BlockRole role = block_role(t, bw, bh, bd);
+    const bool own = role.own, ring = role.ring;
+    const int oc = role.oc, orr = role.orr, oz = role.oz, rc = role.rc, rr = role.rr, rz = role.rz;
+    const int ogi = ix0 - 1 + oc, ogj = iy0 - 1 + orr, ogk = iz0 - 1 + oz;
+    const long long oa = ogi + g.sx * (long long)ogj + g.sxy * (long long)ogk;
+    const int rsi = wrap(px, ix0 - 1 + rc, g.nx), rsj = wrap(py, iy0 - 1 + rr, g.ny), rsk = wrap(pz, iz0 - 1 + rz, g.nz);
+    const long long ra = rsi + g.sx * (long long)rsj + g.sxy * (long long)rsk;
+    double b0o[3], b0r[3];
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        b0o[l] = A.B0_64[l * P + oa];
+        b0r[l] = A.B0_64[l * P + ra];
+    }
+
+    // ---- (1) stage positions of the box: a thread takes one column, groups
+    // of W H threads its planes in turn
+    {
+        const float iWH = __builtin_amdgcn_rcpf((float)WH);
+        const int groups = small_div(NT, iWH), grp = small_div(t, iWH), col0 = t - grp * WH;
+        const int r = small_div(col0, __builtin_amdgcn_rcpf((float)W)), c = col0 - r * W;
+        const int si = wrap(px, ix0 - 1 + c, g.nx), sj = wrap(py, iy0 - 1 + r, g.ny);
+        const bool col = grp < groups && si >= 0 && si <= g.nx + 1 && sj >= 0 && sj <= g.ny + 1;
+        const bool gxy = si == 0 || si == g.nx + 1 || sj == 0 || sj == g.ny + 1;
+        // points within two steps of the block along the axes
+        const int far = max(max(2 - c, c - 1 - bw), 0) + max(max(2 - r, r - 1 - bh), 0);
+        const long long a0 = si + g.sx * (long long)sj;
+        constexpr int U = n >= 4 ? 1 : n >= 2 ? 2 : 4;   // planes loaded at a time
+        for (int z0 = grp; z0 < bd + 4; z0 += U * groups) {
+            struct In {
+                double x[3], k[5][3];
+            } in[U];
+            bool ok[U], gh[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int z = z0 + u * groups, sk = wrap(pz, iz0 - 1 + z, g.nz);
+                ok[u] = col && z < bd + 4 && far + max(max(2 - z, z - 1 - bd), 0) <= 2 && sk >= 0 && sk <= g.nz + 1;
+                gh[u] = gxy || sk == 0 || sk == g.nz + 1;
+                if (ok[u]) {
+                    const long long a = a0 + g.sxy * (long long)sk;
+#pragma unroll
+                    for (int l = 0; l < 3; ++l) in[u].x[l] = X0[l * P + a];
+                    if (!gh[u])
+#pragma unroll
+                        for (int m = 0; m < 5; ++m)
+                            if (m < n)
+#pragma unroll
+                                for (int l = 0; l < 3; ++l) in[u].k[m][l] = K[m * P3 + l * P + a];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (!ok[u]) continue;
+#pragma unroll
+                for (int l = 0; l < 3; ++l) {
+                    // x_n by the reference's incremental stage updates
+                    double x = in[u].x[l];
+                    if (!gh[u])
+#pragma unroll
+                        for (int s2 = 0; s2 < 5; ++s2)
+                            if (s2 < n)
+#pragma unroll
+                                for (int m = 0; m <= s2; ++m) x += c_tab.db[s2 * 6 + m] * in[u].k[m][l];
+                    xs[l * nbox + col0 + WH * (z0 + u * groups)] = x;
+                }
+            }
+        }
+    }
+    __syncthreads();
+
+    // ---- (2) B at the block and its face neighbours.  (si, sj, sk): the
+    // point's source; GH: it may be a line-tied ghost point
+    auto b_at = [&](int i, int si, int sj, int sk, const double b0[3], auto ghost, double Bv[3]) -> double {
+        constexpr bool GH = decltype(ghost)::value;
+        Pos xm, xp, ym, yp, zm, zp;
+        ldx(i - 1, xm);
+        ldx(i + 1, xp);
+        ldx(i - W, ym);
+        ldx(i + W, yp);
+        ldx(i - WH, zm);
+        ldx(i + WH, zp);
+        if constexpr (PERI) {
+            shift(xm, 0, px && si == 1 ? -1 : 0);
+            shift(xp, 0, px && si == g.nx ? 1 : 0);
+            shift(ym, 1, py && sj == 1 ? -1 : 0);
+            shift(yp, 1, py && sj == g.ny ? 1 : 0);
+            shift(zm, 2, pz && sk == 1 ? -1 : 0);
+            shift(zp, 2, pz && sk == g.nz ? 1 : 0);
+        }
+        int normal = -1;
+        if constexpr (GH) {
+            const bool gx = si == 0 || si == g.nx + 1, gy = sj == 0 || sj == g.ny + 1;
+            if (gx || gy) {
+                // the face formula's substitutions (see the march)
+                Pos xg;
+                ldx(i, xg);
+                const int v = sk - 1;
+                if (gx) {
+                    normal = 0;
+                    const int side = si != 0, cu = sj - 1;
+                    Pos x2 = xg;
+                    x2.x[0] = xg.x[0] + (2 * side - 1) * g.dx;
+                    if (side) xp = x2;
+                    else xm = x2;
+                    if (cu % 16 == 0) {
+                        ym = xg;
+                        ym.x[1] = xg.x[1] + (double)(-1) * g.dy;
+                    }
+                    if (cu % 16 == 15 || cu == g.ny - 1) {
+                        yp = xg;
+                        yp.x[1] = xg.x[1] + (double)(+1) * g.dy;
+                    }
+                } else {
+                    normal = 1;
+                    const int side = sj != 0, cu = si - 1;
+                    Pos x2 = xg;
+                    x2.x[1] = xg.x[1] + (2 * side - 1) * g.dy;
+                    if (side) yp = x2;
+                    else ym = x2;
+                    if (cu % 16 == 0) {
+                        xm = xg;
+                        xm.x[0] = xg.x[0] + (double)(-1) * g.dx;
+                    }
+                    if (cu % 16 == 15 || cu == g.nx - 1) {
+                        xp = xg;
+                        xp.x[0] = xg.x[0] + (double)(+1) * g.dx;
+                    }
+                }
+                if (v % 16 == 0) {
+                    zm = xg;
+                    zm.x[2] = xg.x[2] + (double)(-1) * g.dz;
+                }
+                if (v % 16 == 15 || v == g.nz - 1) {
+                    zp = xg;
+                    zp.x[2] = xg.x[2] + (double)(+1) * g.dz;
+                }
+            }
+        }
+        double jac[3][3], d[3];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) d[l] = pdiff(xp, xm, l);
+        jac_col(jac, 0, d, g.dx1);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) d[l] = pdiff(yp, ym, l);
+        jac_col(jac, 1, d, g.dy1);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) d[l] = pdiff(zp, zm, l);
+        jac_col(jac, 2, d, g.dz1);
+        const double detJac1 = cauchy_b(jac, b0, normal, Bv);
+        return 1. / detJac1;
+    };
+    const int xo = oc + W * orr + WH * oz, ib = bi(oc, orr, oz);
+    double Bc[3];
+    const double detv = b_at(xo, ogi, ogj, ogk, b0o, std::false_type{}, Bc);
+    if (own) stb(ib, Bc);
+    if (ring) {
+        const int i = rc + W * rr + WH * rz;
+        double Bv[3];
+        if (!pz && (rsk == 0 || rsk == g.nz + 1)) {
+            const int side = rsk != 0;
+            Pos pin;
+            ldx(side ? i - WH : i + WH, pin);
+            double det;
+            const GhostPt G = A.ghost[A.ghost_off[4 + side] + (rsi - 1) + (long long)nface(g, 2) * (rsj - 1)];
+            ghost_b_f<2>(g, G, side, pin.x, Bv, det);
+        } else {
+            (void)b_at(i, rsi, rsj, rsk, b0r, std::true_type{}, Bv);
+        }
+        stb(bi(rc, rr, rz), Bv);
+    }
+    __syncthreads();
+
+    // ---- (3) J, force and slope at the output point
+    double dmax = 0, e_sum = 0, mx[5] = {0, 0, 0, 0, 0};
+    (void)mx;
+    int nan_seen = 0;
+    if (own) {
+        const int shxm = px && ogi == 1 ? -1 : 0, shxp = px && ogi == g.nx ? 1 : 0;
+        const int shym = py && ogj == 1 ? -1 : 0, shyp = py && ogj == g.ny ? 1 : 0;
+        const int shzm = pz && ogk == 1 ? -1 : 0, shzp = pz && ogk == g.nz ? 1 : 0;
+        (void)shxm; (void)shxp; (void)shym; (void)shyp; (void)shzm; (void)shzp;
+        Pos xm, xp, ym, yp, zm, zp;
+        ldx(xo - 1, xm);
+        ldx(xo + 1, xp);
+        ldx(xo - W, ym);
+        ldx(xo + W, yp);
+        ldx(xo - WH, zm);
+        ldx(xo + WH, zp);
+        if constexpr (PERI) {
+            shift(xm, 0, shxm);
+            shift(xp, 0, shxp);
+            shift(ym, 1, shym);
+            shift(yp, 1, shyp);
+            shift(zm, 2, shzm);
+            shift(zp, 2, shzp);
+        }
+        double Bxm[3], Bxp[3], Bym[3], Byp[3], Bzm[3], Bzp[3];
+        ldb(ib - 1, Bxm);
+        ldb(ib + 1, Bxp);
+        ldb(ib - Wb, Bym);
+        ldb(ib + Wb, Byp);
+        ldb(ib - WHb, Bzm);
+        ldb(ib + WHb, Bzp);
+        double Jv[3], kv[3];
+        {
+            // diamonds in circulation order (src/current.cu:291-382):
+            // xy: W S E N; yz: y- z- y+ z+; xz: z- x- z+ x+
+            const Pos *V[3][4] = {{&xm, &ym, &xp, &yp}, {&ym, &zm, &yp, &zp}, {&zm, &xm, &zp, &xp}};
+            const double *Wv[3][4] = {{Bxm, Bym, Bxp, Byp}, {Bym, Bzm, Byp, Bzp}, {Bzm, Bxm, Bzp, Bxp}};
+            double NA[3][3], II[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                double d[4][3], bv[4][3];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int l = 0; l < 3; ++l) {
+                        d[e][l] = pdiff(*V[q][(e + 1) & 3], *V[q][e], l);
+                        bv[e][l] = Wv[q][e][l];
+                    }
+                II[q] = diamond(d, bv, NA[q]);
+            }
+            solve_na(NA, II, Jv);
+        }
+        cross3(Jv, Bc, kv);
+        const int ii = ogi - 1, jj = ogj - 1, kk = ogk - 1;
+        double eps = 1.0;
+        if (g.epsilonProf) {
+            const double eps_xy = A.epsx[ii] * A.epsy[jj];
+            eps = eps_xy * A.epsz[kk];
+        }
+        double gv[3] = {0, 0, 0};
+        if constexpr (PRESS) {
+            // gradP from second differences (src/gradP.cu:93-154)
+            auto xat = [&](int di, int dj, int dk, Pos &o) {
+                ldx(xo + di + dj * W + dk * WH, o);
+                if constexpr (PERI) {
+                    shift(o, 0, di < 0 ? shxm : di > 0 ? shxp : 0);
+                    shift(o, 1, dj < 0 ? shym : dj > 0 ? shyp : 0);
+                    shift(o, 2, dk < 0 ? shzm : dk > 0 ? shzp : 0);
+                }
+            };
+            Pos pa, pb, pc, pd, x0c;
+            ldx(xo, x0c);
+            double jac[3][3], d2[3][3][3], d[3];
+#pragma unroll
+            for (int l = 0; l < 3; ++l) d[l] = pdiff(xp, xm, l);
+            jac_col(jac, 0, d, g.dx1);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) d[l] = pdiff(yp, ym, l);
+            jac_col(jac, 1, d, g.dy1);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) d[l] = pdiff(zp, zm, l);
+            jac_col(jac, 2, d, g.dz1);
+            const double h1[3] = {g.dx1, g.dy1, g.dz1};
+            const Pos *ax[3][2] = {{&xm, &xp}, {&ym, &yp}, {&zm, &zp}};
+#pragma unroll
+            for (int a2 = 0; a2 < 3; ++a2)
+#pragma unroll
+                for (int l = 0; l < 3; ++l)
+                    d2[l][a2][a2] = (ax[a2][1]->x[l] - 2 * x0c.x[l] + ax[a2][0]->x[l]) * h1[a2] * h1[a2];
+            const int pr[3][2] = {{0, 1}, {0, 2}, {1, 2}};
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const int aa = pr[m][0], bb = pr[m][1];
+                int o1[3] = {0, 0, 0}, o2[3] = {0, 0, 0};
+                o1[aa] = 1;
+                o2[bb] = 1;
+                xat(o1[0] + o2[0], o1[1] + o2[1], o1[2] + o2[2], pa);
+                xat(o1[0] - o2[0], o1[1] - o2[1], o1[2] - o2[2], pb);
+                xat(-o1[0] + o2[0], -o1[1] + o2[1], -o1[2] + o2[2], pc);
+                xat(-o1[0] - o2[0], -o1[1] - o2[1], -o1[2] - o2[2], pd);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) {
+                    double v;
+                    if (m == 2)  // the reference's term order for d2/dy dz
+                        v = (pa.x[l] - pc.x[l] - pb.x[l] + pd.x[l]) * h1[aa] * h1[bb] / 4;
+                    else
+                        v = (pa.x[l] - pb.x[l] - pc.x[l] + pd.x[l]) * h1[aa] * h1[bb] / 4;
+                    d2[l][aa][bb] = v;
+                    d2[l][bb][aa] = v;
+                }
+            }
+            gradp_core(jac, d2, 1 / detv, g.beta, gv);
+        }
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            kv[l] *= dt * eps;
+            if (PRESS) kv[l] += -dt * gv[l];
+        }
+        if (DIAG && A.diag) {
+            double jxb[3];
+            cross3(Jv, Bc, jxb);
+            const double b2 = Bc[0] * Bc[0] + Bc[1] * Bc[1] + Bc[2] * Bc[2];
+            const double nc = sqrt(jxb[0] * jxb[0] + jxb[1] * jxb[1] + jxb[2] * jxb[2]);
+            const double nj = sqrt(Jv[0] * Jv[0] + Jv[1] * Jv[1] + Jv[2] * Jv[2]);
+            const int bound = (ii == 0) + (jj == 0) + (kk == 0) + (ii == g.nx - 1) + (jj == g.ny - 1) + (kk == g.nz - 1);
+            e_sum = b2 * detv / (1 << bound);
+            const double den = nj * sqrt(b2);
+            mx[0] = nb_max(0, nj);
+            mx[1] = nb_max(0, nc / b2);
+            mx[2] = nb_max(0, den > 0 ? nc / den : 0.0);
+            mx[3] = nb_max(0, nc);
+            mx[4] = nb_max(0, den);
+        }
+        if constexpr (!FINAL) {
+#pragma unroll
+            for (int l = 0; l < 3; ++l) A.K64[STAGE * P3 + l * P + oa] = kv[l];
+        } else {
+            // x_6, then the x5/x4 weights, as in the march
+            double *Xd = A.X64[(cur + 1) % 3], *X6 = A.X64[(cur + 2) % 3];
+            Pos x5;
+            ldx(xo, x5);
+#pragma unroll
+            for (int l = 0; l < 3; ++l) {
+                double k6[6];
+#pragma unroll
+                for (int m = 0; m < 5; ++m) k6[m] = K[m * P3 + l * P + oa];
+                k6[5] = kv[l];
+                double x6 = x5.x[l];
+#pragma unroll
+                for (int m = 0; m < 6; ++m) x6 += c_tab.db[5 * 6 + m] * k6[m];
+                X6[l * P + oa] = x6;
+                double xn = x6, xst = x6;
+                if (l < 2 || g.zUpdate)
+#pragma unroll
+                    for (int m = 0; m < 6; ++m) {
+                        xn += c_tab.c[m] * k6[m];
+                        xst += c_tab.cs[m] * k6[m];
+                    }
+                Xd[l * P + oa] = xn;
+                const double dd = fabs(xn - xst);
+                if (dd != dd) nan_seen = 1;
+                dmax = nb_max(dmax, dd);
+            }
+        }
+    }
+
+    // ---- block partials (fixed order: deterministic)
+    if (!FINAL && !(DIAG && A.diag)) return;
+    const int w = t >> 6, lane = t & 63;
+    if (FINAL) {
+        dmax = wave_max63(dmax);
+        if (lane == 63) red[0][w] = dmax;
+        if (nan_seen) atomicOr(&ctl->nan_seen, 1);
+    } else {
+        e_sum = wave_sum63(e_sum);
+        if (lane == 63) red[1][w] = e_sum;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+            mx[m] = wave_max63(mx[m]);
+            if (lane == 63) red[m + 2][w] = mx[m];
+        }
+    }
+    __syncthreads();
+    if (t >= 7) return;
+    // thread q combines one of the seven quantities
+    double v = red[t][0];
+    if (t == 1)
+        for (int q = 1; q < NT / 64; ++q) v += red[1][q];
+    else
+        for (int q = 1; q < NT / 64; ++q) v = nb_max(v, red[t][q]);
+    if (FINAL) {
+        if (t == 0) A.part_delta[lb] = v;
+    } else if (t >= 1) {
+        A.part_diag[(t - 1) * (long long)A.nblocks + lb] = v;
+    }
+}
+
 // ============================================================ controller
 // One workgroup: reduces the stage partials, applies accept/reject and the
 // dt update of src/main.cu:321-383 and logs the attempt.
@@ -892,6 +1330,28 @@ void launch_stage(hipStream_t s, const FusedArgs &A)
     }
 }
 
+template <int STAGE, bool PRESS, bool PERI>
+void launch_b64(hipStream_t s, const FusedArgs &A)
+{
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k_block64<kBlockThreads, STAGE, PRESS, PERI>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBlockLds);
+    (void)attr;
+    const size_t lds = (size_t)24 * ((A.TX + 4) * (A.TY + 4) * (A.CZ + 4) + (A.TX + 2) * (A.TY + 2) * (A.CZ + 2));
+    hipLaunchKernelGGL((k_block64<kBlockThreads, STAGE, PRESS, PERI>), dim3(A.nblocks), dim3(kBlockThreads), lds, s, A);
+}
+template <bool PRESS, bool PERI>
+void launch_block64(hipStream_t s, const FusedArgs &A)
+{
+    switch (A.stage) {
+    case 0: launch_b64<0, PRESS, PERI>(s, A); break;
+    case 1: launch_b64<1, PRESS, PERI>(s, A); break;
+    case 2: launch_b64<2, PRESS, PERI>(s, A); break;
+    case 3: launch_b64<3, PRESS, PERI>(s, A); break;
+    case 4: launch_b64<4, PRESS, PERI>(s, A); break;
+    default: launch_b64<5, PRESS, PERI>(s, A); break;
+    }
+}
+
 // Periodic ghost layers of the FP64 positions the controller left current
 // (buffer ctl->cur, read on the device so that graph replays follow the
 // controller's choice): the reference's setGridPeri (src/boundaries.cu:
@@ -970,7 +1430,10 @@ void launch_fused(hipStream_t s, const FusedArgs &A, int f32k)
         launch_fused32(s, A);
     } else {
         const bool peri = A.g.xPeri || A.g.yPeri || A.g.zPeri;
-        if (pr) peri ? launch_stage<kNT64, true, true>(s, A) : launch_stage<kNT64, true, false>(s, A);
+        if (A.block) {
+            if (pr) peri ? launch_block64<true, true>(s, A) : launch_block64<true, false>(s, A);
+            else peri ? launch_block64<false, true>(s, A) : launch_block64<false, false>(s, A);
+        } else if (pr) peri ? launch_stage<kNT64, true, true>(s, A) : launch_stage<kNT64, true, false>(s, A);
         else peri ? launch_stage<kNT64, false, true>(s, A) : launch_stage<kNT64, false, false>(s, A);
     }
 }

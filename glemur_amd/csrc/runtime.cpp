@@ -112,6 +112,7 @@ int stage_max_rect(const gm_ctx *c, int k)
 
 void set_tile_k(gm_ctx *c, int k, int tx, int ty, int cz)
 {
+    if (k < 6) c->block[k] = false;
     c->TX[k] = std::min(tx, c->p.nx);
     c->TY[k] = std::min(ty, c->p.ny);
     c->tiles_x[k] = (c->p.nx + c->TX[k] - 1) / c->TX[k];
@@ -125,12 +126,12 @@ void set_tile_k(gm_ctx *c, int k, int tx, int ty, int cz)
 // (resident workgroups over all CUs) and each marches its chunk plus five
 // planes of pipeline fill, so the launch takes about
 // ceil(chunks x cols / slots) x (ceil(nz / chunks) + 5) plane steps; the
-// fewest such steps, chunks never thinner than 8 planes
+// fewest such steps
 int best_chunks(int nz, int cols, int slots)
 {
     int best = 1;
     long long best_cost = -1;
-    for (int nch = 1; nch <= std::max(1, nz / 8); ++nch) {
+    for (int nch = 1; nch <= std::max(1, nz / 2); ++nch) {
         const long long rounds = ((long long)nch * cols + slots - 1) / slots;
         const long long cost = rounds * ((nz + nch - 1) / nch + 5);
         if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = nch; }
@@ -162,11 +163,11 @@ double rect_lines(int tlx, int tly, int rw, int rh)
 // per CU resident at a time.  (Stage 0 took 512-point rects, two
 // workgroups per CU, while its loads were issued one plane step ahead; with
 // two steps it is faster on the wide rects: 98 -> 92 us at 129 x 129 x 385.)
+void auto_blocks(gm_ctx *c);
 void auto_tiles(gm_ctx *c, int target, bool member)
 {
     const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
     const bool lines = c->prec == GM_PREC_F32K;
-    (void)member;   // ensemble members take the same rule
     for (int k = 0; k < 7; ++k) {
         const int cap = stage_max_rect(c, k);
         int bx = 4, by = 2;
@@ -184,6 +185,58 @@ void auto_tiles(gm_ctx *c, int target, bool member)
         const int nch = best_chunks(nz, c->tiles_x[k] * c->tiles_y[k], target * stage_blocks_per_cu(c, k));
         set_tile_k(c, k, bx, by, (nz + nch - 1) / nch);
     }
+    if (!member) auto_blocks(c);   // ensemble launches march
+}
+
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+int num_blocks(const gm_ctx *c) { return cdiv(c->p.nx, c->BX) * cdiv(c->p.ny, c->BY) * cdiv(c->p.nz, c->BZ); }
+
+// Workgroups (partial results) of a stage launch
+int launch_blocks(const gm_ctx *c, int k) { return k < 6 && c->block[k] ? num_blocks(c) : c->nblocks[k]; }
+
+// Stage kernels that compute blocks at once, and their block.  A plane step
+// of the march takes 0.75 us (FP32) or 2 us (FP64) however few columns a
+// workgroup holds, so on a small grid a launch lasts its fill of the pipeline;
+// a block costs its halo instead (2.7 to 3 positions and 1.8 B a point).
+// Microseconds an attempt, march -> blocks, F32K and FP64:
+//   33 x 33 x 97     152 -> 51     285 -> 72
+//   49 x 49 x 145    166 -> 93     290 -> 162
+//   61 x 47 x 150    205 -> 160    427 -> 303   (pressure, periodic x and y)
+//   65 x 65 x 193    145 -> 173    372 -> 328   (F32K: chunks of six planes)
+//   81 x 81 x 241    212 -> 289    610 -> 612
+// FP64 stages 1 to 4 alone are still faster at 81 x 81 x 241 (85 to 102 ->
+// 70 to 97 us), stages 0 and 5 not (92 -> 115, 154 -> 163); at 97 x 97 x 289
+// stages 3 and 4 are slower.  Hence the limits, in inner points.
+//
+// The block: the fewest rounds over the CUs times a workgroup's time, taken
+// as 2000 + the points of its box (two thirds of a workgroup's time is its
+// chain of latencies).
+constexpr long long kBlockPoints32 = 600000, kBlockPoints64 = 1000000, kBlockPoints64Mid = 2000000;
+void auto_blocks(gm_ctx *c)
+{
+    const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
+    const bool f64 = c->prec == GM_PREC_F64;
+    auto limit = [&](int k) { return !f64 ? kBlockPoints32 : k == 0 || k == 5 ? kBlockPoints64 : kBlockPoints64Mid; };
+    if (c->N > limit(1)) return;
+    double best = 1e300;
+    for (int kx = 1; kx <= nx; ++kx) {
+        const int bx = cdiv(nx, kx);
+        if (bx > 64) continue;
+        for (int ky = 1; ky <= ny; ++ky) {
+            const int by = cdiv(ny, ky);
+            if ((bx + 4) * (by + 4) > gmd::kBlockThreads) continue;   // a thread a column
+            for (int bz = 2; bz <= 16; ++bz) {
+                if (bx * by * bz > gmd::kBlockThreads || 2 * (bx * by + by * bz + bx * bz) > gmd::kBlockThreads) continue;
+                const int box = (bx + 4) * (by + 4) * (bz + 4);
+                const int nb = cdiv(nx, bx) * cdiv(ny, by) * cdiv(nz, bz);
+                const double cost = (double)cdiv(nb, c->ncu) * (2000 + box) + 1e-3 * nb * box / c->ncu;
+                if (cost < best) { best = cost; c->BX = bx; c->BY = by; c->BZ = bz; }
+            }
+        }
+    }
+    if (best < 1e300)
+        for (int k = 0; k < 6; ++k) c->block[k] = c->N <= limit(k);
 }
 
 // Workgroup rounds per launch: one round over the CUs (at each stage
@@ -196,7 +249,7 @@ int default_blocks(const gm_ctx *c)
 int ensure_partials(gm_ctx *c)
 {
     int need = 0;
-    for (int k = 0; k < 7; ++k) need = std::max(need, c->nblocks[k]);
+    for (int k = 0; k < 7; ++k) need = std::max(need, launch_blocks(c, k));
     if (need <= c->part_cap) return GM_OK;
     dfree(c->part_delta);
     dfree(c->part_diag);
@@ -214,6 +267,12 @@ gmd::FusedArgs fused_args(gm_ctx *c, int stage, int emit, int diag, int check_do
     const int k = stage < 0 ? 6 : stage;
     A.TX = c->TX[k]; A.TY = c->TY[k]; A.CZ = c->CZ[k];
     A.tiles_x = c->tiles_x[k]; A.tiles_y = c->tiles_y[k]; A.nchunks = c->nchunks[k]; A.nblocks = c->nblocks[k];
+    if (k < 6 && c->block[k]) {
+        A.block = 1;
+        A.TX = c->BX; A.TY = c->BY; A.CZ = c->BZ;
+        A.tiles_x = cdiv(c->p.nx, c->BX); A.tiles_y = cdiv(c->p.ny, c->BY); A.nchunks = cdiv(c->p.nz, c->BZ);
+        A.nblocks = num_blocks(c);
+    }
     A.emit = emit; A.diag = diag; A.check_done = check_done;
     // an initial distortion (src/init.cu:388-419) moves the x/y ghost
     // layers off the lattice, where the reference's tile-edge rebuilding and
@@ -256,8 +315,8 @@ void enqueue_step(gm_ctx *c, int diag, int check_done)
     C.ctl = c->ctl;
     C.part_delta = c->part_delta;
     C.part_diag = c->part_diag;
-    C.nb_delta = c->nblocks[5];
-    C.nb_diag = c->nblocks[0];
+    C.nb_delta = launch_blocks(c, 5);
+    C.nb_diag = launch_blocks(c, 0);
     C.diag = diag;
     C.nbuf = f32k ? 2 : 3;
     C.maxError = c->p.maxError;
@@ -1285,7 +1344,20 @@ extern "C" int gm_autotune(gm_ctx *c, int reps, double ms_best[6])
         const int stage = k == 6 ? -1 : k;
         const int cap = stage_max_rect(c, k);
         int bTX = c->TX[k], bTY = c->TY[k], bCZ = c->CZ[k];
-        double best = 1e30;
+        double best = 1e30, block_ms = 1e30;
+        auto timed = [&](double &ms) {
+            gmd::FusedArgs A = fused_args(c, stage, 0, stage == 0 ? 1 : 0, 0);
+            gmd::launch_fused(c->stream, A, f32k);   // warm (and first-launch setup)
+            if (hipEventRecord(e0, c->stream) != hipSuccess) return fail(GM_ERR_HIP, "event");
+            for (int i = 0; i < reps; ++i) gmd::launch_fused(c->stream, A, f32k);
+            if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess)
+                return fail(GM_ERR_HIP, "event");
+            float t = 0;
+            (void)hipEventElapsedTime(&t, e0, e1);
+            ms = t / reps;
+            return GM_OK;
+        };
+        if (k < 6 && c->block[k] && (rc = timed(block_ms))) break;
         // per workgroup size: the fewest-points rect and, for F32K, the
         // fewest-lines one
         std::vector<std::pair<int, int>> rects;
@@ -1307,25 +1379,21 @@ extern "C" int gm_autotune(gm_ctx *c, int reps, double ms_best[6])
             int cand[3] = {best_chunks(c->p.nz, cols, slots), slots / cols, 2 * slots / cols};
             for (int q = 0; q < 3; ++q) {
                 const int nch = cand[q] = std::max(1, std::min(cand[q], std::max(1, c->p.nz / 8)));
-                bool timed = false;
-                for (int r = 0; r < q; ++r) timed |= cand[r] == nch;
-                if (timed) continue;
+                bool seen = false;
+                for (int r = 0; r < q; ++r) seen |= cand[r] == nch;
+                if (seen) continue;
                 set_tile_k(c, k, tx, ty, (c->p.nz + nch - 1) / nch);
                 if ((rc = ensure_partials(c))) break;
-                gmd::FusedArgs A = fused_args(c, stage, 0, stage == 0 ? 1 : 0, 0);
-                gmd::launch_fused(c->stream, A, f32k);   // warm (and first-launch setup)
-                if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fail(GM_ERR_HIP, "event"); break; }
-                for (int i = 0; i < reps; ++i) gmd::launch_fused(c->stream, A, f32k);
-                if (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-                    rc = fail(GM_ERR_HIP, "event");
-                    break;
-                }
-                float ms = 0;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                if (ms / reps < best * kTuneKeep) { best = ms / reps; bTX = tx; bTY = ty; bCZ = c->CZ[k]; }
+                double ms = 0;
+                if ((rc = timed(ms))) break;
+                if (ms < best * kTuneKeep) { best = ms; bTX = tx; bTY = ty; bCZ = c->CZ[k]; }
             }
         }
         set_tile_k(c, k, bTX, bTY, bCZ);
+        if (k < 6 && block_ms < 1e30 && best >= block_ms * kTuneKeep) {
+            c->block[k] = true;
+            best = block_ms;
+        }
         if (ms_best && k < 6) ms_best[k] = best;
     }
     (void)hipEventDestroy(e0);

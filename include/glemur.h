@@ -358,7 +358,10 @@ int gm_hbm_probe(int64_t bytes, int mode, int reps, double *ms_mean);
 int gm_set_tile(gm_ctx *ctx, int tx, int ty, int cz);
 int gm_get_tile(gm_ctx *ctx, int *tx, int *ty, int *cz, int *nblocks);
 /* Tile of one stage kernel (stage 0..5, -1 the fields-only pass); each stage
- * kernel has its own (gm_set_tile sets them all alike). */
+ * kernel has its own (gm_set_tile sets them all alike).  On small grids the
+ * stage kernels compute blocks of points at once until a tile is set; the
+ * tile reported is then the one the marching kernels (ensembles among them)
+ * would take. */
 int gm_get_stage_tile(gm_ctx *ctx, int stage, int *tx, int *ty, int *cz, int *nblocks);
 /* Set the tile of one stage kernel (stage 0..5, -1 the fields-only pass):
  * tx x ty output columns per workgroup, z chunks of cz planes.  The rect
