@@ -96,10 +96,8 @@ struct gm_ctx {
     long long ghost_off[6] = {0, 0, 0, 0, 0, 0};
     gmd::StepRecord *log = nullptr;
     int log_cap = 4096;
-    double *red_out = nullptr, *red_host = nullptr;   // 16 doubles each
-    double *extra_part = nullptr;                     // mesh / error diagnostics partials
-    double *diag_scratch = nullptr;
-    int diag_blocks = 2048;
+    double *red_out = nullptr, *red_host = nullptr;   // 16 doubles each, red_host pinned
+    double *row_part = nullptr;                       // partials of a row's reductions
     int *nanflag = nullptr;
     double *xns_part = nullptr;   // per-kernel path: per-block error maxima of k_xnewstar
     int cur = 0;                  // host copy of ctl->cur (valid after syncs)

@@ -89,25 +89,21 @@ void launch_max_final(hipStream_t s, const double *partials, int n, double *out)
 // the static scratch of the allocation-free xNewStar entry point
 long long noalloc_scratch_doubles();
 double *noalloc_scratch(int device);
-// Diagnostics over inner points from B, J (padded SoA) and det:
-// out[0] = B2 (incl. dx dy dz), out[1] = JMax, out[2] = JxB_B2Max,
-// out[3] = JxB_JBMax, out[4] = max|JxB|, out[5] = max |J||B|.  `scratch`
-// holds 6*blocks doubles.
-template <class R>
-void launch_diag(hipStream_t s, const Geo &g, const R *B, const R *J, const double *det, double *scratch,
-                 int max_blocks, double *out);
-
-// Mesh and error diagnostics (src/diagnostics.cu:33-110): out[0] min
-// convexity, out[1] min octant wedge, out[2] errB_1ez, out[3] errXb_XbAn,
-// out[4] epsilon*, each only when its flag is set; per-point cell volume,
+// What a time-series row reduces over inner points, from the positions, B, J
+// (padded SoA) and det: with diag out[0] = B2 (incl. dx dy dz), out[1] = JMax,
+// out[2] = JxB_B2Max, out[3] = JxB_JBMax, out[4] = max|JxB|, out[5] = max
+// |J||B|; mesh and error diagnostics (src/diagnostics.cu:33-110) out[8] min
+// convexity, out[9] min octant wedge (mesh), out[10] errB_1ez, out[11]
+// errXb_XbAn (errs), out[12] epsilon* (eps).  Per-point cell volume,
 // convexity and wedge minimum (inner points, x fastest) when the arrays are
-// given.  part holds extra_diag_parts() doubles.  Returns -1 when nz is too
-// large for epsilon* (more than 3840 planes).
-int extra_diag_parts();
+// given.  part holds row_parts() doubles; out (null: no reductions) may be
+// pinned host memory.  Returns -1 when nz is too large for epsilon* (more
+// than 3840 planes).
+int row_parts();
 template <class R>
-int launch_extra_diag(hipStream_t s, const Geo &g, const double *x64, const float *xh, const float *xl, const R *B,
-                      const R *J, double ar, double az, double phi1, int mesh, int errs, int eps, double *cellVol,
-                      double *convex, double *wedge, double *part, double *out);
+int launch_row(hipStream_t s, const Geo &g, const double *x64, const float *xh, const float *xl, const R *B, const R *J,
+               const double *det, double ar, double az, double phi1, int diag, int mesh, int errs, int eps,
+               double *cellVol, double *convex, double *wedge, double *part, double *out);
 
 // ---- layout conversion between host AoS padded and device SoA --------
 // dst[c*P + a] = src[3a + c] (src in double) with an optional hi/lo split.

@@ -12,14 +12,19 @@ namespace {
 
 constexpr int kB = 256;
 
+// Positions in the precision of R: FP64 component arrays, or FP32 (hi, lo)
+// triples.  Resolved at compile time: with a test per load the loads of the
+// neighbours waited for one another.
+template <class R>
 struct PosRef {
-    const double *x64;
-    const float *xh, *xl;
+    const R *x;
+    const float *lo;
     long long P;
     __device__ void at(long long a, double v[3]) const
     {
         for (int c = 0; c < 3; ++c)
-            v[c] = x64 ? x64[c * P + a] : (double)xh[3 * a + c] + (double)xl[3 * a + c];   // F32K: triples
+            if constexpr (sizeof(R) == 8) v[c] = x[c * P + a];
+            else v[c] = (double)x[3 * a + c] + (double)lo[3 * a + c];
     }
 };
 
@@ -31,24 +36,28 @@ __device__ inline void cross3d(const double *a, const double *b, double *c)
     c[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-// One inner point (i, j, k): the 8 octant wedge products of the edges to
+// One inner point, x0 at padded offset a, zm and zp the positions below and
+// above it: the 8 octant wedge products of the edges to
 // the face neighbours (src/maths.cu:497-570), oriented so that an
 // undistorted cell is positive; convexity -1 when any is negative
 // (src/maths.cu:573-640); the forward-difference cell volume
 // (src/maths.cu:443-494).
-__device__ void mesh_point(const Geo &g, const PosRef &X, int i, int j, int k, double &wmin, double &conv,
-                           double &vol)
+template <class R>
+__device__ void mesh_point(const Geo &g, const PosRef<R> &X, long long a, const double x0[3], const double zm[3],
+                           const double zp[3], double &wmin, double &conv, double &vol)
 {
-    const long long a = gidx(g, i + 1, j + 1, k + 1);
-    double x0[3], xm[3][2][3];
-    X.at(a, x0);
-    const long long st[3] = {1, g.sx, g.sxy};
+    double xm[3][2][3];
+    X.at(a - 1, xm[0][0]);
+    X.at(a + 1, xm[0][1]);
+    X.at(a - g.sx, xm[1][0]);
+    X.at(a + g.sx, xm[1][1]);
+    for (int c = 0; c < 3; ++c) {
+        xm[2][0][c] = zm[c];
+        xm[2][1][c] = zp[c];
+    }
     for (int d = 0; d < 3; ++d)
-        for (int s = 0; s < 2; ++s) {
-            double v[3];
-            X.at(a + (s ? st[d] : -st[d]), v);
-            for (int c = 0; c < 3; ++c) xm[d][s][c] = v[c] - x0[c];
-        }
+        for (int s = 0; s < 2; ++s)
+            for (int c = 0; c < 3; ++c) xm[d][s][c] -= x0[c];
     wmin = 0;
     conv = 1;
     for (int u = 0; u < 2; ++u)
@@ -67,168 +76,286 @@ __device__ void mesh_point(const Geo &g, const PosRef &X, int i, int j, int k, d
     vol = dot3(cr, xm[2][1]);
 }
 
-__global__ void __launch_bounds__(kB) k_mesh(Geo g, PosRef X, double *cellVol, double *convex, double *wedge,
-                                             double *part, int nb)
+// The joining operation of row quantity q (NaN-blind, as findDevMax) and
+// the value it starts from
+__device__ inline double row_join(int q, double a, double b)
 {
-    __shared__ double sw[kB], sc[kB];
-    const long long N = (long long)g.nx * g.ny * g.nz;
-    double wm = 1e300, cm = 1;
-    for (long long t = (long long)blockIdx.x * kB + threadIdx.x; t < N; t += (long long)gridDim.x * kB) {
-        const int i = (int)(t % g.nx), j = (int)((t / g.nx) % g.ny), k = (int)(t / ((long long)g.nx * g.ny));
-        double w, c, v;
-        mesh_point(g, X, i, j, k, w, c, v);
-        if (cellVol) cellVol[t] = v;
-        if (convex) convex[t] = c;
-        if (wedge) wedge[t] = w;
-        wm = w < wm ? w : wm;
-        cm = c < cm ? c : cm;
+    if (q == 0 || q == 8 || q == 9) return a + b;
+    if (q == 6 || q == 7) return b < a ? b : a;
+    return nb_max(a, b);
+}
+__device__ inline double row_start(int q) { return q == 6 ? 1.0 : q == 7 ? 1e300 : 0.0; }
+__device__ inline double wave_min(double v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const double u = __shfl_xor(v, o, 64);
+        v = u < v ? u : v;
     }
-    sw[threadIdx.x] = wm;
-    sc[threadIdx.x] = cm;
-    __syncthreads();
-    for (int s = kB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            sw[threadIdx.x] = fmin(sw[threadIdx.x], sw[threadIdx.x + s]);
-            sc[threadIdx.x] = fmin(sc[threadIdx.x], sc[threadIdx.x + s]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = sc[0];
-        part[nb + blockIdx.x] = sw[0];
-    }
+    return v;
 }
 
-// sums of |B - ez|^2 (src/maths.cu:294-330) and |x - x_an|^2
-// (src/maths.cu:334-377) over inner points
-template <class R>
-__global__ void __launch_bounds__(kB) k_errs(Geo g, PosRef X, const R *B, double ar, double az, double phi1,
-                                             double *part, int nb)
-{
-    __shared__ double s1[kB], s2[kB];
-    const long long N = (long long)g.nx * g.ny * g.nz;
-    double e1 = 0, e2 = 0;
-    for (long long t = (long long)blockIdx.x * kB + threadIdx.x; t < N; t += (long long)gridDim.x * kB) {
-        const int i = (int)(t % g.nx), j = (int)((t / g.nx) % g.ny), k = (int)(t / ((long long)g.nx * g.ny));
-        const long long a = gidx(g, i + 1, j + 1, k + 1);
-        const double b0 = B[a], b1 = B[g.P + a], b2 = (double)B[2 * g.P + a] - 1.;
-        e1 += b0 * b0 + b1 * b1 + b2 * b2;
-        const double x = i * g.dx + g.Ox, y = j * g.dy + g.Oy, z = k * g.dz + g.Oz;
-        const double f = exp(-(x * x + y * y) / (ar * ar) - z * z / (az * az)) * phi1;
-        double p[3];
-        X.at(a, p);
-        const double d0 = p[0] - cos(f) * x - sin(f) * y;
-        const double d1 = p[1] + sin(f) * x - cos(f) * y;
-        const double d2 = p[2] - z;
-        e2 += d0 * d0 + d1 * d1 + d2 * d2;
-    }
-    s1[threadIdx.x] = e1;
-    s2[threadIdx.x] = e2;
-    __syncthreads();
-    for (int s = kB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            s1[threadIdx.x] += s1[threadIdx.x + s];
-            s2[threadIdx.x] += s2[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[2 * nb + blockIdx.x] = s1[0];
-        part[3 * nb + blockIdx.x] = s2[0];
-    }
-}
+// Everything a time-series row reduces over the inner points, in one pass.
+//  - diag: energy density |B|^2 det / 2^(#boundary faces)
+//    (src/maths.cu:647-680), |J|, |JxB|/|B|^2 (src/maths.cu:168-200) and
+//    |JxB|/(|J||B|) (0/0 := 0), and the maxima of |JxB| and |J||B| (their
+//    quotient is the relaxation criterion);
+//  - mesh: convexity and wedge minimum (mesh_point);
+//  - errs: |B - ez|^2 (src/maths.cu:294-330) and |x - x_an|^2
+//    (src/maths.cu:334-377);
+//  - eps: epsilon* (src/maths.cu:204-290): along the column i = nx/2,
+//    j = ny/2, a_k = J.B / B^2 and z_k = z of the position; the maximum over
+//    all pairs of sqrt2 |a_n - a_k| / |z_n - z_k| (pairs with equal z count
+//    0), by neps further workgroups of 16 rows k each.
+// Bound by memory: 56 bytes a point in FP32 (positions 24, B 12, J 12, det
+// 8), read once here and three times by a pass per quantity.  A thread
+// marches KZ planes of one column, so its z neighbours stay in registers
+// and the index divisions are done once; the other neighbours hit in cache.
+// 129 x 129 x 385 (FP32, all quantities): 0.19 ms in one launch, 1.9 TB/s,
+// against 0.6 ms in four launches of 512 workgroups, one wave of them
+// summing their partials serially; what is left is FP64 arithmetic.
+// Partials of a workgroup go to part[q * nb + block], q = energy, |J|max,
+// the four other maxima, convexity, wedge, and the two error sums.
+constexpr int kQ = 10, kRowBlocks = 4096, kEpsRows = 16;
 
-// epsilon* (src/maths.cu:204-290): along the column i = nx/2, j = ny/2,
-// a_k = J.B / B^2 and z_k = z of the position; the maximum over all pairs
-// of sqrt2 |a_n - a_k| / |z_n - z_k| (pairs with equal z count 0).
 template <class R>
-__global__ void __launch_bounds__(kB) k_eps_star(Geo g, PosRef X, const R *B, const R *J, double *part, int nb)
+struct RowArgs {
+    Geo g;
+    PosRef<R> X;
+    const double *det;
+    double ar, az, phi1;
+    int diag, mesh, errs, eps;
+    double *cellVol, *convex, *wedge;
+    int nb, bx, KZ, neps;     // workgroups over points (bx per layer of KZ planes), and of epsilon*
+    double *part;
+};
+
+template <class R>
+__device__ void eps_star_rows(const RowArgs<R> &A, const R *B, const R *J, int blk)
 {
-    extern __shared__ double sh[];
-    double *za = sh, *aa = sh + g.nz;
-    __shared__ double red[kB];
-    const int i = g.nx / 2, j = g.ny / 2;
-    for (int k = threadIdx.x; k < g.nz; k += kB) {
-        const long long a = gidx(g, i + 1, j + 1, k + 1);
+    const Geo &g = A.g;
+    __shared__ double zr[kEpsRows], ar[kEpsRows], red[kB / 64];
+    auto column = [&](int k, double &z, double &al) {
+        const long long a = gidx(g, g.nx / 2 + 1, g.ny / 2 + 1, k + 1);
         const double b[3] = {(double)B[a], (double)B[g.P + a], (double)B[2 * g.P + a]};
         const double jj[3] = {(double)J[a], (double)J[g.P + a], (double)J[2 * g.P + a]};
-        aa[k] = dot3(jj, b) / dot3(b, b);
+        al = dot3(jj, b) / dot3(b, b);
         double p[3];
-        X.at(a, p);
-        za[k] = p[2];
-    }
+        A.X.at(a, p);
+        z = p[2];
+    };
+    const int k0 = blk * kEpsRows, rows = min(kEpsRows, g.nz - k0);
+    if ((int)threadIdx.x < rows) column(k0 + threadIdx.x, zr[threadIdx.x], ar[threadIdx.x]);
     __syncthreads();
     const double SQRT2 = 1.414213562373095;   // the reference's literal (src/global.h:18)
     double m = 0;
-    for (int k = threadIdx.x; k < g.nz; k += kB)
-        for (int n = 0; n < g.nz; ++n)
-            if (za[n] != za[k]) {
-                const double v = SQRT2 * fabs((aa[n] - aa[k]) / (za[n] - za[k]));
+    for (int n = threadIdx.x; n < g.nz; n += kB) {
+        double zn, an;
+        column(n, zn, an);
+        for (int r = 0; r < rows; ++r)
+            if (zn != zr[r]) {
+                const double v = SQRT2 * fabs((an - ar[r]) / (zn - zr[r]));
                 if (v > m) m = v;
             }
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int s = kB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s && red[threadIdx.x + s] > red[threadIdx.x]) red[threadIdx.x] = red[threadIdx.x + s];
-        __syncthreads();
     }
-    if (threadIdx.x == 0) part[4 * nb] = red[0];
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kB / 64; ++q) m = nb_max(m, red[q]);
+        A.part[kQ * A.nb + blk] = m;
+    }
 }
 
-// out[0] = min convexity, out[1] = min wedge, out[2] = errB_1ez,
-// out[3] = errXb_XbAn, out[4] = epsilon*
-__global__ void k_extra_final(const double *part, int nb, long long N, int mesh, int errs, int eps, double *out)
+// errB and errXb of the columns of workgroup blk
+template <class R>
+__device__ void errs_block(const RowArgs<R> &A, const R *B, int blk)
 {
-    if (threadIdx.x != 0) return;
-    if (mesh) {
-        double c = 1, w = 1e300;
-        for (int b = 0; b < nb; ++b) {
-            c = fmin(c, part[b]);
-            w = fmin(w, part[nb + b]);
+    const Geo &g = A.g;
+    const int layer = blk / A.bx, k0 = layer * A.KZ, k1 = min(k0 + A.KZ, g.nz), nxy = g.nx * g.ny;
+    double e1 = 0, e2 = 0;
+    for (int t = (blk - layer * A.bx) * kB + threadIdx.x; t < nxy; t += A.bx * kB) {
+        const int j = t / g.nx, i = t - j * g.nx;
+        long long a = gidx(g, i + 1, j + 1, k0 + 1);
+        const double x = i * g.dx + g.Ox, y = j * g.dy + g.Oy;
+#pragma unroll 1
+        for (int k = k0; k < k1; ++k, a += g.sxy) {
+            double p[3], sf, cf;
+            A.X.at(a, p);
+            const double b0 = B[a], b1 = B[g.P + a], b2 = (double)B[2 * g.P + a] - 1.;
+            e1 += b0 * b0 + b1 * b1 + b2 * b2;
+            const double z = k * g.dz + g.Oz;
+            const double f = exp(-(x * x + y * y) / (A.ar * A.ar) - z * z / (A.az * A.az)) * A.phi1;
+            sincos(f, &sf, &cf);
+            const double d0 = p[0] - cf * x - sf * y;
+            const double d1 = p[1] + sf * x - cf * y;
+            const double d2 = p[2] - z;
+            e2 += d0 * d0 + d1 * d1 + d2 * d2;
         }
-        out[0] = c;
-        out[1] = w;
     }
-    if (errs) {
-        double s1 = 0, s2 = 0;
-        for (int b = 0; b < nb; ++b) {
-            s1 += part[2 * nb + b];
-            s2 += part[3 * nb + b];
+    __shared__ double red[2][kB / 64];
+    const double s1 = wave_sum(e1), s2 = wave_sum(e2);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = s1;
+        red[1][threadIdx.x >> 6] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double v = 0;
+        for (int s = 0; s < kB / 64; ++s) v += red[threadIdx.x][s];
+        A.part[(8 + threadIdx.x) * A.nb + blk] = v;
+    }
+}
+
+// EXTRA: more than the diag quantities is wanted.  With errs every workgroup
+// of points has a second one for the two error sums, eight further on (the
+// same XCD, whose L2 then holds the positions and B): the exponential and
+// angle functions bind the vector units while the rest waits for memory, but
+// in one thread their constants cost it half the waves.
+template <class R, bool EXTRA>
+__global__ void __launch_bounds__(kB, sizeof(R) == 8 ? 3 : 4) k_row(RowArgs<R> A, const R *B, const R *J)
+{
+    // the few workgroups of epsilon* first, their chain is the longest
+    if ((int)blockIdx.x < A.neps) return eps_star_rows(A, B, J, blockIdx.x);
+    int blk = blockIdx.x - A.neps;
+    if (EXTRA && A.errs) {
+        const bool main = A.diag || A.mesh, second = blk >> 3 & 1;
+        if (main) blk = (blk >> 4) * 8 + (blk & 7);
+        if (blk >= A.nb) return;
+        if (!main || second) return errs_block(A, B, blk);
+    }
+    const int layer = blk / A.bx;
+    const Geo &g = A.g;
+    const int k0 = layer * A.KZ, k1 = min(k0 + A.KZ, g.nz), nxy = g.nx * g.ny;
+    double e = 0, jm = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0, cm = 1, wm = 1e300;
+    for (int t = (blk - layer * A.bx) * kB + threadIdx.x; t < nxy; t += A.bx * kB) {
+        const int j = t / g.nx, i = t - j * g.nx;
+        const int bxy = (i == 0) + (j == 0) + (i == g.nx - 1) + (j == g.ny - 1);
+        long long a = gidx(g, i + 1, j + 1, k0 + 1);
+        const long long t0 = (long long)nxy * k0 + t;
+        double xm[3], x0[3], xp[3];
+        if (EXTRA && A.mesh) {
+            A.X.at(a, x0);
+            A.X.at(a - g.sxy, xm);
         }
-        out[2] = sqrt(s1) / sqrt((double)N);
-        out[3] = sqrt(s2) / sqrt((double)N);
+#pragma unroll 1
+        for (int k = k0; k < k1; ++k, a += g.sxy) {
+            if (A.diag) {
+                const double b[3] = {(double)B[a], (double)B[g.P + a], (double)B[2 * g.P + a]};
+                const double jj[3] = {(double)J[a], (double)J[g.P + a], (double)J[2 * g.P + a]};
+                const double b2 = b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
+                e += ldexp(b2 * A.det[a], -(bxy + (k == 0) + (k == g.nz - 1)));
+                double c[3];
+                cross3(jj, b, c);
+                const double nc = sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
+                const double nj = sqrt(jj[0] * jj[0] + jj[1] * jj[1] + jj[2] * jj[2]);
+                const double den = nj * sqrt(b2);
+                jm = nb_max(jm, nj);
+                r1 = nb_max(r1, nc / b2);
+                r2 = nb_max(r2, den > 0 ? nc / den : 0.0);
+                r3 = nb_max(r3, nc);
+                r4 = nb_max(r4, den);
+            }
+            if (!EXTRA || !A.mesh) continue;
+            double w, c, v;
+            A.X.at(a + g.sxy, xp);
+            mesh_point(g, A.X, a, x0, xm, xp, w, c, v);
+            const long long at = t0 + (long long)nxy * (k - k0);
+            if (A.cellVol) A.cellVol[at] = v;
+            if (A.convex) A.convex[at] = c;
+            if (A.wedge) A.wedge[at] = w;
+            wm = w < wm ? w : wm;
+            cm = c < cm ? c : cm;
+            for (int q = 0; q < 3; ++q) { xm[q] = x0[q]; x0[q] = xp[q]; }
+        }
     }
-    if (eps) out[4] = part[4 * nb];
+    __shared__ double red[kQ][kB / 64];
+    const int w = threadIdx.x >> 6;
+    auto put = [&](int q, double v) { if ((threadIdx.x & 63) == 0) red[q][w] = v; };
+    if (A.diag) {
+        put(0, wave_sum(e));
+        put(1, wave_max(jm));
+        put(2, wave_max(r1));
+        put(3, wave_max(r2));
+        put(4, wave_max(r3));
+        put(5, wave_max(r4));
+    }
+    if (EXTRA) {
+        put(6, wave_min(cm));
+        put(7, wave_min(wm));
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < (EXTRA ? 8 : 6)) {
+        const int q = threadIdx.x;
+        double v = red[q][0];
+        for (int s = 1; s < kB / 64; ++s) v = row_join(q, v, red[q][s]);
+        A.part[q * A.nb + blk] = v;
+    }
+}
+
+// out[0..5] the diag quantities, out[8] min convexity, out[9] min wedge,
+// out[10] errB_1ez, out[11] errXb_XbAn, out[12] epsilon*: a wave each
+template <class R>
+__global__ void __launch_bounds__(64 * (kQ + 1)) k_row_final(RowArgs<R> A, long long N, double *out)
+{
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (q < 6 ? !A.diag : q < 8 ? !A.mesh : q < kQ ? !A.errs : !A.eps) return;
+    const int n = q < kQ ? A.nb : A.neps;
+    const double *p = A.part + q * A.nb;
+    double v = row_start(q);
+    for (int i = lane; i < n; i += 64 * 8) {   // eight loads in flight a lane
+        double u[8];
+        for (int r = 0; r < 8; ++r) u[r] = p[min(i + 64 * r, n - 1)];
+        for (int r = 0; r < 8; ++r) v = row_join(q, v, i + 64 * r < n ? u[r] : row_start(q));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = row_join(q, v, __shfl_xor(v, o, 64));
+    if (lane != 0) return;
+    if (q == 0) v = v * A.g.dx * A.g.dy * A.g.dz;
+    if (q == 8 || q == 9) v = sqrt(v) / sqrt((double)N);
+    out[q < 6 ? q : q + 2] = v;
 }
 
 }  // namespace
 
-int extra_diag_parts() { return 4 * 512 + 1; }
+int row_parts() { return kQ * kRowBlocks + 3840 / kEpsRows; }
 
 template <class R>
-int launch_extra_diag(hipStream_t s, const Geo &g, const double *x64, const float *xh, const float *xl, const R *B,
-                      const R *J, double ar, double az, double phi1, int mesh, int errs, int eps, double *cellVol,
-                      double *convex, double *wedge, double *part, double *out)
+int launch_row(hipStream_t s, const Geo &g, const double *x64, const float *xh, const float *xl, const R *B, const R *J,
+               const double *det, double ar, double az, double phi1, int diag, int mesh, int errs, int eps,
+               double *cellVol, double *convex, double *wedge, double *part, double *out)
 {
-    const int nb = 512;
-    const PosRef X{x64, xh, xl, g.P};
-    if (mesh || cellVol || convex || wedge)
-        hipLaunchKernelGGL(k_mesh, dim3(nb), dim3(kB), 0, s, g, X, cellVol, convex, wedge, part, nb);
-    if (errs) hipLaunchKernelGGL(k_errs<R>, dim3(nb), dim3(kB), 0, s, g, X, B, ar, az, phi1, part, nb);
-    if (eps) {
-        const size_t lds = 2 * (size_t)g.nz * sizeof(double);
-        if (lds > 60 * 1024) return -1;
-        hipLaunchKernelGGL(k_eps_star<R>, dim3(1), dim3(kB), lds, s, g, X, B, J, part, nb);
-    }
-    hipLaunchKernelGGL(k_extra_final, dim3(1), dim3(64), 0, s, part, nb, (long long)g.nx * g.ny * g.nz, mesh, errs,
-                       eps, out);
+    if (eps && g.nz > 3840) return -1;
+    const bool maps = cellVol || convex || wedge, extra = mesh || errs || maps;
+    PosRef<R> X{nullptr, xl, g.P};
+    if constexpr (sizeof(R) == 8) X.x = x64;
+    else X.x = xh;
+    RowArgs<R> A{g, X, det, ar, az, phi1, diag, mesh || maps, errs, eps, cellVol, convex, wedge,
+              0, 0, 0, 0, part};
+    // as many planes a thread as leave at most kRowBlocks workgroups: one on
+    // small grids (more workgroups), 7 at 129 x 129 x 385
+    const long long cols = ((long long)g.nx * g.ny + kB - 1) / kB;
+    A.bx = (int)(cols < kRowBlocks ? cols : kRowBlocks);
+    const int layers = kRowBlocks / A.bx;
+    A.KZ = (g.nz + layers - 1) / layers;
+    A.nb = diag || extra ? A.bx * ((g.nz + A.KZ - 1) / A.KZ) : 0;
+    A.neps = eps ? (g.nz + kEpsRows - 1) / kEpsRows : 0;
+    const bool two = errs && (diag || A.mesh);
+    const dim3 grid(A.neps + (two ? 2 * ((A.nb + 7) / 8 * 8) : A.nb));
+    if (extra)
+        hipLaunchKernelGGL((k_row<R, true>), grid, dim3(kB), 0, s, A, B, J);
+    else
+        hipLaunchKernelGGL((k_row<R, false>), grid, dim3(kB), 0, s, A, B, J);
+    A.mesh = mesh;
+    if (out)
+        hipLaunchKernelGGL(k_row_final<R>, dim3(1), dim3(64 * (kQ + 1)), 0, s, A, (long long)g.nx * g.ny * g.nz, out);
     return 0;
 }
-template int launch_extra_diag<double>(hipStream_t, const Geo &, const double *, const float *, const float *,
-                                       const double *, const double *, double, double, double, int, int, int,
-                                       double *, double *, double *, double *, double *);
-template int launch_extra_diag<float>(hipStream_t, const Geo &, const double *, const float *, const float *,
-                                      const float *, const float *, double, double, double, int, int, int, double *,
-                                      double *, double *, double *, double *);
+template int launch_row<double>(hipStream_t, const Geo &, const double *, const float *, const float *, const double *,
+                                const double *, const double *, double, double, double, int, int, int, int, double *,
+                                double *, double *, double *, double *);
+template int launch_row<float>(hipStream_t, const Geo &, const double *, const float *, const float *, const float *,
+                               const float *, const double *, double, double, double, int, int, int, int, double *,
+                               double *, double *, double *, double *);
 
 }  // namespace gmd

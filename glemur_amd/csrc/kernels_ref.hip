@@ -633,79 +633,6 @@ __global__ void __launch_bounds__(kBlock) k_inner_aos_to_padded(Geo g, const dou
     for (int l = 0; l < 3; ++l) dst[l * g.P + a] = src[3 * t + l];
 }
 
-// ------------------------------------------------------------ diagnostics
-// Per point: energy density |B|^2 det / 2^(#boundary faces)
-// (src/maths.cu:647-680), |J|, |JxB|/|B|^2 (src/maths.cu:168-200) and
-// |JxB|/(|J||B|) (0/0 := 0), and the maxima of |JxB| and |J||B| (their
-// quotient is the relaxation criterion); grid-stride, per-block partials.
-template <class R>
-__global__ void __launch_bounds__(kBlock) k_diag(Geo g, const R *B, const R *J, const double *det, double *part,
-                                                 int nblk)
-{
-    __shared__ double red[6][kBlock / 64];
-    long long N = (long long)g.nx * g.ny * g.nz;
-    double e = 0, jm = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0;
-    for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < N; t += (long long)gridDim.x * blockDim.x) {
-        int i = (int)(t % g.nx), j = (int)((t / g.nx) % g.ny), k = (int)(t / ((long long)g.nx * g.ny));
-        long long a = gidx(g, i + 1, j + 1, k + 1);
-        double b[3] = {(double)B[a], (double)B[g.P + a], (double)B[2 * g.P + a]};
-        double jj[3] = {(double)J[a], (double)J[g.P + a], (double)J[2 * g.P + a]};
-        double v = (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) * det[a];
-        int bound = (i == 0) + (j == 0) + (k == 0) + (i == g.nx - 1) + (j == g.ny - 1) + (k == g.nz - 1);
-        bound = 1 << bound;
-        v /= bound;
-        e += v;
-        double c[3];
-        cross3(jj, b, c);
-        double nc = sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
-        double nj = sqrt(jj[0] * jj[0] + jj[1] * jj[1] + jj[2] * jj[2]);
-        double b2 = b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
-        double nb = sqrt(b2);
-        jm = nb_max(jm, nj);
-        r1 = nb_max(r1, nc / b2);
-        double den = nj * nb;
-        r2 = nb_max(r2, den > 0 ? nc / den : 0.0);
-        r3 = nb_max(r3, nc);
-        r4 = nb_max(r4, den);
-    }
-    e = wave_sum(e);
-    jm = wave_max(jm);
-    r1 = wave_max(r1);
-    r2 = wave_max(r2);
-    r3 = wave_max(r3);
-    r4 = wave_max(r4);
-    int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[0][w] = e;
-        red[1][w] = jm;
-        red[2][w] = r1;
-        red[3][w] = r2;
-        red[4][w] = r3;
-        red[5][w] = r4;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0, a[5] = {0, 0, 0, 0, 0};
-        for (int q = 0; q < kBlock / 64; ++q) {
-            s += red[0][q];
-            for (int m = 0; m < 5; ++m) a[m] = nb_max(a[m], red[m + 1][q]);
-        }
-        part[blockIdx.x] = s;
-        for (int m = 0; m < 5; ++m) part[(m + 1) * nblk + blockIdx.x] = a[m];
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_diag_final(Geo g, const double *part, int nblk, double *out)
-{
-    // one wave per quantity, fixed order
-    int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (q >= 6) return;
-    double v = 0;
-    for (int i = lane; i < nblk; i += 64) v = q == 0 ? v + part[i] : nb_max(v, part[q * nblk + i]);
-    v = q == 0 ? wave_sum(v) : wave_max(v);
-    if (lane == 0) out[q] = q == 0 ? v * g.dx * g.dy * g.dz : v;
-}
-
 // ------------------------------------------------------------ layouts
 __global__ void k_aos_to_soa_f64(long long P, const double *src, double *dst)
 {
@@ -921,18 +848,6 @@ void launch_max_final(hipStream_t s, const double *partials, int n, double *out)
 {
     hipLaunchKernelGGL(k_max_final, dim3(1), dim3(1024), 0, s, partials, n, out);
 }
-template <class R>
-void launch_diag(hipStream_t s, const Geo &g, const R *B, const R *J, const double *det, double *scratch,
-                 int max_blocks, double *out)
-{
-    int nb = blocks_for(ninner(g));
-    if (nb > max_blocks) nb = max_blocks;
-    hipLaunchKernelGGL(k_diag<R>, dim3(nb), dim3(kBlock), 0, s, g, B, J, det, scratch, nb);
-    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(6 * 64), 0, s, g, scratch, nb, out);  // one wave per quantity
-}
-template void launch_diag<double>(hipStream_t, const Geo &, const double *, const double *, const double *, double *, int, double *);
-template void launch_diag<float>(hipStream_t, const Geo &, const float *, const float *, const double *, double *, int, double *);
-
 void launch_aos_to_soa_f64(hipStream_t s, long long P, const double *src, double *dst)
 {
     hipLaunchKernelGGL(k_aos_to_soa_f64, dim3(blocks_for(P)), dim3(kBlock), 0, s, P, src, dst);

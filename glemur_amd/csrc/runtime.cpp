@@ -461,8 +461,7 @@ extern "C" int gm_create(const gm_params *pp, int precision, gm_ctx **out)
     c->ctlh->n_cycle = 1LL << 62;
     c->ctlh->max_attempt = 1LL << 62;
     if ((r = dalloc(&c->log, (size_t)c->log_cap))) return bail(r);
-    if ((r = dalloc(&c->red_out, 16)) || (r = dalloc(&c->diag_scratch, (size_t)6 * c->diag_blocks)) ||
-        (r = dalloc(&c->extra_part, (size_t)gmd::extra_diag_parts())) ||
+    if ((r = dalloc(&c->red_out, 16)) || (r = dalloc(&c->row_part, (size_t)gmd::row_parts())) ||
         (r = dalloc(&c->nanflag, 1)))
         return bail(r);
     if (hipHostMalloc((void **)&c->red_host, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)
@@ -490,7 +489,7 @@ extern "C" int gm_destroy(gm_ctx *c)
     dfree(c->B0_32); dfree(c->K32); dfree(c->B32); dfree(c->J32); dfree(c->G32);
     dfree(c->det); dfree(c->epsx); dfree(c->epsy); dfree(c->epsz);
     dfree(c->ctl); dfree(c->part_delta); dfree(c->part_diag); dfree(c->tab_dev); dfree(c->log); dfree(c->ghost);
-    dfree(c->red_out); dfree(c->diag_scratch); dfree(c->nanflag); dfree(c->extra_part); dfree(c->xns_part);
+    dfree(c->red_out); dfree(c->row_part); dfree(c->nanflag); dfree(c->xns_part);
     if (c->ctlh) (void)hipHostFree(c->ctlh);
     if (c->red_host) (void)hipHostFree(c->red_host);
     c->tm.destroy();
@@ -595,7 +594,7 @@ extern "C" int gm_synchronize(gm_ctx *c)
     return GM_OK;
 }
 
-static int extra_diag(gm_ctx *c, int mesh, int errs, int eps, double *cellVol, double *convex, double *wedge);
+static int row_diag(gm_ctx *c, int diag, int mesh, int errs, int eps, double *cellVol, double *convex, double *wedge);
 
 extern "C" int gm_download(gm_ctx *c, int field, double *host)
 {
@@ -649,7 +648,7 @@ extern "C" int gm_download(gm_ctx *c, int field, double *host)
     case GM_FIELD_WEDGEMIN: {
         n = (size_t)c->N;
         if ((r = dalloc(&tmp, n))) return r;
-        r = extra_diag(c, 0, 0, 0, field == GM_FIELD_CELLVOL ? tmp : nullptr, field == GM_FIELD_CONVEXITY ? tmp : nullptr,
+        r = row_diag(c, 0, 0, 0, 0, field == GM_FIELD_CELLVOL ? tmp : nullptr, field == GM_FIELD_CONVEXITY ? tmp : nullptr,
                        field == GM_FIELD_WEDGEMIN ? tmp : nullptr);
         if (r) { dfree(tmp); return r; }
         break;
@@ -846,18 +845,21 @@ extern "C" int gm_accept(gm_ctx *c)
     return push_ctl(c);
 }
 
-// Mesh / error diagnostics of the current state into red_out[8..12] and,
-// when given, per-point device arrays (inner points).
-static int extra_diag(gm_ctx *c, int mesh, int errs, int eps, double *cellVol, double *convex, double *wedge)
+// Reductions of the current state into red_host (when any flag is set) and,
+// when given, per-point device arrays (inner points).  The last kernel
+// writes red_host itself: valid once the stream has been waited for.
+static int row_diag(gm_ctx *c, int diag, int mesh, int errs, int eps, double *cellVol, double *convex, double *wedge)
 {
     const bool f64 = c->prec == GM_PREC_F64;
     const int k = c->cur;
-    const int rc = f64 ? gmd::launch_extra_diag<double>(c->stream, c->geo, c->X64[k], nullptr, nullptr, c->B64, c->J64,
-                                                        c->p.ar, c->p.az, c->p.phi1, mesh, errs, eps, cellVol, convex,
-                                                        wedge, c->extra_part, c->red_out + 8)
-                       : gmd::launch_extra_diag<float>(c->stream, c->geo, nullptr, c->Xh[k], c->Xl[k], c->B32, c->J32,
-                                                       c->p.ar, c->p.az, c->p.phi1, mesh, errs, eps, cellVol, convex,
-                                                       wedge, c->extra_part, c->red_out + 8);
+    const gm_params &p = c->p;
+    double *out = diag || mesh || errs || eps ? c->red_host : nullptr;
+    const int rc = f64 ? gmd::launch_row<double>(c->stream, c->geo, c->X64[k], nullptr, nullptr, c->B64, c->J64, c->det,
+                                                 p.ar, p.az, p.phi1, diag, mesh, errs, eps, cellVol, convex, wedge,
+                                                 c->row_part, out)
+                       : gmd::launch_row<float>(c->stream, c->geo, nullptr, c->Xh[k], c->Xl[k], c->B32, c->J32, c->det,
+                                                p.ar, p.az, p.phi1, diag, mesh, errs, eps, cellVol, convex, wedge,
+                                                c->row_part, out);
     if (rc) return fail(GM_ERR_UNSUPPORTED, "epsilonStar: more than 3840 planes along z");
     HIPCHK(hipGetLastError());
     return GM_OK;
@@ -866,18 +868,11 @@ static int extra_diag(gm_ctx *c, int mesh, int errs, int eps, double *cellVol, d
 extern "C" int gm_reductions(gm_ctx *c, gm_reduction *red)
 {
     if (!c || !red) return fail(GM_ERR_ARG, "gm_reductions: null pointer");
-    if (c->prec == GM_PREC_F64)
-        gmd::launch_diag<double>(c->stream, c->geo, c->B64, c->J64, c->det, c->diag_scratch, c->diag_blocks, c->red_out);
-    else
-        gmd::launch_diag<float>(c->stream, c->geo, c->B32, c->J32, c->det, c->diag_scratch, c->diag_blocks, c->red_out);
     const gm_params &p = c->p;
     const int mesh = p.redConvex || p.redWedgeMin, errs = p.redErrB_1ez || p.redErrXb_XbAn, eps = p.redEpsilonStar;
-    if (mesh || errs || eps) {
-        if (int r = extra_diag(c, mesh, errs, eps, nullptr, nullptr, nullptr)) return r;
-    }
+    if (int r = row_diag(c, 1, mesh, errs, eps, nullptr, nullptr, nullptr)) return r;
     const bool udiag = p.inertia && (p.redU2 || p.redUMax);
-    if (udiag) gmd::launch_u_diag(c->stream, c->geo, c->U64[c->ucur], c->det, c->diag_scratch, c->red_out + 13);
-    HIPCHK(hipMemcpyAsync(c->red_host, c->red_out, 16 * 8, hipMemcpyDeviceToHost, c->stream));
+    if (udiag) gmd::launch_u_diag(c->stream, c->geo, c->U64[c->ucur], c->det, c->row_part, c->red_host + 13);
     HIPCHK(hipStreamSynchronize(c->stream));
     memset(red, 0, sizeof *red);
     if (udiag) {
@@ -981,8 +976,7 @@ static int step_per_kernel(gm_ctx *c)
     if (h.done) return GM_OK;
     int r;
     if ((r = fields_per_kernel(c))) return r;
-    gmd::launch_diag<double>(c->stream, c->geo, c->B64, c->J64, c->det, c->diag_scratch, c->diag_blocks, c->red_out);
-    HIPCHK(hipMemcpyAsync(c->red_host, c->red_out, 6 * 8, hipMemcpyDeviceToHost, c->stream));
+    if ((r = row_diag(c, 1, 0, 0, 0, nullptr, nullptr, nullptr))) return r;
     HIPCHK(hipStreamSynchronize(c->stream));
     const double *d = c->red_host;
     const double crit = d[5] > 0 ? d[4] / d[5] : 0.0;
