@@ -15,6 +15,7 @@
 #include "gm_device.hpp"
 #include "gm_fused.hpp"
 #include "gm_internal.hpp"
+#include "transfer.hpp"
 
 using gm::fail;
 
@@ -386,6 +387,7 @@ extern "C" int gm_create(const gm_params *pp, int precision, gm_ctx **out)
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail(GM_ERR_HIP, "no HIP device");
     gm_ctx *c = new gm_ctx();
+    gm::staging_retain();
     c->p = *pp;
     c->prec = precision;
     (void)hipGetDevice(&c->device);
@@ -494,6 +496,7 @@ extern "C" int gm_destroy(gm_ctx *c)
     if (c->red_host) (void)hipHostFree(c->red_host);
     c->tm.destroy();
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    gm::staging_release();
     delete c;
     return GM_OK;
 }
@@ -506,13 +509,13 @@ extern "C" int gm_upload(gm_ctx *c, const double *B0, const double *xb, double t
     int r;
     if ((r = dalloc(&stage, P3))) return r;
     auto s = c->stream;
-    HIPCHK(hipMemcpyAsync(stage, xb, P3 * 8, hipMemcpyHostToDevice, s));
+    HIPCHK(gm::copy_to_device(s, stage, xb, P3 * 8));
     if (c->prec == GM_PREC_F64) {
         for (int i = 0; i < 3; ++i) gmd::launch_aos_to_soa_f64(s, c->P, stage, c->X64[i]);
     } else {
         for (int i = 0; i < 2; ++i) gmd::launch_aos_to_soa_f32k(s, c->P, stage, c->Xh[i], c->Xl[i]);
     }
-    HIPCHK(hipMemcpyAsync(stage, B0, P3 * 8, hipMemcpyHostToDevice, s));
+    HIPCHK(gm::copy_to_device(s, stage, B0, P3 * 8));
     if (c->prec == GM_PREC_F64) {
         gmd::launch_aos_to_soa_f64(s, c->P, stage, c->B0_64);
         // B starts as a copy of B0 (src/main.cu:195); ghost edges keep it
@@ -560,7 +563,7 @@ extern "C" int gm_upload_velocity(gm_ctx *c, const double *uu)
     double *stage = nullptr;
     int r = dalloc(&stage, N3);
     if (r) return r;
-    HIPCHK(hipMemcpyAsync(stage, uu, N3 * 8, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(gm::copy_to_device(c->stream, stage, uu, N3 * 8));
     gmd::launch_inner_aos_to_padded(c->stream, c->geo, stage, c->U64[c->ucur]);
     HIPCHK(hipStreamSynchronize(c->stream));
     dfree(stage);
@@ -632,8 +635,7 @@ extern "C" int gm_download(gm_ctx *c, int field, double *host)
         break;
     }
     case GM_FIELD_DETJAC:
-        HIPCHK(hipMemcpyAsync(host, c->det, c->P * 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
+        HIPCHK(gm::copy_to_host(s, host, c->det, c->P * 8));
         return GM_OK;
     case GM_FIELD_J:
     case GM_FIELD_GRADP: {
@@ -670,8 +672,7 @@ extern "C" int gm_download(gm_ctx *c, int field, double *host)
                 gmd::launch_padded_to_inner_aos<double>(s, c->geo, c->KU64 + m * P3, tmp + (6 + m) * N3);
             }
             std::vector<double> h(n);
-            hipError_t e = hipMemcpyAsync(h.data(), tmp, n * 8, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
+            hipError_t e = gm::copy_to_host(s, h.data(), tmp, n * 8);
             dfree(tmp);
             if (e != hipSuccess) return fail(GM_ERR_HIP, std::string("download: ") + hipGetErrorString(e));
             const size_t N = (size_t)c->N;
@@ -695,8 +696,7 @@ extern "C" int gm_download(gm_ctx *c, int field, double *host)
     default:
         return fail(GM_ERR_ARG, "unknown field");
     }
-    hipError_t e = hipMemcpyAsync(host, tmp, n * 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipError_t e = gm::copy_to_host(s, host, tmp, n * 8);
     dfree(tmp);
     if (e != hipSuccess) return fail(GM_ERR_HIP, std::string("download: ") + hipGetErrorString(e));
     return GM_OK;
