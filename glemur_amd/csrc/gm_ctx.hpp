@@ -75,11 +75,11 @@ struct gm_ctx {
     long long P = 0, N = 0;
     // F64
     double *X64[3] = {nullptr, nullptr, nullptr};
-    double *B0_64 = nullptr, *K64 = nullptr, *B64 = nullptr, *J64 = nullptr, *G64 = nullptr, *Xtmp64 = nullptr;
+    double *B0_64 = nullptr, *K64 = nullptr, *B64 = nullptr, *J64 = nullptr, *G64 = nullptr;
     // F64 with inertia: velocity (padded SoA, inner points used; U64[ucur]
-    // current, the other the candidate of the last attempt), its stage copy
-    // and six velocity slopes
-    double *U64[2] = {nullptr, nullptr}, *Utmp64 = nullptr, *KU64 = nullptr;
+    // current, the other the candidate of the last attempt) and six velocity
+    // slopes
+    double *U64[2] = {nullptr, nullptr}, *KU64 = nullptr;
     int ucur = 0;
     // F32K
     float *Xh[2] = {nullptr, nullptr}, *Xl[2] = {nullptr, nullptr};
@@ -96,7 +96,7 @@ struct gm_ctx {
     long long ghost_off[6] = {0, 0, 0, 0, 0, 0};
     gmd::StepRecord *log = nullptr;
     int log_cap = 4096;
-    double *red_out = nullptr, *red_host = nullptr;   // 16 doubles each, red_host pinned
+    double *red_host = nullptr;                       // results of reductions, 16 doubles, pinned
     double *row_part = nullptr;                       // partials of a row's reductions
     int *nanflag = nullptr;
     double *xns_part = nullptr;   // per-kernel path: per-block error maxima of k_xnewstar

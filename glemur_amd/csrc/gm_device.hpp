@@ -69,12 +69,14 @@ void launch_jstokes(hipStream_t s, const Geo &g, const double *X, const double *
 void launch_jclassic(hipStream_t s, const Geo &g, const double *X, const double *B0, const double *det, double *J);
 void launch_jstokes4th(hipStream_t s, const Geo &g, const double *X, const double *B, double *J);
 void launch_gradp(hipStream_t s, const Geo &g, const double *X, const double *det, double *G);
-// With g.inertia, K holds the position slopes dt u, KU the velocity slopes
-// and U / Utmp the stage velocity (padded SoA, like the positions); det is
-// read only then.  Without inertia U, KU, Utmp and det may be null.
-void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X,
-               const double *B, const double *J, const double *G, double *K, double *Xtmp, const double *det,
-               const double *U, double *KU, double *Utmp);
+// B and det of inner points and of every ghost face (the two above in one launch)
+void launch_b_all(hipStream_t s, const Geo &g, const double *X, const double *B0, double *B, double *det);
+// Slope n (0..5) and the stage positions, which replace X.  With g.inertia,
+// K holds the position slopes dt u, KU the velocity slopes, and the stage
+// velocity replaces U (padded SoA, like the positions); det is read only
+// then.  Without inertia U, KU and det may be null.
+void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, double *X, const double *B,
+               const double *J, const double *G, double *K, const double *det, double *U, double *KU);
 // x_new (and u_new with inertia) and per-block error maxima of the
 // positions; returns the number of partials written.
 int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const double *X, const double *K,
@@ -84,8 +86,9 @@ int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const doubl
 void launch_u_diag(hipStream_t s, const Geo &g, const double *U, const double *det, double *part, double *out);
 // dst (padded SoA, inner points) <- src (inner AoS 3N)
 void launch_inner_aos_to_padded(hipStream_t s, const Geo &g, const double *src, double *dst);
-// Final NaN-blind max of n partials into out[0].
-void launch_max_final(hipStream_t s, const double *partials, int n, double *out);
+// Final NaN-blind max of n partials into out[0] and the NaN flag into out[1]
+// (out may be pinned host memory).
+void launch_max_final(hipStream_t s, const double *partials, int n, const int *nanflag, double *out);
 // the static scratch of the allocation-free xNewStar entry point
 long long noalloc_scratch_doubles();
 double *noalloc_scratch(int device);

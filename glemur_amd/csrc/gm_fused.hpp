@@ -61,6 +61,16 @@ struct CtlArgs {
     double maxError, dtMin, cell;     // cell = dx dy dz
     StepRecord *log;
     int log_cap;
+    Ctl *mirror;                      // pinned copy of the block after the attempt (may be null)
+};
+
+// Start of a run: n_cycle accepted steps and attempts more from here (<= 0:
+// no limit)
+struct ArmArgs {
+    Ctl *ctl;
+    double stop_ratio, ev_dump, ev_save;
+    long long n_cycle, attempts;
+    int reset_diag;
 };
 
 // Block launches (FusedArgs::block): threads a workgroup, at least the points
@@ -89,6 +99,8 @@ void launch_set_grid_peri32(hipStream_t s, const Geo &g, float *const Xh[2], flo
 // FP64 periodic ghost layers of the positions in buffer ctl->cur (read on the device)
 void launch_set_grid_peri64(hipStream_t s, const FusedArgs &A);
 void launch_controller(hipStream_t s, const CtlArgs &A);
+void launch_arm(hipStream_t s, const ArmArgs &A);
+void launch_put(hipStream_t s, Ctl *ctl, const Ctl &h, StepRecord *log, const StepRecord &rec);
 // Ensemble launches: every workgroup of n instances in one launch of the
 // FP32 stage kernel in `nt`-thread workgroups (512, or 768 / 1024 where the
 // stage is built for them), and one controller workgroup per instance.

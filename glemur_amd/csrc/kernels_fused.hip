@@ -1192,6 +1192,10 @@ __device__ __forceinline__ void controller_body(const CtlArgs &A)
     }
     __syncthreads();
     if (threadIdx.x != 0 || h.done) return;
+    auto leave = [&] {
+        *ctl = h;
+        if (A.mirror) *A.mirror = h;   // pinned: the host waits for the stream only
+    };
     double md = 0, es = 0, jmx = 0, rr1 = 0, rr2 = 0, rr3 = 0, rr4 = 0;
     for (int q = 0; q < (int)(blockDim.x >> 6); ++q) {
         md = nb_max(md, red[0][q]);
@@ -1231,7 +1235,7 @@ __device__ __forceinline__ void controller_body(const CtlArgs &A)
         h.accepted = 0;
         rec.accepted = -1;
         if (A.log) A.log[h.n_attempt % A.log_cap] = rec;
-        *ctl = h;
+        leave();
         return;
     }
     const double dt = h.dt;
@@ -1256,10 +1260,38 @@ __device__ __forceinline__ void controller_body(const CtlArgs &A)
     else if (!(h.dt > A.dtMin)) { h.done = 1; h.stop_reason = 2; }
     else if (h.n_attempt >= h.max_attempt) { h.done = 1; h.stop_reason = 4; }
     else if (h.event) { h.done = 1; h.stop_reason = 5; }
-    *ctl = h;
+    leave();
 }
 
 __global__ void __launch_bounds__(kCtlThreads) k_controller(CtlArgs A) { controller_body(A); }
+
+// Start of a run: limits and flags, set where the state is.  A copy of the
+// block to the host and back costs two round trips (10 us each on a 72 us
+// attempt of the 33 x 33 x 97 grid in FP64), this 3 us.
+__global__ void k_arm(ArmArgs A)
+{
+    if (threadIdx.x != 0) return;
+    Ctl &h = *A.ctl;
+    h.done = 0;
+    h.converged = 0;
+    h.stop_reason = 0;
+    h.nan_seen = 0;
+    h.event = 0;
+    if (A.reset_diag) h.diag_valid = 0;
+    h.stop_ratio = A.stop_ratio;
+    h.ev_dump = A.ev_dump;
+    h.ev_save = A.ev_save;
+    h.n_cycle = A.n_cycle > 0 ? h.n_accept + A.n_cycle : 1LL << 62;
+    h.max_attempt = A.attempts > 0 ? h.n_attempt + A.attempts : 1LL << 62;
+}
+
+// The host's control block and the record of an attempt, by value
+__global__ void k_put(Ctl *ctl, Ctl h, StepRecord *log, StepRecord rec)
+{
+    if (threadIdx.x != 0) return;
+    *ctl = h;
+    *log = rec;
+}
 
 // Ensemble: one workgroup per instance.
 __global__ void __launch_bounds__(kCtlThreads) k_controller_batch(const CtlArgs *__restrict__ args)
@@ -1461,6 +1493,13 @@ void launch_set_grid_peri64(hipStream_t s, const FusedArgs &A)
 void launch_controller(hipStream_t s, const CtlArgs &A)
 {
     hipLaunchKernelGGL(k_controller, dim3(1), dim3(kCtlThreads), 0, s, A);
+}
+
+void launch_arm(hipStream_t s, const ArmArgs &A) { hipLaunchKernelGGL(k_arm, dim3(1), dim3(64), 0, s, A); }
+
+void launch_put(hipStream_t s, Ctl *ctl, const Ctl &h, StepRecord *log, const StepRecord &rec)
+{
+    hipLaunchKernelGGL(k_put, dim3(1), dim3(64), 0, s, ctl, h, log, rec);
 }
 
 void launch_controller_batch(hipStream_t s, const CtlArgs *args, int n)

@@ -30,9 +30,9 @@ __device__ __forceinline__ void ld3(const double *F, long long P, long long a, d
 }
 
 // ---------------------------------------------------------------- B_JacB0
-__global__ void __launch_bounds__(kBlock) k_b_jacb0(Geo g, const double *X, const double *B0, double *B, double *det)
+__device__ __forceinline__ void b_jacb0_point(const Geo &g, const double *X, const double *B0, double *B, double *det,
+                                              long long t)
 {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     long long N = (long long)g.nx * g.ny * g.nz;
     if (t >= N) return;
     int i = (int)(t % g.nx) + 1, j = (int)((t / g.nx) % g.ny) + 1, k = (int)(t / ((long long)g.nx * g.ny)) + 1;
@@ -56,6 +56,10 @@ __global__ void __launch_bounds__(kBlock) k_b_jacb0(Geo g, const double *X, cons
     B[g.P + a] = b[1];
     B[2 * g.P + a] = b[2];
     det[a] = 1. / detJac1;
+}
+__global__ void __launch_bounds__(kBlock) k_b_jacb0(Geo g, const double *X, const double *B0, double *B, double *det)
+{
+    b_jacb0_point(g, X, B0, B, det, (long long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // ----------------------------------------------------------- updateBbound
@@ -168,15 +172,28 @@ __device__ void bbound_point(const Geo &g, const double *X, const double *B0, do
     det[a] = 1 / detJac1;
 }
 
-__global__ void __launch_bounds__(kBlock) k_bbound(Geo g, const double *X, const double *B0, double *B, double *det, int face)
+__device__ __forceinline__ void bbound_face(const Geo &g, const double *X, const double *B0, double *B, double *det,
+                                            int face, long long t)
 {
     int nu = face == 0 ? g.ny : g.nx, nv = face == 2 ? g.ny : g.nz;
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     long long per = (long long)nu * nv;
     if (t >= 2 * per) return;
     int side = (int)(t / per);
     long long r = t % per;
     bbound_point(g, X, B0, B, det, face, side, (int)(r % nu), (int)(r / nu));
+}
+// Workgroups of one face after the other (f2, f1, f0 of them), then those of
+// the inner points.  A face point lasts as long as its chain of loads and
+// divisions (15 us a launch at 65 x 65 x 193, three launches); no point reads
+// what another writes, so all run at once.
+__global__ void __launch_bounds__(kBlock) k_b_all(Geo g, const double *X, const double *B0, double *B, double *det,
+                                                  int f2, int f1, int f0)
+{
+    int b = blockIdx.x;
+    if (b < f2) return bbound_face(g, X, B0, B, det, 2, (long long)b * kBlock + threadIdx.x);
+    if ((b -= f2) < f1) return bbound_face(g, X, B0, B, det, 1, (long long)b * kBlock + threadIdx.x);
+    if ((b -= f1) < f0) return bbound_face(g, X, B0, B, det, 0, (long long)b * kBlock + threadIdx.x);
+    b_jacb0_point(g, X, B0, B, det, (long long)(b - f0) * kBlock + threadIdx.x);
 }
 
 // ------------------------------------------------------ periodic copies
@@ -437,43 +454,58 @@ __global__ void __launch_bounds__(kBlock) k_gradp(Geo g, const double *X, const 
 }
 
 // --------------------------------------------------------------------- kk
-__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *tab, int n, double dt, const double *X,
-                                               const double *B, const double *J, const double *G, double *K,
-                                               double *Xtmp, const double *det, const double *U, double *KU,
-                                               double *Utmp)
+// Bound by memory: at most 2 x 5 earlier slopes, J, B, x and u in, both
+// slopes, x and u out.  All of a point's loads are issued before its stores
+// (N is a template argument), and x and u are replaced in place: the stage
+// copies and their way back cost three further passes (65 x 65 x 193 with
+// inertia: 61 us and 26 us of copies a stage before).
+template <int N>
+__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict__ tab, double dt, double *X,
+                                               const double *__restrict__ B, const double *__restrict__ J,
+                                               const double *__restrict__ G, double *K, const double *__restrict__ det,
+                                               double *U, double *KU)
 {
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long N = (long long)g.nx * g.ny * g.nz;
-    if (t >= N) return;
+    if (t >= (long long)g.nx * g.ny * g.nz) return;
     int i = (int)(t % g.nx), j = (int)((t / g.nx) % g.ny), k = (int)(t / ((long long)g.nx * g.ny));
     long long a = gidx(g, i + 1, j + 1, k + 1);
     const long long P3 = 3 * g.P;
-    double jv[3], bv[3], kv[3];
+    double w[N + 1], jv[3], bv[3], kv[3], x[3], kp[N + 1][3], gp[3] = {0, 0, 0};
+    for (int m = 0; m <= N; ++m) w[m] = tab->b[m + (N + 1) * 6] - tab->b[m + N * 6];
     ld3(J, g.P, a, jv);
     ld3(B, g.P, a, bv);
+    ld3(X, g.P, a, x);
+#pragma unroll
+    for (int m = 0; m < N; ++m) ld3(K + m * P3, g.P, a, kp[m]);
+    if (g.pressure) ld3(G, g.P, a, gp);
     cross3(jv, bv, kv);
     if (g.inertia) {
         // inertia branch (src/rungeKutta.cu:195-212, 216-246): position
         // slope dt u, velocity slope dt det (J x B) - dt nu u det - dt gradP;
         // no friction profile and no averaging here
         const double dj = det[a];
+        double u[3], up[N + 1][3];
+        ld3(U, g.P, a, u);
+#pragma unroll
+        for (int m = 0; m < N; ++m) ld3(KU + m * P3, g.P, a, up[m]);
         for (int l = 0; l < 3; ++l) {
-            const double u = U[l * g.P + a];
-            K[n * P3 + l * g.P + a] = dt * u;
+            kp[N][l] = dt * u[l];
             kv[l] *= dt * dj;
-            kv[l] -= dt * g.nu * u * dj;
-            if (g.pressure) kv[l] += -dt * G[l * g.P + a];
-            KU[n * P3 + l * g.P + a] = kv[l];
+            kv[l] -= dt * g.nu * u[l] * dj;
+            if (g.pressure) kv[l] += -dt * gp[l];
+            up[N][l] = kv[l];
         }
         for (int l = 0; l < 3; ++l) {
-            double x = X[l * g.P + a], v = U[l * g.P + a];
-            for (int m = 0; m < n + 1; ++m) {
-                const double w = tab->b[m + (n + 1) * 6] - tab->b[m + n * 6];
-                x += w * K[m * P3 + l * g.P + a];
-                v += w * KU[m * P3 + l * g.P + a];
+            double v = u[l];
+#pragma unroll
+            for (int m = 0; m <= N; ++m) {
+                x[l] += w[m] * kp[m][l];
+                v += w[m] * up[m][l];
             }
-            Xtmp[l * g.P + a] = x;
-            Utmp[l * g.P + a] = v;
+            K[N * P3 + l * g.P + a] = kp[N][l];
+            KU[N * P3 + l * g.P + a] = up[N][l];
+            X[l * g.P + a] = x[l];
+            U[l * g.P + a] = v;
         }
         return;
     }
@@ -502,14 +534,12 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *tab, int n,
     double eps = g.epsilonProf ? eps_axis(i, g.nx) * eps_axis(j, g.ny) * eps_axis(k, g.nz) : 1.0;
     for (int l = 0; l < 3; ++l) {
         kv[l] *= dt * eps;
-        if (g.pressure) kv[l] += -dt * G[l * g.P + a];
-        K[n * P3 + l * g.P + a] = kv[l];
-    }
-    for (int l = 0; l < 3; ++l) {
-        double x = X[l * g.P + a];
-        for (int m = 0; m < n + 1; ++m)
-            x += (tab->b[m + (n + 1) * 6] - tab->b[m + n * 6]) * K[m * P3 + l * g.P + a];
-        Xtmp[l * g.P + a] = x;
+        if (g.pressure) kv[l] += -dt * gp[l];
+        kp[N][l] = kv[l];
+#pragma unroll
+        for (int m = 0; m <= N; ++m) x[l] += w[m] * kp[m][l];
+        K[N * P3 + l * g.P + a] = kv[l];
+        X[l * g.P + a] = x[l];
     }
 }
 
@@ -558,7 +588,7 @@ __global__ void __launch_bounds__(kBlock) k_xnewstar(Geo g, const Tableau *tab, 
     }
 }
 
-__global__ void __launch_bounds__(1024) k_max_final(const double *partials, int n, double *out)
+__global__ void __launch_bounds__(1024) k_max_final(const double *partials, int n, const int *nanflag, double *out)
 {
     __shared__ double wmax[16];
     double m = 0;
@@ -570,6 +600,7 @@ __global__ void __launch_bounds__(1024) k_max_final(const double *partials, int 
         double r = 0;
         for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r = nb_max(r, wmax[w]);
         out[0] = r;
+        out[1] = *nanflag;
     }
 }
 
@@ -785,13 +816,22 @@ void launch_b_jacb0(hipStream_t s, const Geo &g, const double *X, const double *
 {
     hipLaunchKernelGGL(k_b_jacb0, dim3(blocks_for(ninner(g))), dim3(kBlock), 0, s, g, X, B0, B, det);
 }
+// Ghost faces 2, 1, 0 as setBbound (src/boundaries.cu:637-642), and the
+// inner points when asked for; each writes disjoint points and reads only X
+// and B0
+static void launch_b(hipStream_t s, const Geo &g, const double *X, const double *B0, double *B, double *det, bool inner)
+{
+    const int f2 = blocks_for(2LL * g.nx * g.ny), f1 = blocks_for(2LL * g.nx * g.nz), f0 = blocks_for(2LL * g.ny * g.nz);
+    const int in = inner ? blocks_for(ninner(g)) : 0;
+    hipLaunchKernelGGL(k_b_all, dim3(f2 + f1 + f0 + in), dim3(kBlock), 0, s, g, X, B0, B, det, f2, f1, f0);
+}
 void launch_bbound(hipStream_t s, const Geo &g, const double *X, const double *B0, double *B, double *det)
 {
-    // faces 2, 1, 0 as setBbound (src/boundaries.cu:637-642); each writes
-    // disjoint ghost points and reads only X and B0
-    const long long per[3] = {2LL * g.ny * g.nz, 2LL * g.nx * g.nz, 2LL * g.nx * g.ny};
-    for (int face = 2; face >= 0; --face)
-        hipLaunchKernelGGL(k_bbound, dim3(blocks_for(per[face])), dim3(kBlock), 0, s, g, X, B0, B, det, face);
+    launch_b(s, g, X, B0, B, det, false);
+}
+void launch_b_all(hipStream_t s, const Geo &g, const double *X, const double *B0, double *B, double *det)
+{
+    launch_b(s, g, X, B0, B, det, true);
 }
 void launch_set_peri(hipStream_t s, const Geo &g, double *F)
 {
@@ -821,12 +861,18 @@ void launch_gradp(hipStream_t s, const Geo &g, const double *X, const double *de
 {
     hipLaunchKernelGGL(k_gradp, dim3(blocks_for(ninner(g))), dim3(kBlock), 0, s, g, X, det, G);
 }
-void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X, const double *B,
-               const double *J, const double *G, double *K, double *Xtmp, const double *det, const double *U,
-               double *KU, double *Utmp)
+void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, double *X, const double *B,
+               const double *J, const double *G, double *K, const double *det, double *U, double *KU)
 {
-    hipLaunchKernelGGL(k_kk, dim3(blocks_for(ninner(g))), dim3(kBlock), 0, s, g, tab, n, dt, X, B, J, G, K, Xtmp, det,
-                       U, KU, Utmp);
+    const dim3 nb(blocks_for(ninner(g))), nt(kBlock);
+    switch (n) {
+    case 0: hipLaunchKernelGGL(k_kk<0>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    case 1: hipLaunchKernelGGL(k_kk<1>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    case 2: hipLaunchKernelGGL(k_kk<2>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    case 3: hipLaunchKernelGGL(k_kk<3>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    case 4: hipLaunchKernelGGL(k_kk<4>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    default: hipLaunchKernelGGL(k_kk<5>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    }
 }
 int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const double *X, const double *K, double *Xnew,
                     double *partials, int *nanflag, const double *U, const double *KU, double *Unew)
@@ -844,9 +890,9 @@ void launch_inner_aos_to_padded(hipStream_t s, const Geo &g, const double *src, 
 {
     hipLaunchKernelGGL(k_inner_aos_to_padded, dim3(blocks_for(ninner(g))), dim3(kBlock), 0, s, g, src, dst);
 }
-void launch_max_final(hipStream_t s, const double *partials, int n, double *out)
+void launch_max_final(hipStream_t s, const double *partials, int n, const int *nanflag, double *out)
 {
-    hipLaunchKernelGGL(k_max_final, dim3(1), dim3(1024), 0, s, partials, n, out);
+    hipLaunchKernelGGL(k_max_final, dim3(1), dim3(1024), 0, s, partials, n, nanflag, out);
 }
 void launch_aos_to_soa_f64(hipStream_t s, long long P, const double *src, double *dst)
 {

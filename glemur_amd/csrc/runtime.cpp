@@ -303,7 +303,7 @@ void ev_begin(gm_ctx *c, int kind) { c->tm.begin(c->stream, kind); }
 void ev_end(gm_ctx *c) { c->tm.end(c->stream); }
 
 // Enqueue one attempted step: stages 0..5 and the controller.
-void enqueue_step(gm_ctx *c, int diag, int check_done)
+void enqueue_step(gm_ctx *c, int diag, int check_done, gmd::Ctl *mirror = nullptr)
 {
     int f32k = c->prec == GM_PREC_F32K;
     for (int s = 0; s < 6; ++s) {
@@ -325,6 +325,7 @@ void enqueue_step(gm_ctx *c, int diag, int check_done)
     C.cell = c->p.dx * c->p.dy * c->p.dz;
     C.log = c->log;
     C.log_cap = c->log_cap;
+    C.mirror = mirror;
     ev_begin(c, 6);
     gmd::launch_controller(c->stream, C);
     ev_end(c);
@@ -413,10 +414,10 @@ extern "C" int gm_create(const gm_params *pp, int precision, gm_ctx **out)
         (void)hipMemset(c->J64, 0, P3 * sizeof(double));
         (void)hipMemset(c->G64, 0, P3 * sizeof(double));
         if (pp->inertia) {
-            if ((r = dalloc(&c->U64[0], P3)) || (r = dalloc(&c->U64[1], P3)) || (r = dalloc(&c->Utmp64, P3)) ||
+            if ((r = dalloc(&c->U64[0], P3)) || (r = dalloc(&c->U64[1], P3)) ||
                 (r = dalloc(&c->KU64, 6 * P3)))
                 return bail(r);
-            for (double *u : {c->U64[0], c->U64[1], c->Utmp64}) (void)hipMemset(u, 0, P3 * sizeof(double));
+            for (double *u : {c->U64[0], c->U64[1]}) (void)hipMemset(u, 0, P3 * sizeof(double));
             (void)hipMemset(c->KU64, 0, 6 * P3 * sizeof(double));
         }
     } else {
@@ -463,7 +464,7 @@ extern "C" int gm_create(const gm_params *pp, int precision, gm_ctx **out)
     c->ctlh->n_cycle = 1LL << 62;
     c->ctlh->max_attempt = 1LL << 62;
     if ((r = dalloc(&c->log, (size_t)c->log_cap))) return bail(r);
-    if ((r = dalloc(&c->red_out, 16)) || (r = dalloc(&c->row_part, (size_t)gmd::row_parts())) ||
+    if ((r = dalloc(&c->row_part, (size_t)gmd::row_parts())) ||
         (r = dalloc(&c->nanflag, 1)))
         return bail(r);
     if (hipHostMalloc((void **)&c->red_host, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)
@@ -485,13 +486,13 @@ extern "C" int gm_destroy(gm_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     for (int i = 0; i < 3; ++i) dfree(c->X64[i]);
-    dfree(c->B0_64); dfree(c->K64); dfree(c->B64); dfree(c->J64); dfree(c->G64); dfree(c->Xtmp64);
-    dfree(c->U64[0]); dfree(c->U64[1]); dfree(c->Utmp64); dfree(c->KU64);
+    dfree(c->B0_64); dfree(c->K64); dfree(c->B64); dfree(c->J64); dfree(c->G64);
+    dfree(c->U64[0]); dfree(c->U64[1]); dfree(c->KU64);
     for (int i = 0; i < 2; ++i) { dfree(c->Xh[i]); dfree(c->Xl[i]); }
     dfree(c->B0_32); dfree(c->K32); dfree(c->B32); dfree(c->J32); dfree(c->G32);
     dfree(c->det); dfree(c->epsx); dfree(c->epsy); dfree(c->epsz);
     dfree(c->ctl); dfree(c->part_delta); dfree(c->part_diag); dfree(c->tab_dev); dfree(c->log); dfree(c->ghost);
-    dfree(c->red_out); dfree(c->row_part); dfree(c->nanflag); dfree(c->xns_part);
+    dfree(c->row_part); dfree(c->nanflag); dfree(c->xns_part);
     if (c->ctlh) (void)hipHostFree(c->ctlh);
     if (c->red_host) (void)hipHostFree(c->red_host);
     c->tm.destroy();
@@ -756,21 +757,11 @@ extern "C" int gm_rk_kk(gm_ctx *c, int n, double dt)
     if (!c) return fail(GM_ERR_ARG, "null context");
     if (int r = need_f64(c, "gm_rk_kk")) return r;
     if (n < 0 || n > 5) return fail(GM_ERR_ARG, "stage index must be 0..5");
-    const size_t P3 = 3 * (size_t)c->P;
-    if (!c->Xtmp64) {
-        int r = dalloc(&c->Xtmp64, P3);
-        if (r) return r;
-    }
-    // xb_tmp starts as xb so its ghost layers match (src/main.cu:202)
-    HIPCHK(hipMemcpyAsync(c->Xtmp64, c->X64[c->cur], P3 * 8, hipMemcpyDeviceToDevice, c->stream));
+    // xb <- xb_tmp, uu <- uu_tmp (src/main.cu:288-305): written in place
     const bool in = c->p.inertia;
-    gmd::launch_kk(c->stream, c->geo, c->tab_dev, n, dt, c->X64[c->cur], c->B64, c->J64, c->G64, c->K64, c->Xtmp64,
-                   in ? c->det : nullptr, in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr,
-                   in ? c->Utmp64 : nullptr);
-    if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, c->Xtmp64);
-    HIPCHK(hipMemcpyAsync(c->X64[c->cur], c->Xtmp64, P3 * 8, hipMemcpyDeviceToDevice, c->stream));
-    // uu <- uu_tmp (src/main.cu:296-305)
-    if (in) HIPCHK(hipMemcpyAsync(c->U64[c->ucur], c->Utmp64, P3 * 8, hipMemcpyDeviceToDevice, c->stream));
+    gmd::launch_kk(c->stream, c->geo, c->tab_dev, n, dt, c->X64[c->cur], c->B64, c->J64, c->G64, c->K64,
+                   in ? c->det : nullptr, in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr);
+    if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, c->X64[c->cur]);
     return GM_OK;
 }
 extern "C" int gm_rk_xnewstar(gm_ctx *c, double *maxDelta)
@@ -791,8 +782,7 @@ extern "C" int gm_rk_xnewstar(gm_ctx *c, double *maxDelta)
                                  in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr,
                                  in ? c->U64[c->ucur ^ 1] : nullptr);
     if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, xnew);
-    gmd::launch_max_final(c->stream, parts, n, c->red_out);
-    HIPCHK(hipMemcpyAsync(c->red_host, c->red_out, 8, hipMemcpyDeviceToHost, c->stream));
+    gmd::launch_max_final(c->stream, parts, n, c->nanflag, c->red_host);
     HIPCHK(hipStreamSynchronize(c->stream));
     if (maxDelta) *maxDelta = c->red_host[0];
     return GM_OK;
@@ -817,7 +807,7 @@ extern "C" int gm_rk_xnewstar_noalloc(gm_ctx *c, double *maxDelta)
     if (hipGetDevice(&dev) != hipSuccess || dev != c->device) HIPCHK(hipSetDevice(c->device));
     double *S = gmd::noalloc_scratch(c->device);
     if (!S) return fail(GM_ERR_HIP, "gm_rk_xnewstar_noalloc: hipGetSymbolAddress of the scratch failed");
-    double *out = S, *parts = S + 8;
+    double *parts = S + 8;
     int *nan = reinterpret_cast<int *>(S + 1);
     gmd::launch_fill_f64(c->stream, S, 2, 0.0);   // grid maximum and NaN flag start at zero
     double *xnew = c->X64[(c->cur + 1) % 3];
@@ -828,8 +818,7 @@ extern "C" int gm_rk_xnewstar_noalloc(gm_ctx *c, double *maxDelta)
                                  in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr,
                                  in ? c->U64[c->ucur ^ 1] : nullptr);
     if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, xnew);
-    gmd::launch_max_final(c->stream, parts, n, out);
-    HIPCHK(hipMemcpyAsync(c->red_host, out, 8, hipMemcpyDeviceToHost, c->stream));
+    gmd::launch_max_final(c->stream, parts, n, nan, c->red_host);
     HIPCHK(hipStreamSynchronize(c->stream));
     if (maxDelta) *maxDelta = c->red_host[0];
     return GM_OK;
@@ -920,8 +909,8 @@ static bool per_kernel_path(gm_ctx *c)
 static int fields_per_kernel(gm_ctx *c)
 {
     int r;
-    if ((r = gm_b_jacb0(c)) || (r = gm_set_bbound(c)) || (r = gm_set_peri(c, GM_FIELD_B)) || (r = gm_current(c)))
-        return r;
+    gmd::launch_b_all(c->stream, c->geo, c->X64[c->cur], c->B0_64, c->B64, c->det);
+    if ((r = gm_set_peri(c, GM_FIELD_B)) || (r = gm_current(c))) return r;
     if (c->p.pressure && (r = gm_gradp(c))) return r;
     return GM_OK;
 }
@@ -969,7 +958,7 @@ static void fill_info(gm_ctx *c, gm_step_info *info)
 // reference).  The stage positions update x in place (src/main.cu:288), so
 // a rejected attempt continues from that x, as the reference does; the
 // criterion of the starting state is evaluated before the stages.
-// Expects c->ctlh synchronised; pushes it back.
+// Expects c->ctlh synchronised; enqueues its way back.
 static int step_per_kernel(gm_ctx *c)
 {
     gmd::Ctl &h = *c->ctlh;
@@ -994,8 +983,11 @@ static int step_per_kernel(gm_ctx *c)
     rec.energy = d[0];
     rec.jxb_b2 = d[2];
     rec.jmax = d[1];
-    auto log = [&](void) -> int {
-        HIPCHK(hipMemcpy(c->log + (h.n_attempt % c->log_cap), &rec, sizeof rec, hipMemcpyHostToDevice));
+    const long long at = h.n_attempt;
+    auto leave = [&](void) -> int {
+        c->cur = h.cur;
+        gmd::launch_put(c->stream, c->ctl, h, c->log + at % c->log_cap, rec);
+        HIPCHK(hipGetLastError());
         return GM_OK;
     };
     if (h.stop_ratio > 0 && crit <= h.stop_ratio) {
@@ -1004,8 +996,7 @@ static int step_per_kernel(gm_ctx *c)
         h.stop_reason = 3;
         h.accepted = 0;
         rec.accepted = -1;
-        if ((r = log())) return r;
-        return push_ctl(c);
+        return leave();
     }
     const double dt = h.dt;
     for (int n = 0; n < 6; ++n) {
@@ -1014,8 +1005,7 @@ static int step_per_kernel(gm_ctx *c)
     }
     double md = 0;
     if ((r = gm_rk_xnewstar(c, &md))) return r;
-    int nan = 0;
-    HIPCHK(hipMemcpy(&nan, c->nanflag, sizeof nan, hipMemcpyDeviceToHost));
+    const int nan = c->red_host[1] != 0;
     h.nan_seen |= nan;
     rec.nan_seen = nan;
     rec.maxDelta = md;
@@ -1032,43 +1022,34 @@ static int step_per_kernel(gm_ctx *c)
     if (md > 0) h.dt = dt * std::pow(0.9 * c->p.maxError / md, 0.2);
     rec.accepted = acc;
     rec.t = h.t;
-    if ((r = log())) return r;
     h.n_attempt += 1;
     h.event = acc && (gmd::interval_crossed(h.t, h.dt, h.ev_dump) || gmd::interval_crossed(h.t, h.dt, h.ev_save));
     if (h.n_accept >= h.n_cycle) { h.done = 1; h.stop_reason = 1; }
     else if (!(h.dt > c->p.dtMin)) { h.done = 1; h.stop_reason = 2; }
     else if (h.n_attempt >= h.max_attempt) { h.done = 1; h.stop_reason = 4; }
     else if (h.event) { h.done = 1; h.stop_reason = 5; }
-    c->cur = h.cur;
-    return push_ctl(c);
+    return leave();
 }
 
 
 extern "C" int gm_step(gm_ctx *c, gm_step_info *info)
 {
     if (!c) return fail(GM_ERR_ARG, "null context");
-    if (!per_kernel_path(c))
+    const bool pk = per_kernel_path(c);
+    if (!pk)
         if (int r = check_fused(c)) return r;
-    int r = sync_ctl(c);
-    if (r) return r;
-    gmd::Ctl &h = *c->ctlh;
-    h.done = 0;
-    h.converged = 0;
-    h.stop_reason = 0;
-    h.nan_seen = 0;
-    h.stop_ratio = 0;
-    h.n_cycle = 1LL << 62;
-    h.max_attempt = 1LL << 62;
-    h.event = 0;
-    h.ev_dump = h.ev_save = 0;
-    if ((r = push_ctl(c))) return r;
-    if (per_kernel_path(c)) {
-        if ((r = step_per_kernel(c))) return r;
+    int r;
+    gmd::launch_arm(c->stream, {c->ctl, 0, 0, 0, 0, 0, 0});
+    if (pk) {
+        if ((r = sync_ctl(c)) || (r = step_per_kernel(c))) return r;
     } else {
-        enqueue_step(c, 1, 1);
+        enqueue_step(c, 1, 1, c->ctlh);
     }
     HIPCHK(hipGetLastError());
-    if ((r = sync_ctl(c))) return r;
+    HIPCHK(hipStreamSynchronize(c->stream));
+    c->tm.collect();
+    const gmd::Ctl &h = *c->ctlh;
+    c->cur = h.cur;
     if (info) fill_info(c, info);
     if (h.nan_seen) return fail(GM_ERR_NAN, "NaN in the error estimate (the reference's max would skip it)");
     return GM_OK;
@@ -1079,22 +1060,11 @@ extern "C" int gm_run(gm_ctx *c, const gm_run_opts *o, gm_run_stats *st)
     if (!c || !o) return fail(GM_ERR_ARG, "gm_run: null pointer");
     if (!per_kernel_path(c))
         if (int r = check_fused(c)) return r;
-    int r = sync_ctl(c);
-    if (r) return r;
+    int r;
     gmd::Ctl &h = *c->ctlh;
-    h.done = 0;
-    h.converged = 0;
-    h.stop_reason = 0;
-    h.nan_seen = 0;
-    h.diag_valid = 0;
-    h.stop_ratio = o->stop_ratio;
-    h.event = 0;
-    h.ev_dump = o->dt_dump;
-    h.ev_save = o->dt_save;
-    long long ncyc = o->n_cycle > 0 ? o->n_cycle : c->p.nCycle;
-    h.n_cycle = h.n_accept + ncyc;
-    h.max_attempt = h.n_attempt + (o->max_attempts > 0 ? o->max_attempts : (1LL << 40));
-    if ((r = push_ctl(c))) return r;
+    gmd::launch_arm(c->stream, {c->ctl, o->stop_ratio, o->dt_dump, o->dt_save, o->n_cycle > 0 ? o->n_cycle : c->p.nCycle,
+                                o->max_attempts > 0 ? o->max_attempts : 1LL << 40, 1});
+    if (per_kernel_path(c) && (r = sync_ctl(c))) return r;
     int batch = std::max(1, o->batch);
     bool graph = o->use_graph && !c->tm.on && !per_kernel_path(c);
     auto t0 = std::chrono::steady_clock::now();
