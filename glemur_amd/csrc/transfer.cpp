@@ -26,8 +26,11 @@ constexpr int kSlots = 8, kThreads = 6;
 constexpr size_t kSlotBytes = 4 << 20, kMinChunk = 256 << 10;
 // Below these the threads cost more than they save (plain -> staged): up
 // 9 MB 0.28 -> 0.44 ms, 21 MB 0.65 -> 0.72 ms, 158 MB 6.4 -> 3.9 ms; down
-// 3 MB 0.46 -> 0.40 ms, 9 MB 0.97 -> 0.70 ms, 21 MB 2.3 -> 0.85 ms.
-constexpr size_t kMinUp = 32 << 20, kMinDown = 6 << 20;
+// 9 MB 0.97 -> 0.70 ms, 21 MB 2.3 -> 0.85 ms.  Beside a program whose own
+// threads spin (a torch program's after each host operation) a short copy
+// waits for its threads to be scheduled: 11 MB down 0.7 ms plain, 2.5 ms
+// staged, hence no less than 16 MB.
+constexpr size_t kMinUp = 32 << 20, kMinDown = 16 << 20;
 
 struct Staging {
     std::mutex m;             // held by the copy that uses the slots

@@ -1,5 +1,5 @@
 """Uploads and downloads of arrays that are staged through pinned slots
-(downloads from 6 MB, uploads from 32 MB) and of arrays just below: the
+(downloads from 16 MB, uploads from 32 MB) and of arrays just below: the
 positions and B0 come back as they went up, bit for bit, also from several
 threads at once, of which one at a time has the slots, and from and into
 pinned memory, which is copied as it is."""
@@ -31,9 +31,9 @@ def round_trip(g, shape, seed, out):
             B0, xb = xb, B0
 
 
-# 6 MB and 32 MB lie at 262144 and 1398101 padded points; 33 is one chunk of
-# 4 MB past eight, the largest wraps the slots twice
-@pytest.mark.parametrize("shape", [(60, 62, 64), (62, 62, 62), (62, 62, 64), (110, 111, 107), (110, 112, 108),
+# 16 MB and 32 MB lie at 699050 and 1398101 padded points; 33 MB is one chunk
+# of 4 MB past eight, the largest wraps the slots twice
+@pytest.mark.parametrize("shape", [(60, 62, 64), (86, 88, 86), (87, 87, 87), (110, 111, 107), (110, 112, 108),
                                    (118, 111, 109), (150, 140, 139)])
 def test_round_trip(g, shape):
     out = []
