@@ -25,6 +25,7 @@
 
 #include "gm_ctx.hpp"
 #include "gm_internal.hpp"
+#include "transfer.hpp"
 #include "unet_kernels.hpp"
 
 using gm::fail;
@@ -48,8 +49,9 @@ int pad32(int k) { return (k + 31) / 32 * 32; }
 
 struct ULayer {
     int cin = 0, cout = 0, coutp = 0, kpad = 0, kpadT = 0;
-    float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;   // [coutp][kpad]
-    float *b = nullptr, *bm = nullptr, *bv = nullptr, *bg = nullptr; // [coutp]
+    long long at = 0;        // first float in the network's parameter arrays
+    float *w = nullptr, *g = nullptr;   // [coutp][kpad]
+    float *b = nullptr, *bg = nullptr;  // [coutp]
     bf16_t *wf = nullptr;    // packed bf16 weights (coutp * kpad)
     bf16_t *wb = nullptr;    // packed flipped transpose, the input gradient's (cin * kpadT)
 };
@@ -63,6 +65,11 @@ struct gm_unet {
     double scale = 1.0;
     int step = 0;
     hipStream_t stream = nullptr;
+    // weights and biases of all layers one after the other, their gradients
+    // and Adam's moments: ULayer points into them
+    float *pw = nullptr, *pg = nullptr, *pm = nullptr, *pv = nullptr;
+    long long np = 0;            // floats in each
+    double *pbuf = nullptr;      // parameters or gradients as the caller has them
     bf16_t *x0 = nullptr, *a1 = nullptr, *cat1 = nullptr, *p2 = nullptr, *a3 = nullptr, *cat2 = nullptr;
     bf16_t *p3 = nullptr, *a5 = nullptr, *a6 = nullptr, *a7 = nullptr, *a8 = nullptr, *a9 = nullptr, *a10 = nullptr;
     float *y = nullptr;          // [P1][16]
@@ -190,13 +197,7 @@ void backward(gm_unet *u, const bf16_t *x0, const float *target)
     wgrad(u, 0, x0, 8, u->g1);
 }
 
-void zero_grads(gm_unet *u)
-{
-    for (auto &L : u->L) {
-        gmu::launch_zero(u->stream, L.g, (long long)L.coutp * L.kpad * 4);
-        gmu::launch_zero(u->stream, L.bg, (long long)L.coutp * 4);
-    }
-}
+void zero_grads(gm_unet *u) { gmu::launch_zero(u->stream, u->pg, u->np * 4); }
 
 void refresh_bf16(gm_unet *u)
 {
@@ -209,21 +210,50 @@ void refresh_bf16(gm_unet *u)
 void adam(gm_unet *u, float lr, float gscale)
 {
     ++u->step;
-    for (auto &L : u->L) {
-        gmu::launch_adam(u->stream, L.w, L.g, L.m, L.v, (long long)L.coutp * L.kpad, gscale, lr, 0.9f, 0.999f, 1e-8f,
-                         u->step);
-        gmu::launch_adam(u->stream, L.b, L.bg, L.bm, L.bv, L.coutp, gscale, lr, 0.9f, 0.999f, 1e-8f, u->step);
-    }
+    gmu::launch_adam(u->stream, u->pw, u->pg, u->pm, u->pv, u->np, gscale, lr, 0.9f, 0.999f, 1e-8f, u->step);
     refresh_bf16(u);
 }
 
-int upload_feat(gm_unet *u, const double *feat)
+// Features (and targets, if any) as the caller has them, converted on the
+// device: one host thread converts about 1 GB/s.  The weight gradients'
+// partials take them meanwhile (at least 162 bytes a point).
+int upload_sample(gm_unet *u, const double *feat, const double *target)
 {
-    const long long n = u->P[1] * 8;
-    std::vector<float> f(feat, feat + n);
-    HIPCHK(hipMemcpyAsync(u->y, f.data(), n * 4, hipMemcpyHostToDevice, u->stream));   // y as fp32 staging
-    gmu::launch_f32_to_bf16(u->stream, u->y, n, u->x0);
-    HIPCHK(hipStreamSynchronize(u->stream));
+    const long long P1 = u->P[1];
+    double *f = reinterpret_cast<double *>(u->part), *t = f + 8 * P1;
+    HIPCHK(gm::copy_to_device(u->stream, f, feat, (size_t)P1 * 64));
+    gmu::launch_f64_to_bf16(u->stream, f, P1 * 8, u->x0);
+    if (target) {
+        HIPCHK(gm::copy_to_device(u->stream, t, target, (size_t)P1 * 24));
+        gmu::launch_f64_to_f32(u->stream, t, P1 * 3, u->tgt);
+    }
+    return GM_OK;
+}
+
+gmu::ParamMap param_map(const gm_unet *u)
+{
+    gmu::ParamMap m{};
+    long long n = 0;
+    for (int l = 0; l < NL; ++l) {
+        const ULayer &L = u->L[l];
+        m.first[l] = n;
+        m.at[l] = L.at;
+        m.k[l] = 27 * L.cin;
+        m.kpad[l] = L.kpad;
+        m.nw[l] = L.cout * 27 * L.cin;
+        m.bias[l] = L.at + (long long)L.coutp * L.kpad;
+        n += m.nw[l] + L.cout;
+    }
+    m.first[NL] = n;
+    return m;
+}
+
+// Parameters or gradients to the caller's array, without the padding
+int download_params(gm_unet *u, const float *src, double *out)
+{
+    const gmu::ParamMap m = param_map(u);
+    gmu::launch_params_out(u->stream, m, src, u->pbuf);
+    HIPCHK(gm::copy_to_host(u->stream, out, u->pbuf, (size_t)m.first[NL] * 8));
     return GM_OK;
 }
 
@@ -242,6 +272,7 @@ extern "C" int gm_unet_destroy(gm_unet *u)
     if (u->stream) (void)hipStreamSynchronize(u->stream);
     for (void *p : u->allocs) (void)hipFree(p);
     if (u->stream) (void)hipStreamDestroy(u->stream);
+    gm::staging_release();
     delete u;
     return GM_OK;
 }
@@ -256,6 +287,7 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
             return fail(GM_ERR_ARG, "gm_unet_create: every grid size must be 4m+1 >= 5 (two exact coarsenings)");
     if (capacity < 0) return fail(GM_ERR_ARG, "gm_unet_create: negative capacity");
     gm_unet *u = new gm_unet();
+    gm::staging_retain();
     for (int d = 0; d < 3; ++d) {
         u->n[1][d] = dims[d];
         u->n[2][d] = (dims[d] + 1) / 2;
@@ -274,14 +306,23 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
         L.kpad = pad32(27 * L.cin);
         L.kpadT = pad32(27 * L.coutp);
         const size_t nw = (size_t)L.coutp * L.kpad;
+        L.at = u->np;
+        u->np += nw + L.coutp;
         int r;
-        if ((r = ualloc(u, &L.w, nw)) || (r = ualloc(u, &L.m, nw)) || (r = ualloc(u, &L.v, nw)) ||
-            (r = ualloc(u, &L.g, nw)) || (r = ualloc(u, &L.b, L.coutp)) || (r = ualloc(u, &L.bm, L.coutp)) ||
-            (r = ualloc(u, &L.bv, L.coutp)) || (r = ualloc(u, &L.bg, L.coutp)) || (r = ualloc(u, &L.wf, nw)))
-            return bail(r);
+        if ((r = ualloc(u, &L.wf, nw))) return bail(r);
         if (l > 0 && (r = ualloc(u, &L.wb, (size_t)L.cin * L.kpadT))) return bail(r);
         const int *n = u->n[LEVEL[l]];
         part_cap = std::max(part_cap, gmu::wgrad_part_floats(n[0], n[1], n[2], L.cin, L.coutp));
+    }
+    for (float **p : {&u->pw, &u->pg, &u->pm, &u->pv})
+        if (int r = ualloc(u, p, u->np)) return bail(r);
+    if (int r = ualloc(u, &u->pbuf, gm_unet_num_params())) return bail(r);
+    for (auto &L : u->L) {
+        const long long nw = (long long)L.coutp * L.kpad;
+        L.w = u->pw + L.at;
+        L.b = L.w + nw;
+        L.g = u->pg + L.at;
+        L.bg = L.g + nw;
     }
     const long long P1 = u->P[1], P2 = u->P[2], P3 = u->P[3];
     int r;
@@ -313,22 +354,11 @@ extern "C" int gm_unet_set_params(gm_unet *u, const double *params, int64_t n)
     if (!u || !params) return fail(GM_ERR_ARG, "gm_unet_set_params: null pointer");
     if (n != gm_unet_num_params()) return fail(GM_ERR_ARG, "gm_unet_set_params: wrong parameter count");
     if (!(params[n - 1] > 0)) return fail(GM_ERR_ARG, "gm_unet_set_params: the output scale must be > 0");
-    const double *q = params;
-    for (auto &L : u->L) {
-        std::vector<float> w((size_t)L.coutp * L.kpad, 0.f), b(L.coutp, 0.f);
-        for (int co = 0; co < L.cout; ++co)
-            for (int k = 0; k < 27 * L.cin; ++k) w[(size_t)co * L.kpad + k] = (float)q[(size_t)co * 27 * L.cin + k];
-        q += (size_t)L.cout * 27 * L.cin;
-        for (int co = 0; co < L.cout; ++co) b[co] = (float)q[co];
-        q += L.cout;
-        HIPCHK(hipMemcpy(L.w, w.data(), w.size() * 4, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(L.b, b.data(), b.size() * 4, hipMemcpyHostToDevice));
-        HIPCHK(hipMemset(L.m, 0, w.size() * 4));
-        HIPCHK(hipMemset(L.v, 0, w.size() * 4));
-        HIPCHK(hipMemset(L.bm, 0, b.size() * 4));
-        HIPCHK(hipMemset(L.bv, 0, b.size() * 4));
-    }
-    u->scale = *q;
+    HIPCHK(gm::copy_to_device(u->stream, u->pbuf, params, (size_t)(n - 1) * 8));
+    gmu::launch_params_in(u->stream, param_map(u), u->pbuf, u->pw);
+    gmu::launch_zero(u->stream, u->pm, u->np * 4);
+    gmu::launch_zero(u->stream, u->pv, u->np * 4);
+    u->scale = params[n - 1];
     u->step = 0;
     refresh_bf16(u);
     HIPCHK(hipStreamSynchronize(u->stream));
@@ -339,19 +369,8 @@ extern "C" int gm_unet_get_params(gm_unet *u, double *params, int64_t n)
 {
     if (!u || !params) return fail(GM_ERR_ARG, "gm_unet_get_params: null pointer");
     if (n != gm_unet_num_params()) return fail(GM_ERR_ARG, "gm_unet_get_params: wrong parameter count");
-    HIPCHK(hipStreamSynchronize(u->stream));
-    double *q = params;
-    for (auto &L : u->L) {
-        std::vector<float> w((size_t)L.coutp * L.kpad), b(L.coutp);
-        HIPCHK(hipMemcpy(w.data(), L.w, w.size() * 4, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(b.data(), L.b, b.size() * 4, hipMemcpyDeviceToHost));
-        for (int co = 0; co < L.cout; ++co)
-            for (int k = 0; k < 27 * L.cin; ++k) q[(size_t)co * 27 * L.cin + k] = w[(size_t)co * L.kpad + k];
-        q += (size_t)L.cout * 27 * L.cin;
-        for (int co = 0; co < L.cout; ++co) q[co] = b[co];
-        q += L.cout;
-    }
-    *q = u->scale;
+    if (int r = download_params(u, u->pw, params)) return r;
+    params[n - 1] = u->scale;
     return GM_OK;
 }
 
@@ -384,14 +403,11 @@ extern "C" int gm_unet_forward(gm_unet *u, const double *feat, double *y)
 {
     if (!u || !feat || !y) return fail(GM_ERR_ARG, "gm_unet_forward: null pointer");
     if (!(u->scale > 0)) return fail(GM_ERR_ARG, "gm_unet_forward: no output scale (set parameters or train first)");
-    if (int r = upload_feat(u, feat)) return r;
+    if (int r = upload_sample(u, feat, nullptr)) return r;
     forward(u, u->x0);
-    const long long P1 = u->P[1];
-    std::vector<float> h((size_t)P1 * 16);
-    HIPCHK(hipMemcpyAsync(h.data(), u->y, h.size() * 4, hipMemcpyDeviceToHost, u->stream));
-    HIPCHK(hipStreamSynchronize(u->stream));
-    for (long long p = 0; p < P1; ++p)
-        for (int c = 0; c < 3; ++c) y[p * 3 + c] = u->scale * h[p * 16 + c];
+    double *out = reinterpret_cast<double *>(u->part);
+    gmu::launch_scale_out(u->stream, u->y, u->P[1], u->scale, out);
+    HIPCHK(gm::copy_to_host(u->stream, y, out, (size_t)u->P[1] * 24));
     return GM_OK;
 }
 
@@ -399,31 +415,17 @@ extern "C" int gm_unet_loss_grad(gm_unet *u, const double *feat, const double *t
 {
     if (!u || !feat || !target) return fail(GM_ERR_ARG, "gm_unet_loss_grad: null pointer");
     if (!(u->scale > 0)) return fail(GM_ERR_ARG, "gm_unet_loss_grad: no output scale");
-    if (int r = upload_feat(u, feat)) return r;
-    const long long P1 = u->P[1];
-    std::vector<float> t(target, target + P1 * 3);
-    HIPCHK(hipMemcpyAsync(u->tgt, t.data(), t.size() * 4, hipMemcpyHostToDevice, u->stream));
+    if (int r = upload_sample(u, feat, target)) return r;
     zero_grads(u);
     gmu::launch_zero(u->stream, u->dacc, 8);
     forward(u, u->x0);
     backward(u, u->x0, u->tgt);
+    if (grad)
+        if (int r = download_params(u, u->pg, grad)) return r;
     double l = 0;
     HIPCHK(hipMemcpyAsync(&l, u->dacc, 8, hipMemcpyDeviceToHost, u->stream));
     HIPCHK(hipStreamSynchronize(u->stream));
     if (loss) *loss = l;
-    if (grad) {
-        double *q = grad;
-        for (auto &L : u->L) {
-            std::vector<float> w((size_t)L.coutp * L.kpad), b(L.coutp);
-            HIPCHK(hipMemcpy(w.data(), L.g, w.size() * 4, hipMemcpyDeviceToHost));
-            HIPCHK(hipMemcpy(b.data(), L.bg, b.size() * 4, hipMemcpyDeviceToHost));
-            for (int co = 0; co < L.cout; ++co)
-                for (int k = 0; k < 27 * L.cin; ++k) q[(size_t)co * 27 * L.cin + k] = w[(size_t)co * L.kpad + k];
-            q += (size_t)L.cout * 27 * L.cin;
-            for (int co = 0; co < L.cout; ++co) q[co] = b[co];
-            q += L.cout;
-        }
-    }
     return GM_OK;
 }
 

@@ -420,8 +420,9 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k
 // Bias gradient partials of 4096 points, ph = 256 / c threads a channel:
 // thread k sums the points k, k + ph, ... in turn, and the ph sums are added
 // in turn.  A workgroup takes 32 channels and stages 512 points of them in
-// LDS at a time, 16 bytes a lane: one chain of 2-byte loads a thread had
-// taken 224 us a layer on average at 65 x 65 x 193
+// LDS at a time, 16 bytes a lane, the next 512 on their way meanwhile: one
+// chain of 2-byte loads a thread had taken 224 us a layer on average at 65 x
+// 65 x 193, without the loads ahead 23 us
 constexpr int BG_CHUNK = 4096, BG_PTS = 512, BG_CH = 32;
 
 __global__ __launch_bounds__(256) void k_bias_part(const bf16_t *g, int P, int c, float *part)
@@ -431,15 +432,27 @@ __global__ __launch_bounds__(256) void k_bias_part(const bf16_t *g, int P, int c
     const int w = c < BG_CH ? c : BG_CH, ph = 256 / c, ch = threadIdx.x % w, k = threadIdx.x / w, c0 = blockIdx.y * BG_CH;
     const int p0 = blockIdx.x * BG_CHUNK, p1 = min(p0 + BG_CHUNK, P);
     float s = 0.f;
+    constexpr int NL = BG_PTS * BG_CH / 8 / 256;
+    u32x4 v[NL];
+    auto load = [&](int pb) {   // 512 points on their way while those before are summed
+        const int n = min(BG_PTS, p1 - pb) * (w / 8);
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int q = min((int)threadIdx.x + 256 * u, n - 1), i = q / (w / 8), e = q % (w / 8);
+            v[u] = ld16(g + (long long)(pb + i) * c + c0 + 8 * e);
+        }
+    };
+    load(p0);
     for (int pb = p0; pb < p1; pb += BG_PTS) {
         const int n = min(BG_PTS, p1 - pb);
         __syncthreads();
-#pragma unroll 8
-        for (int q = threadIdx.x; q < n * (w / 8); q += 256) {
-            const int i = q / (w / 8), e = q % (w / 8);
-            st16(st + 8 * q, ld16(g + (long long)(pb + i) * c + c0 + 8 * e));
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int q = threadIdx.x + 256 * u;
+            if (q < n * (w / 8)) st16(st + 8 * q, v[u]);
         }
         __syncthreads();
+        if (pb + BG_PTS < p1) load(pb + BG_PTS);
         if (k < ph) {
             int i = k;
             for (; i + 15 * ph < n; i += 16 * ph) {
@@ -656,12 +669,22 @@ __global__ __launch_bounds__(256) void k_loss(const float *y, const float *targe
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-__global__ void k_loss_final(const double *part, int n, long long P, double *acc)
+// The partials in turn; 256 threads bring them into LDS (one thread's own
+// loads, in turn too, took 50 us at 65 x 65 x 193)
+__global__ __launch_bounds__(256) void k_loss_final(const double *part, int n, long long P, double *acc)
 {
-    if (threadIdx.x != 0) return;
+    __shared__ double st[256];
     double s = 0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    acc[0] += s / (3.0 * (double)P);
+    for (int i0 = 0; i0 < n; i0 += 256) {
+        __syncthreads();
+        if (i0 + (int)threadIdx.x < n) st[threadIdx.x] = part[i0 + threadIdx.x];
+        __syncthreads();
+        const int m = min(256, n - i0);
+        if (threadIdx.x == 0)
+#pragma unroll 16
+            for (int i = 0; i < m; ++i) s += st[i];
+    }
+    if (threadIdx.x == 0) acc[0] += s / (3.0 * (double)P);
 }
 
 __global__ void k_adam(float *w, const float *g, float *m, float *v, long long n, float gscale, float lr, float b1,
@@ -677,10 +700,41 @@ __global__ void k_adam(float *w, const float *g, float *m, float *v, long long n
     w[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
-__global__ void k_f2b(const float *in, long long n, bf16_t *out)
+__global__ void k_d2b(const double *in, long long n, bf16_t *out)
+{
+    const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 8;   // n: a multiple of 8
+    if (i >= n) return;
+    float v[8];
+    for (int e = 0; e < 8; ++e) v[e] = (float)in[i + e];
+    st16(out + i, pack8(v));
+}
+__global__ void k_d2f(const double *in, long long n, float *out)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (bf16_t)f2bf2(in[i], 0.f);
+    if (i < n) out[i] = (float)in[i];
+}
+__global__ void k_scale_out(const float *y, long long n, double scale, double *out)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // 3 p + c
+    if (i < n) out[i] = scale * y[i / 3 * 16 + i % 3];
+}
+// Where parameter i of the caller's array lies in the device arrays
+__device__ inline long long param_at(const ParamMap &m, long long i)
+{
+    int l = 0;
+    while (i >= m.first[l + 1]) ++l;
+    const int j = (int)(i - m.first[l]), row = j / m.k[l];
+    return j < m.nw[l] ? m.at[l] + (long long)row * m.kpad[l] + (j - row * m.k[l]) : m.bias[l] + (j - m.nw[l]);
+}
+__global__ void k_params_out(ParamMap m, const float *src, double *out)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < m.first[kLayers]) out[i] = src[param_at(m, i)];
+}
+__global__ void k_params_in(ParamMap m, const double *in, float *dst)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < m.first[kLayers]) dst[param_at(m, i)] = (float)in[i];
 }
 
 // ------------------------------------------------- context <-> network
@@ -793,14 +847,17 @@ __global__ __launch_bounds__(256) void k_min_det(const double *det, int nx, int 
     }
 }
 
-__global__ void k_min_det_final(const double *part, int n, double *out)
+__global__ __launch_bounds__(64) void k_min_det_final(const double *part, int n, double *out)
 {
-    if (threadIdx.x != 0) return;
-    double mn = 1e300, nan = 0;
-    for (int i = 0; i < n; ++i) {
+    double mn = 1e300;
+    int nan = 0;
+    for (int i = threadIdx.x; i < n; i += 64) {
         mn = fmin(mn, part[2 * i]);
         if (part[2 * i + 1] != 0) nan = 1;
     }
+    for (int o = 32; o > 0; o >>= 1) mn = fmin(mn, __shfl_xor(mn, o, 64));
+    nan = __any(nan);
+    if (threadIdx.x != 0) return;
     out[0] = mn;
     out[1] = nan;
 }
@@ -954,7 +1011,7 @@ void launch_loss(hipStream_t s, const float *y, const float *target, float inv_s
 {
     const int n = loss_blocks(P);
     k_loss<<<n, 256, 0, s>>>(y, target, inv_scale, P, g, part);
-    k_loss_final<<<1, 64, 0, s>>>(part, n, P, loss_acc);
+    k_loss_final<<<1, 256, 0, s>>>(part, n, P, loss_acc);
 }
 
 void launch_adam(hipStream_t s, float *w, const float *g, float *m, float *v, long long n, float gscale, float lr,
@@ -971,9 +1028,25 @@ void launch_pack(hipStream_t s, const float *w, int coutp, int cin, int kpad, bf
                                                                                               wf, wb, kpadT);
 }
 
-void launch_f32_to_bf16(hipStream_t s, const float *in, long long n, bf16_t *out)
+void launch_f64_to_bf16(hipStream_t s, const double *in, long long n, bf16_t *out)
 {
-    k_f2b<<<nblk(n), 256, 0, s>>>(in, n, out);
+    k_d2b<<<nblk(n / 8), 256, 0, s>>>(in, n, out);
+}
+void launch_f64_to_f32(hipStream_t s, const double *in, long long n, float *out)
+{
+    k_d2f<<<nblk(n), 256, 0, s>>>(in, n, out);
+}
+void launch_scale_out(hipStream_t s, const float *y, long long P, double scale, double *out)
+{
+    k_scale_out<<<nblk(3 * P), 256, 0, s>>>(y, 3 * P, scale, out);
+}
+void launch_params_out(hipStream_t s, const ParamMap &m, const float *src, double *out)
+{
+    k_params_out<<<nblk(m.first[kLayers]), 256, 0, s>>>(m, src, out);
+}
+void launch_params_in(hipStream_t s, const ParamMap &m, const double *in, float *dst)
+{
+    k_params_in<<<nblk(m.first[kLayers]), 256, 0, s>>>(m, in, dst);
 }
 
 void launch_zero(hipStream_t s, void *p, long long bytes) { (void)hipMemsetAsync(p, 0, (size_t)bytes, s); }

@@ -86,7 +86,22 @@ void launch_adam(hipStream_t s, float *w, const float *g, float *m, float *v, lo
 // input gradient, the flipped transpose W[co][(26 - t') cin + ci] at row ci,
 // k = t' coutp + co.
 void launch_pack(hipStream_t s, const float *w, int coutp, int cin, int kpad, bf16_t *wf, bf16_t *wb, int kpadT);
-void launch_f32_to_bf16(hipStream_t s, const float *in, long long n, bf16_t *out);
+// Doubles rounded to FP32, and from there to bf16
+void launch_f64_to_bf16(hipStream_t s, const double *in, long long n, bf16_t *out);
+void launch_f64_to_f32(hipStream_t s, const double *in, long long n, float *out);
+// out[p][c] = scale * y[p][c], c < 3 of 16
+void launch_scale_out(hipStream_t s, const float *y, long long P, double scale, double *out);
+
+// The caller's parameters are, layer by layer, nw weights in rows of k and
+// the biases, from first[l] on; in the device arrays the weights' rows start
+// at at[l] with pitch kpad[l], the biases at bias[l].
+constexpr int kLayers = 11;
+struct ParamMap {
+    long long first[kLayers + 1], at[kLayers], bias[kLayers];
+    int k[kLayers], kpad[kLayers], nw[kLayers];
+};
+void launch_params_out(hipStream_t s, const ParamMap &m, const float *src, double *out);
+void launch_params_in(hipStream_t s, const ParamMap &m, const double *in, float *dst);
 void launch_zero(hipStream_t s, void *p, long long bytes);
 
 // Features of a relaxation context's B0 (SoA, padded (nx+2)(ny+2)(nz+2),
