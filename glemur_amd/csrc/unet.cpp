@@ -309,8 +309,9 @@ extern "C" int gm_unet_create(int nx, int ny, int nz, int capacity, gm_unet **ou
         L.at = u->np;
         u->np += nw + L.coutp;
         int r;
-        if ((r = ualloc(u, &L.wf, nw))) return bail(r);
-        if (l > 0 && (r = ualloc(u, &L.wb, (size_t)L.cin * L.kpadT))) return bail(r);
+        // nine steps of a convolution more than the weights: it loads ahead
+        if ((r = ualloc(u, &L.wf, nw + 9 * 32 * (size_t)L.coutp))) return bail(r);
+        if (l > 0 && (r = ualloc(u, &L.wb, (size_t)L.cin * (L.kpadT + 9 * 32)))) return bail(r);
         const int *n = u->n[LEVEL[l]];
         part_cap = std::max(part_cap, gmu::wgrad_part_floats(n[0], n[1], n[2], L.cin, L.coutp));
     }

@@ -76,18 +76,22 @@ __device__ inline int xcd_run(int b, int n)
 // banks.  A thread's staged words differ only in z (and y in a few steps), so
 // the grid tests cost next to nothing.  The weights come in the order the lanes take them
 // (k_pack), 1 KB a tile and step, straight from memory (L1, L2) into a ring
-// of registers kRing steps ahead.  The weights are the first operand and
-// the points the second, so a lane ends up with four consecutive channels
-// of one point and stores them in 8 bytes.
+// of registers kRing steps ahead, the points from LDS one step ahead; the
+// scheduling barriers hold the loads where they are written.  The weights are
+// the first operand and the points the second, so a lane ends up with four
+// consecutive channels of one point and stores them in 8 bytes.
 // K runs as (tap, channel) in steps of 32 whatever the layer, one
 // accumulator per output: every output is the same sum in the same order
 // for any box.
 // What bounds it: LDS and L1 reads against the matrix pipe, about even at 32
 // output channels (MTW LDS and NTW L1 reads of 1 KB for MTW NTW matrix
 // instructions a step); at the coarsest level the few hundred workgroups.
-// 65 x 65 x 193, all layers and input gradients of a sample: 5.0 -> 1.6 ms
-// against operands loaded straight from memory per tap, with a grid test per
-// tap and lane
+// 65 x 65 x 193, all layers and input gradients of a sample: 5.0 ms with
+// operands loaded straight from memory per tap and a grid test per tap and
+// lane; 1.6 ms from LDS boxes, but with the weight loads moved down to their
+// use by the compiler, a wait for memory every step; 1.2 ms with them held
+// (96 -> 32 channels 289 -> 223 us, 192 -> 64 189 -> 108, 128 -> 128 65 -> 36,
+// 64 -> 64 41 -> 28, 32 -> 32 77 -> 64).
 constexpr int CBX = 8, CBY = 4;                   // box, z planes by the variant
 constexpr int CPX = CBX + 2, CPY = CBY + 2;       // halo points per y, y per z
 // LDS layout, in 16-byte words: a point, a y and a z of the halo
@@ -100,7 +104,7 @@ constexpr int conv_zw(int cin) { return CPY * conv_yw(cin); }
 enum ConvEnd { kRelu, kHead, kPlain, kMask };
 
 template <int CIN, int NTW, int WN, int MTW, int WM, int END>
-__global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CIN == 128 ? 2 : 3))) void k_conv(ConvArgs a)
+__global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CIN == 192 ? 1 : CIN == 128 ? 2 : 3))) void k_conv(ConvArgs a)
 {
     static_assert(MTW % 2 == 0, "two tiles of 16 points make one z plane of the box");
     constexpr int NT = 64 * WN * WM, BZ = MTW * WM / 2, KS = (27 * CIN + 31) / 32, CW = CIN / 8;
@@ -117,10 +121,12 @@ __global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CI
     // this wave's weights: tile nt of step s at ((s * tiles + nt) * 64 + lane) * 8
     const int nt0 = (blockIdx.y * WN + wn) * NTW;
     const long long wstep = (long long)(a.coutp / 16) * 512;
-    const bf16_t *wl = a.w + ((long long)nt0 * 64 + lane) * 8;
+    const int wlane = (nt0 * 64 + lane) * 8;
     // steps ahead: nine (a z plane of taps) where a step is two tiles, three
-    // where it is more; all of the few steps of 8 and 16 channels
-    constexpr int kRing = CIN < 32 ? KS : NTW <= 2 ? 9 : 3;
+    // where it is more or the masks take the registers (nine spilled there:
+    // 32 -> 32 channels 87 us against 64); all of the few steps of 8 and 16
+    // channels
+    constexpr int kRing = CIN < 32 ? KS : NTW <= 2 && !(END == kMask && MTW == 4) ? 9 : 3;
     // staging: LN lanes take one y of the halo, 16 bytes each, YR of them at a time
     constexpr int LN = CPX * CW, Y1 = NT / LN, YR = Y1 >= CPY ? Y1 / CPY * CPY : Y1 >= 3 ? 3 : Y1;
     constexpr int NS = (CPY * (BZ + 2) + YR - 1) / YR;
@@ -159,7 +165,7 @@ __global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CI
 #pragma unroll
     for (int s = 0; s < kRing; ++s)
 #pragma unroll
-        for (int n = 0; n < NTW; ++n) W[s][n] = as_bf(ld16(wl + s * wstep + 512 * n));
+        for (int n = 0; n < NTW; ++n) W[s][n] = as_bf(ld16(a.w + s * wstep + wlane + 512 * n));
     // the ReLU masks of the lane's outputs, ready when the sums are
     u32x2 mask[END == kMask ? MTW : 1][NTW];
     if constexpr (END == kMask)
@@ -193,25 +199,45 @@ __global__ __launch_bounds__(64 * WN * WM) __attribute__((amdgpu_waves_per_eu(CI
             }
         }
     } else {
-        constexpr int CC = CIN / 32;
+        // A step's points are read from LDS one step ahead and its weights
+        // loaded kRing steps ahead; the scheduling barriers keep them there
+        // (left to itself the compiler moves a load down to its use, and
+        // every step waits for memory).
+        constexpr int CC = CIN / 32, QN = 9 * CC;
+        static_assert(QN % kRing == 0 && KS == 3 * QN);
         const u32x4 *xl = Xs + lrow + g;
+        auto at = [](int q) { return PW * (q / CC % 3) + YW * (q / CC / 3) + 4 * (q % CC); };
+        bf16x8 X[2][MTW];
+#pragma unroll
+        for (int m = 0; m < MTW; ++m) X[0][m] = as_bf(xl[mrow(m)]);
+        // (the last kRing steps load past the weights, into the array's
+        // padding, and the last one reads its points again)
+        const bf16_t *wr = a.w + kRing * wstep;
 #pragma unroll 1
-        for (int tz = 0; tz < 3; ++tz, xl += ZW) {
+        for (int tz = 0; tz < 3; ++tz) {
+            const u32x4 *xn = tz < 2 ? xl + ZW : xl;
 #pragma unroll
-            for (int q = 0; q < 9 * CC; ++q) {
-                const int t = q / CC, at = PW * (t % 3) + YW * (t / 3) + 4 * (q % CC);
-                bf16x8 X[MTW];
+            for (int q = 0; q < QN; ++q) {
+                // (after an odd number of steps the next points lie in X[1])
+                bf16x8(&Xq)[MTW] = X[q & 1], (&Xp)[MTW] = X[(q + 1) & 1];
 #pragma unroll
-                for (int m = 0; m < MTW; ++m) X[m] = as_bf(xl[at + mrow(m)]);
+                for (int m = 0; m < MTW; ++m)
+                    Xp[m] = as_bf(q + 1 < QN ? xl[at(q + 1) + mrow(m)] : xn[mrow(m)]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int m = 0; m < MTW; ++m)
 #pragma unroll
                     for (int n = 0; n < NTW; ++n)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[q % kRing][n], X[m], acc[m][n], 0, 0, 0);
-                const int sn = min(tz * 9 * CC + q + kRing, KS - 1);
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[q % kRing][n], Xq[m], acc[m][n], 0, 0, 0);
 #pragma unroll
-                for (int n = 0; n < NTW; ++n) W[q % kRing][n] = as_bf(ld16(wl + sn * wstep + 512 * n));
+                for (int n = 0; n < NTW; ++n) W[q % kRing][n] = as_bf(ld16(wr + q * wstep + wlane + 512 * n));
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (QN & 1)
+#pragma unroll
+                for (int m = 0; m < MTW; ++m) X[0][m] = X[1][m];
+            wr += QN * wstep;
+            xl = xn;
         }
     }
 
@@ -308,6 +334,68 @@ __host__ __device__ inline int wgrad_rows(int nx) { return WT + (WT - 1) / nx + 
 // away from a multiple of n, relative to the quotient more than the rounding
 __device__ inline int small_div(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
 
+// Bias gradient partials of 4096 points, by workgroups of the weight
+// gradient's launch: a value per channel and k < ph = 256 / c sums the points
+// k, k + ph, ... in turn, and the ph sums are added in turn.  A workgroup
+// takes 32 channels and stages 384 points of them in LDS at a time, the next
+// ones on their way meanwhile; a thread has two of the 256 sums at most.  Its
+// chain of loads (20 us a layer as a launch of 200 workgroups) passes beside
+// the matrix work.
+constexpr int BG_CHUNK = 4096, BG_PTS = 384, BG_CH = 32;
+constexpr int kBiasLds = BG_PTS * BG_CH * 2 + 256 * 4;
+
+__device__ inline void bias_part(const WgradArgs &a, bf16_t *st, int chunk, int c0)
+{
+    float *red = reinterpret_cast<float *>(st + BG_PTS * BG_CH);
+    const int c = a.cout, w = c < BG_CH ? c : BG_CH, ph = 256 / c, cw = w / 8;
+    const int ch = threadIdx.x % w, k0 = threadIdx.x / w, k1 = k0 + 192 / w;
+    const int P = a.nx * a.ny * a.nz, p0 = chunk * BG_CHUNK, p1 = min(p0 + BG_CHUNK, P);
+    constexpr int NL = BG_PTS * BG_CH / 8 / 192;
+    u32x4 v[NL];
+    auto load = [&](int pb) {
+        const int n = min(BG_PTS, p1 - pb) * cw;
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int q = min((int)threadIdx.x + 192 * u, n - 1);
+            v[u] = ld16(a.g + (long long)(pb + q / cw) * c + c0 + 8 * (q % cw));
+        }
+    };
+    float s0 = 0.f, s1 = 0.f;
+    auto sum = [&](int k, int n, float &s) {
+        int i = k;
+        for (; i + 15 * ph < n; i += 16 * ph) {
+            bf16_t e[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) e[u] = st[(i + u * ph) * w + ch];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s += bf2f(e[u]);
+        }
+        for (; i < n; i += ph) s += bf2f(st[i * w + ch]);
+    };
+    load(p0);
+    for (int pb = p0; pb < p1; pb += BG_PTS) {
+        const int n = min(BG_PTS, p1 - pb);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int q = threadIdx.x + 192 * u;
+            if (q < n * cw) st16(st + 8 * q, v[u]);
+        }
+        __syncthreads();
+        if (pb + BG_PTS < p1) load(pb + BG_PTS);
+        if (k0 < ph) sum(k0, n, s0);
+        if (k1 < ph) sum(k1, n, s1);
+    }
+    if (k0 < ph) red[k0 * w + ch] = s0;
+    if (k1 < ph) red[k1 * w + ch] = s1;
+    __syncthreads();
+    if ((int)threadIdx.x < w) {
+        float s = red[ch];
+        for (int j = 1; j < ph; ++j) s += red[j * w + ch];
+        a.bpart[(long long)chunk * c + c0 + ch] = s;
+    }
+}
+
 template <int MCO, int NCI>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_wgrad(WgradArgs a)
 {
@@ -316,7 +404,13 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k
     constexpr int gn = WT * 16;
     const int tid = threadIdx.x, lane = tid & 63, ty = tid >> 6, g = lane >> 4, r16 = lane & 15;
     bf16_t *Xs = lds + ty * NCI * xn, *Gs = lds + 3 * NCI * xn;
-    const int tz = blockIdx.y % 3, blk = blockIdx.y / 3;
+    // the first workgroups of the launch sum the bias gradient
+    const int nbias = (a.cout + BG_CH - 1) / BG_CH, by = (int)blockIdx.y - nbias;
+    if (by < 0) {
+        if ((int)blockIdx.x * BG_CHUNK < a.nx * a.ny * a.nz) bias_part(a, lds, blockIdx.x, BG_CH * blockIdx.y);
+        return;
+    }
+    const int tz = by % 3, blk = by / 3;
     const int nciB = (a.cin + 16 * NCI - 1) / (16 * NCI);
     const int co0 = blk / nciB * 16 * MCO, ci0 = blk % nciB * 16 * NCI;
     const int P = a.nx * a.ny * a.nz;
@@ -417,69 +511,13 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k
                 *reinterpret_cast<f32x4 *>(part + (((9 * tz + 3 * ty + j) * MCO + m) * NCI + n) * 256 + 4 * lane) = acc[j][m][n];
 }
 
-// Bias gradient partials of 4096 points, ph = 256 / c threads a channel:
-// thread k sums the points k, k + ph, ... in turn, and the ph sums are added
-// in turn.  A workgroup takes 32 channels and stages 512 points of them in
-// LDS at a time, 16 bytes a lane, the next 512 on their way meanwhile: one
-// chain of 2-byte loads a thread had taken 224 us a layer on average at 65 x
-// 65 x 193, without the loads ahead 23 us
-constexpr int BG_CHUNK = 4096, BG_PTS = 512, BG_CH = 32;
-
-__global__ __launch_bounds__(256) void k_bias_part(const bf16_t *g, int P, int c, float *part)
-{
-    __shared__ __attribute__((aligned(16))) bf16_t st[BG_PTS * BG_CH];
-    __shared__ float red[256];
-    const int w = c < BG_CH ? c : BG_CH, ph = 256 / c, ch = threadIdx.x % w, k = threadIdx.x / w, c0 = blockIdx.y * BG_CH;
-    const int p0 = blockIdx.x * BG_CHUNK, p1 = min(p0 + BG_CHUNK, P);
-    float s = 0.f;
-    constexpr int NL = BG_PTS * BG_CH / 8 / 256;
-    u32x4 v[NL];
-    auto load = [&](int pb) {   // 512 points on their way while those before are summed
-        const int n = min(BG_PTS, p1 - pb) * (w / 8);
-#pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int q = min((int)threadIdx.x + 256 * u, n - 1), i = q / (w / 8), e = q % (w / 8);
-            v[u] = ld16(g + (long long)(pb + i) * c + c0 + 8 * e);
-        }
-    };
-    load(p0);
-    for (int pb = p0; pb < p1; pb += BG_PTS) {
-        const int n = min(BG_PTS, p1 - pb);
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int q = threadIdx.x + 256 * u;
-            if (q < n * (w / 8)) st16(st + 8 * q, v[u]);
-        }
-        __syncthreads();
-        if (pb + BG_PTS < p1) load(pb + BG_PTS);
-        if (k < ph) {
-            int i = k;
-            for (; i + 15 * ph < n; i += 16 * ph) {
-                bf16_t v[16];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) v[u] = st[(i + u * ph) * w + ch];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) s += bf2f(v[u]);
-            }
-            for (; i < n; i += ph) s += bf2f(st[i * w + ch]);
-        }
-    }
-    if (k < ph) red[threadIdx.x] = s;
-    __syncthreads();
-    if (k == 0) {
-        for (int j = 1; j < ph; ++j) s += red[j * w + ch];
-        part[(long long)blockIdx.x * c + c0 + ch] = s;
-    }
-}
-
 // Sums of partials in turn, added to the layer's weight gradient, and (the
 // last workgroups of the grid) to its bias gradient: 64 values a workgroup;
 // its 256 threads load 64 partials of each into LDS, and one wave adds them
 // in order while the next 64 are on their way
 template <int MCO, int NCI>
-__global__ __launch_bounds__(256) void k_wgrad_sum(WgradArgs a, int nchunks, int kpad, float *grad, const float *bpart,
-                                                   int nbparts, float *bgrad)
+__global__ __launch_bounds__(256) void k_wgrad_sum(WgradArgs a, int nchunks, int kpad, float *grad, int nbparts,
+                                                   float *bgrad)
 {
     __shared__ float st[2][64][64];
     constexpr int N = 27 * MCO * NCI * 256;
@@ -490,7 +528,7 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(WgradArgs a, int nchunks, int
     const int n = bias ? nbparts : nchunks;
     const long long ld = bias ? a.cout : N;
     const bool live = !bias || bi < a.cout;
-    const float *p = bias ? bpart + bi : a.part + (long long)blockIdx.y * nchunks * N + i;
+    const float *p = bias ? a.bpart + bi : a.part + (long long)blockIdx.y * nchunks * N + i;
     float v[16], s = 0.f;
     auto load = [&](int c0) {
 #pragma unroll
@@ -905,7 +943,10 @@ void launch_conv_k(hipStream_t s, const ConvArgs &a)
 // The network's layers and their input gradients: boxes of eight planes
 // while the halo fits three workgroups a CU (32 channels, 54 KB of 160), of
 // four or two above that; channels split over two waves, or two workgroups,
-// where the box has few tiles of points
+// where the box has few tiles of points.  Four tiles of points a wave at 192
+// channels, one workgroup a CU: 131 -> 108 us at 33 x 33 x 97, 29 -> 24 at 17
+// x 17 x 49.  The same at 96 and 128 channels gains 4 to 17% on the largest
+// grid of a level and loses 9 to 80% on the smallest.
 int launch_conv(hipStream_t s, const ConvArgs &a)
 {
     const bool fwd = a.bias != nullptr;
@@ -929,7 +970,7 @@ int launch_conv(hipStream_t s, const ConvArgs &a)
     case 128128:
         fwd ? launch_conv_k<128, 2, 2, 2, 2, kRelu>(s, a) : launch_conv_k<128, 2, 2, 2, 2, kMask>(s, a);
         return 0;
-    case 192064: launch_conv_k<192, 2, 2, 2, 4, kRelu>(s, a); return 0;
+    case 192064: launch_conv_k<192, 2, 2, 4, 2, kRelu>(s, a); return 0;
     }
     return -1;   // no layer of the network
 }
@@ -947,14 +988,15 @@ int wgrad_blocks(int cin, int cout)
 template <int MCO, int NCI>
 void launch_wgrad_k(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad)
 {
-    const int lds = (3 * NCI * wgrad_rows(a.nx) + MCO * WT) * 32 + 3 * wgrad_rows(a.nx) * 4;   // at most 40 KB
+    const int lds = std::max((3 * NCI * wgrad_rows(a.nx) + MCO * WT) * 32 + 3 * wgrad_rows(a.nx) * 4, kBiasLds);   // at most 40 KB
     const long long P = (long long)a.nx * a.ny * a.nz;
     const int nch = wgrad_chunks(P), blocks = wgrad_blocks(a.cin, a.cout), nb = (int)((P + BG_CHUNK - 1) / BG_CHUNK);
-    float *bpart = a.part + (long long)nch * blocks * 27 * MCO * NCI * 256;
-    k_wgrad<MCO, NCI><<<dim3(nch, 3 * blocks), 192, lds, s>>>(a);
-    k_bias_part<<<dim3(nb, (a.cout + BG_CH - 1) / BG_CH), 256, 0, s>>>(a.g, (int)P, a.cout, bpart);
+    const int nbias = (a.cout + BG_CH - 1) / BG_CH;
+    WgradArgs w = a;
+    w.bpart = a.part + (long long)nch * blocks * 27 * MCO * NCI * 256;
+    k_wgrad<MCO, NCI><<<dim3(nch, 3 * blocks + nbias), 192, lds, s>>>(w);
     k_wgrad_sum<MCO, NCI><<<dim3(27 * MCO * NCI * 4 + 1, blocks), 256, 0, s>>>(
-        a, nch, kpad, grad, bpart, nb, bgrad);
+        w, nch, kpad, grad, nb, bgrad);
 }
 }  // namespace
 

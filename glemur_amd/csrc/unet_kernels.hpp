@@ -25,7 +25,7 @@ using bf16_t = uint16_t;
 struct ConvArgs {
     const bf16_t *in = nullptr;
     long long ldi = 0;
-    const bf16_t *w = nullptr;   // packed by launch_pack
+    const bf16_t *w = nullptr;   // packed by launch_pack; 9 * 32 * coutp more may be read
     const float *bias = nullptr;
     bf16_t *out = nullptr;
     long long ldo = 0;
@@ -52,6 +52,7 @@ struct WgradArgs {
     int nx = 0, ny = 0, nz = 0;
     int cin = 0, cout = 0;    // cin 8, 16 or a multiple of 32; cout 16 or a multiple of 32
     float *part = nullptr;
+    float *bpart = nullptr;   // (set by launch_wgrad: the bias partials, behind the weights')
 };
 void launch_wgrad(hipStream_t s, const WgradArgs &a, int kpad, float *grad, float *bgrad);
 long long wgrad_part_floats(int nx, int ny, int nz, int cin, int cout);
