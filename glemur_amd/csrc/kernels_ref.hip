@@ -387,13 +387,8 @@ __global__ void __launch_bounds__(kBlock) k_jclassic(Geo g, const double *X, con
     for (int c = 0; c < 3; ++c) J[c * g.P + a0] = Jv[c];
 }
 
-__global__ void __launch_bounds__(kBlock) k_jstokes(Geo g, const double *X, const double *B, double *J)
+__device__ __forceinline__ void jstokes_point(const Geo &g, const double *X, const double *B, long long a, double Jv[3])
 {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long N = (long long)g.nx * g.ny * g.nz;
-    if (t >= N) return;
-    int i = (int)(t % g.nx) + 1, j = (int)((t / g.nx) % g.ny) + 1, k = (int)(t / ((long long)g.nx * g.ny)) + 1;
-    long long a = gidx(g, i, j, k);
     long long im = a - 1, ip = a + 1, jm = a - g.sx, jp = a + g.sx, km = a - g.sxy, kp = a + g.sxy;
     // diamonds in circulation order (src/current.cu:291-382)
     const long long quad[3][4] = {{im, jm, ip, jp}, {jm, km, jp, kp}, {km, im, kp, ip}};
@@ -412,8 +407,17 @@ __global__ void __launch_bounds__(kBlock) k_jstokes(Geo g, const double *X, cons
         }
         II[q] = diamond(d, bv, NA[q]);
     }
-    double Jv[3];
     solve_na(NA, II, Jv);
+}
+__global__ void __launch_bounds__(kBlock) k_jstokes(Geo g, const double *X, const double *B, double *J)
+{
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    long long N = (long long)g.nx * g.ny * g.nz;
+    if (t >= N) return;
+    int i = (int)(t % g.nx) + 1, j = (int)((t / g.nx) % g.ny) + 1, k = (int)(t / ((long long)g.nx * g.ny)) + 1;
+    long long a = gidx(g, i, j, k);
+    double Jv[3];
+    jstokes_point(g, X, B, a, Jv);
     J[a] = Jv[0];
     J[g.P + a] = Jv[1];
     J[2 * g.P + a] = Jv[2];
@@ -459,9 +463,12 @@ __global__ void __launch_bounds__(kBlock) k_gradp(Geo g, const double *X, const 
 // (N is a template argument), and x and u are replaced in place: the stage
 // copies and their way back cost three further passes (65 x 65 x 193 with
 // inertia: 61 us and 26 us of copies a stage before).
-template <int N>
-__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict__ tab, double dt, double *X,
-                                               const double *__restrict__ B, const double *__restrict__ J,
+// CUR: the current by JStokes is computed here from X and B instead of read
+// (a pass of 21 us and 48 bytes a point), stored if J is given; the neighbours
+// of X are read, so the positions go to another array Xo (X itself otherwise).
+template <int N, bool CUR>
+__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict__ tab, double dt, const double *X,
+                                               double *Xo, const double *__restrict__ B, double *J,
                                                const double *__restrict__ G, double *K, const double *__restrict__ det,
                                                double *U, double *KU)
 {
@@ -472,11 +479,14 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict_
     const long long P3 = 3 * g.P;
     double w[N + 1], jv[3], bv[3], kv[3], x[3], kp[N + 1][3], gp[3] = {0, 0, 0};
     for (int m = 0; m <= N; ++m) w[m] = tab->b[m + (N + 1) * 6] - tab->b[m + N * 6];
-    ld3(J, g.P, a, jv);
+    if constexpr (CUR) jstokes_point(g, X, B, a, jv);
+    else ld3(J, g.P, a, jv);
     ld3(B, g.P, a, bv);
     ld3(X, g.P, a, x);
 #pragma unroll
     for (int m = 0; m < N; ++m) ld3(K + m * P3, g.P, a, kp[m]);
+    if (CUR && J)
+        for (int l = 0; l < 3; ++l) J[l * g.P + a] = jv[l];
     if (g.pressure) ld3(G, g.P, a, gp);
     cross3(jv, bv, kv);
     if (g.inertia) {
@@ -504,12 +514,12 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict_
             }
             K[N * P3 + l * g.P + a] = kp[N][l];
             KU[N * P3 + l * g.P + a] = up[N][l];
-            X[l * g.P + a] = x[l];
+            Xo[l * g.P + a] = x[l];
             U[l * g.P + a] = v;
         }
         return;
     }
-    if (g.jxbAver) {
+    if (!CUR && g.jxbAver) {
         // jxbAver (src/rungeKutta.cu:172-177, 357-443): (1 - w) J x B plus
         // w/6 J x B of each face neighbour that is an inner point, in the
         // order -x, +x, -y, +y, -z, +z; the +z neighbour's B is read at its
@@ -539,7 +549,7 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict_
 #pragma unroll
         for (int m = 0; m <= N; ++m) x[l] += w[m] * kp[m][l];
         K[N * P3 + l * g.P + a] = kv[l];
-        X[l * g.P + a] = x[l];
+        Xo[l * g.P + a] = x[l];
     }
 }
 
@@ -861,17 +871,25 @@ void launch_gradp(hipStream_t s, const Geo &g, const double *X, const double *de
 {
     hipLaunchKernelGGL(k_gradp, dim3(blocks_for(ninner(g))), dim3(kBlock), 0, s, g, X, det, G);
 }
-void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, double *X, const double *B,
-               const double *J, const double *G, double *K, const double *det, double *U, double *KU)
+template <int N>
+static void launch_kk_n(hipStream_t s, const Geo &g, const Tableau *tab, double dt, const double *X, double *Xo,
+                        const double *B, double *J, const double *G, double *K, const double *det, double *U, double *KU,
+                        bool cur)
 {
     const dim3 nb(blocks_for(ninner(g))), nt(kBlock);
+    if (cur) hipLaunchKernelGGL((k_kk<N, true>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
+    else hipLaunchKernelGGL((k_kk<N, false>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
+}
+void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X, double *Xo,
+               const double *B, double *J, const double *G, double *K, const double *det, double *U, double *KU, bool cur)
+{
     switch (n) {
-    case 0: hipLaunchKernelGGL(k_kk<0>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
-    case 1: hipLaunchKernelGGL(k_kk<1>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
-    case 2: hipLaunchKernelGGL(k_kk<2>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
-    case 3: hipLaunchKernelGGL(k_kk<3>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
-    case 4: hipLaunchKernelGGL(k_kk<4>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
-    default: hipLaunchKernelGGL(k_kk<5>, nb, nt, 0, s, g, tab, dt, X, B, J, G, K, det, U, KU); break;
+    case 0: launch_kk_n<0>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
+    case 1: launch_kk_n<1>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
+    case 2: launch_kk_n<2>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
+    case 3: launch_kk_n<3>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
+    case 4: launch_kk_n<4>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
+    default: launch_kk_n<5>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
     }
 }
 int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const double *X, const double *K, double *Xnew,

@@ -759,15 +759,19 @@ extern "C" int gm_gradp(gm_ctx *c)
     gmd::launch_gradp(c->stream, c->geo, c->X64[c->cur], c->det, c->G64);
     return GM_OK;
 }
+static void kk(gm_ctx *c, int n, double dt, const double *X, double *Xo, double *J, bool cur)
+{
+    const bool in = c->p.inertia;
+    gmd::launch_kk(c->stream, c->geo, c->tab_dev, n, dt, X, Xo, c->B64, J, c->G64, c->K64, in ? c->det : nullptr,
+                   in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr, cur);
+}
 extern "C" int gm_rk_kk(gm_ctx *c, int n, double dt)
 {
     if (!c) return fail(GM_ERR_ARG, "null context");
     if (int r = need_f64(c, "gm_rk_kk")) return r;
     if (n < 0 || n > 5) return fail(GM_ERR_ARG, "stage index must be 0..5");
     // xb <- xb_tmp, uu <- uu_tmp (src/main.cu:288-305): written in place
-    const bool in = c->p.inertia;
-    gmd::launch_kk(c->stream, c->geo, c->tab_dev, n, dt, c->X64[c->cur], c->B64, c->J64, c->G64, c->K64,
-                   in ? c->det : nullptr, in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr);
+    kk(c, n, dt, c->X64[c->cur], c->X64[c->cur], c->J64, false);
     if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, c->X64[c->cur]);
     return GM_OK;
 }
@@ -1006,9 +1010,27 @@ static int step_per_kernel(gm_ctx *c)
         return leave();
     }
     const double dt = h.dt;
-    for (int n = 0; n < 6; ++n) {
-        if (n > 0 && (r = fields_per_kernel(c))) return r;
-        if ((r = gm_rk_kk(c, n, dt))) return r;
+    if (gm::starts(c->p.jMethod, "Stokes ") && !c->p.jxbAver) {
+        // the current within the slope's launch; the stage positions go back
+        // and forth between the current buffer and the one behind the
+        // candidate, whose ghost layers are the same, and end in the current
+        // one.  J64 holds the last stage's current, as from the calls one by one.
+        double *x[2] = {c->X64[c->cur], c->X64[(c->cur + 2) % 3]};
+        for (int n = 0; n < 6; ++n) {
+            double *X = x[n & 1], *Xo = x[~n & 1];
+            if (n > 0) {
+                gmd::launch_b_all(c->stream, c->geo, X, c->B0_64, c->B64, c->det);
+                if ((r = gm_set_peri(c, GM_FIELD_B))) return r;
+                if (c->p.pressure) gmd::launch_gradp(c->stream, c->geo, X, c->det, c->G64);
+            }
+            kk(c, n, dt, X, Xo, n == 5 ? c->J64 : nullptr, true);
+            if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, Xo);
+        }
+    } else {
+        for (int n = 0; n < 6; ++n) {
+            if (n > 0 && (r = fields_per_kernel(c))) return r;
+            if ((r = gm_rk_kk(c, n, dt))) return r;
+        }
     }
     double md = 0;
     if ((r = gm_rk_xnewstar(c, &md))) return r;
