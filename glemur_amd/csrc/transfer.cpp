@@ -39,10 +39,17 @@ struct Staging {
     int device = -1;
     hipEvent_t ev[kSlots] = {};
 
-    bool ready()
+    // Events are recorded on streams of their own device only: a caller whose
+    // current device is another one than the stream's goes the plain way
+    bool ready(hipStream_t s)
     {
         int d = 0;
-        if (hipGetDevice(&d) != hipSuccess) return false;
+        hipDevice_t sd = 0;
+        if (hipGetDevice(&d) != hipSuccess || hipStreamGetDevice(s, &sd) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (sd != d) return false;
         if (!buf && hipHostMalloc((void **)&buf, kSlots * kSlotBytes, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
             buf = nullptr;
@@ -223,7 +230,7 @@ hipError_t copy_to_device(hipStream_t s, void *dst, const void *src, size_t byte
     if (bytes >= kMinUp && pageable(src)) {
         Staging &g = staging();
         std::unique_lock<std::mutex> l(g.m, std::try_to_lock);
-        if (l.owns_lock() && g.ready()) {
+        if (l.owns_lock() && g.ready(s)) {
             try {
                 Chunks c(g.buf, (char *)src, bytes, true);
                 return up(s, (char *)dst, c, g.ev);
@@ -239,7 +246,7 @@ hipError_t copy_to_host(hipStream_t s, void *dst, const void *src, size_t bytes)
     if (bytes >= kMinDown && pageable(dst)) {
         Staging &g = staging();
         std::unique_lock<std::mutex> l(g.m, std::try_to_lock);
-        if (l.owns_lock() && g.ready()) {
+        if (l.owns_lock() && g.ready(s)) {
             try {
                 Chunks c(g.buf, (char *)dst, bytes, false);
                 return down(s, (const char *)src, c, g.ev);
