@@ -79,6 +79,11 @@ void launch_b_all(hipStream_t s, const Geo &g, const double *X, const double *B0
 // read only then.  Without inertia U, KU and det may be null.
 void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X, double *Xo,
                const double *B, double *J, const double *G, double *K, const double *det, double *U, double *KU, bool cur);
+// The last stage with the current formed and x_new, u_new and the error maxima
+// of launch_xnewstar in the same pass; returns the number of partials written.
+int launch_kk_end(hipStream_t s, const Geo &g, const Tableau *tab, double dt, const double *X, double *Xo, const double *B,
+                  double *J, const double *G, double *K, const double *det, double *U, double *KU, double *Xnew,
+                  double *Unew, double *partials, int *nanflag);
 // x_new (and u_new with inertia) and per-block error maxima of the
 // positions; returns the number of partials written.
 int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const double *X, const double *K,

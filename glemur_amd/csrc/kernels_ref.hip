@@ -466,14 +466,52 @@ __global__ void __launch_bounds__(kBlock) k_gradp(Geo g, const double *X, const 
 // CUR: the current by JStokes is computed here from X and B instead of read
 // (a pass of 21 us and 48 bytes a point), stored if J is given; the neighbours
 // of X are read, so the positions go to another array Xo (X itself otherwise).
-template <int N, bool CUR>
-__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict__ tab, double dt, const double *X,
-                                               double *Xo, const double *__restrict__ B, double *J,
-                                               const double *__restrict__ G, double *K, const double *__restrict__ det,
-                                               double *U, double *KU)
+// END (after the last stage): x_new, x_star and u_new of xNewStar as well, as
+// k_xnewstar forms them from the same slopes: that pass reads all twelve again
+// and its output is first copied for the ghost layers, which the candidate's
+// buffer already holds (65 x 65 x 193 with inertia: 78 + 63 us and the copy ->
+// 88 us; 30 attempts with their transfers 21.0 -> 19.2 ms).
+struct KkEnd {
+    double *Xnew, *Unew, *partials;
+    int *nanflag;
+};
+__device__ __forceinline__ void new_star(const Geo &g, const Tableau *__restrict__ tab, long long a, const double x[3],
+                                         const double (*kp)[3], const KkEnd &E, double &dmax, bool &nan)
 {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)g.nx * g.ny * g.nz) return;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        double xn = x[l], xs = xn;
+        if (l < 2 || g.zUpdate)
+#pragma unroll
+            for (int s = 0; s < 6; ++s) {
+                xn += tab->c[s] * kp[s][l];
+                xs += tab->cs[s] * kp[s][l];
+            }
+        E.Xnew[l * g.P + a] = xn;
+        const double d = fabs(xn - xs);
+        if (d != d) nan = true;
+        dmax = nb_max(dmax, d);
+    }
+}
+// Maximum of a workgroup's values >= 0 into its slot
+__device__ __forceinline__ void block_max(double m, double *partials)
+{
+    __shared__ double wmax[kBlock / 64];
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double r = 0;
+        for (int w = 0; w < kBlock / 64; ++w) r = nb_max(r, wmax[w]);
+        partials[blockIdx.x] = r;
+    }
+}
+template <int N, bool CUR, bool END>
+__device__ __forceinline__ void kk_point(const Geo &g, const Tableau *__restrict__ tab, double dt, const double *X,
+                                         double *Xo, const double *__restrict__ B, double *J,
+                                         const double *__restrict__ G, double *K, const double *__restrict__ det,
+                                         double *U, double *KU, const KkEnd &E, long long t, double &dmax, bool &nan)
+{
     int i = (int)(t % g.nx), j = (int)((t / g.nx) % g.ny), k = (int)(t / ((long long)g.nx * g.ny));
     long long a = gidx(g, i + 1, j + 1, k + 1);
     const long long P3 = 3 * g.P;
@@ -516,7 +554,13 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict_
             KU[N * P3 + l * g.P + a] = up[N][l];
             Xo[l * g.P + a] = x[l];
             U[l * g.P + a] = v;
+            if constexpr (END) {   // u5 (src/rungeKutta.cu:311-322); no error term
+#pragma unroll
+                for (int m = 0; m <= N; ++m) v += tab->c[m] * up[m][l];
+                E.Unew[l * g.P + a] = v;
+            }
         }
+        if constexpr (END) new_star(g, tab, a, x, kp, E, dmax, nan);
         return;
     }
     if (!CUR && g.jxbAver) {
@@ -551,6 +595,30 @@ __global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict_
         K[N * P3 + l * g.P + a] = kv[l];
         Xo[l * g.P + a] = x[l];
     }
+    if constexpr (END) new_star(g, tab, a, x, kp, E, dmax, nan);
+}
+template <int N, bool CUR>
+__global__ void __launch_bounds__(kBlock) k_kk(Geo g, const Tableau *__restrict__ tab, double dt, const double *X,
+                                               double *Xo, const double *__restrict__ B, double *J,
+                                               const double *__restrict__ G, double *K, const double *__restrict__ det,
+                                               double *U, double *KU)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    double m;
+    bool nan;
+    if (t < (long long)g.nx * g.ny * g.nz) kk_point<N, CUR, false>(g, tab, dt, X, Xo, B, J, G, K, det, U, KU, {}, t, m, nan);
+}
+__global__ void __launch_bounds__(kBlock) k_kk_end(Geo g, const Tableau *__restrict__ tab, double dt, const double *X,
+                                                   double *Xo, const double *__restrict__ B, double *J,
+                                                   const double *__restrict__ G, double *K,
+                                                   const double *__restrict__ det, double *U, double *KU, KkEnd E)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    double m = 0;
+    bool nan = false;
+    if (t < (long long)g.nx * g.ny * g.nz) kk_point<5, true, true>(g, tab, dt, X, Xo, B, J, G, K, det, U, KU, E, t, m, nan);
+    if (nan) atomicOr(E.nanflag, 1);
+    block_max(m, E.partials);
 }
 
 // --------------------------------------------------------------- xNewStar
@@ -558,7 +626,6 @@ __global__ void __launch_bounds__(kBlock) k_xnewstar(Geo g, const Tableau *tab, 
                                                      double *Xnew, double *partials, int *nanflag, const double *U,
                                                      const double *KU, double *Unew)
 {
-    __shared__ double wmax[kBlock / 64];
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     long long N = (long long)g.nx * g.ny * g.nz;
     double m = 0;
@@ -588,14 +655,7 @@ __global__ void __launch_bounds__(kBlock) k_xnewstar(Geo g, const Tableau *tab, 
             }
         if (nan) atomicOr(nanflag, 1);
     }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double r = 0;
-        for (int w = 0; w < kBlock / 64; ++w) r = nb_max(r, wmax[w]);
-        partials[blockIdx.x] = r;
-    }
+    block_max(m, partials);
 }
 
 __global__ void __launch_bounds__(1024) k_max_final(const double *partials, int n, const int *nanflag, double *out)
@@ -891,6 +951,15 @@ void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt
     case 4: launch_kk_n<4>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
     default: launch_kk_n<5>(s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU, cur); break;
     }
+}
+int launch_kk_end(hipStream_t s, const Geo &g, const Tableau *tab, double dt, const double *X, double *Xo, const double *B,
+                  double *J, const double *G, double *K, const double *det, double *U, double *KU, double *Xnew,
+                  double *Unew, double *partials, int *nanflag)
+{
+    const int nb = blocks_for(ninner(g));
+    hipLaunchKernelGGL(k_kk_end, dim3(nb), dim3(kBlock), 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU,
+                       KkEnd{Xnew, Unew, partials, nanflag});
+    return nb;
 }
 int launch_xnewstar(hipStream_t s, const Geo &g, const Tableau *tab, const double *X, const double *K, double *Xnew,
                     double *partials, int *nanflag, const double *U, const double *KU, double *Unew)

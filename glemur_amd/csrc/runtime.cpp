@@ -775,14 +775,16 @@ extern "C" int gm_rk_kk(gm_ctx *c, int n, double dt)
     if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, c->X64[c->cur]);
     return GM_OK;
 }
+// one per-block maximum per 256 inner points, kept for later attempts
+static int ensure_xns(gm_ctx *c)
+{
+    return c->xns_part ? GM_OK : dalloc(&c->xns_part, (size_t)((c->N + 255) / 256));
+}
 extern "C" int gm_rk_xnewstar(gm_ctx *c, double *maxDelta)
 {
     if (!c) return fail(GM_ERR_ARG, "null context");
     if (int r = need_f64(c, "gm_rk_xnewstar")) return r;
-    if (!c->xns_part) {   // one per-block maximum per 256 inner points, kept for later attempts
-        int r = dalloc(&c->xns_part, (size_t)((c->N + 255) / 256));
-        if (r) return r;
-    }
+    if (int r = ensure_xns(c)) return r;
     double *parts = c->xns_part;
     (void)hipMemsetAsync(c->nanflag, 0, sizeof(int), c->stream);
     double *xnew = c->X64[(c->cur + 1) % 3];
@@ -1015,6 +1017,9 @@ static int step_per_kernel(gm_ctx *c)
         // and forth between the current buffer and the one behind the
         // candidate, whose ghost layers are the same, and end in the current
         // one.  J64 holds the last stage's current, as from the calls one by one.
+        // The last slope's launch forms the candidate too.
+        if ((r = ensure_xns(c))) return r;
+        (void)hipMemsetAsync(c->nanflag, 0, sizeof(int), c->stream);
         double *x[2] = {c->X64[c->cur], c->X64[(c->cur + 2) % 3]};
         for (int n = 0; n < 6; ++n) {
             double *X = x[n & 1], *Xo = x[~n & 1];
@@ -1023,17 +1028,30 @@ static int step_per_kernel(gm_ctx *c)
                 if ((r = gm_set_peri(c, GM_FIELD_B))) return r;
                 if (c->p.pressure) gmd::launch_gradp(c->stream, c->geo, X, c->det, c->G64);
             }
-            kk(c, n, dt, X, Xo, n == 5 ? c->J64 : nullptr, true);
+            if (n < 5) {
+                kk(c, n, dt, X, Xo, nullptr, true);
+            } else {
+                const bool in = c->p.inertia;
+                double *xnew = c->X64[(c->cur + 1) % 3];
+                const int parts = gmd::launch_kk_end(
+                    c->stream, c->geo, c->tab_dev, dt, X, Xo, c->B64, c->J64, c->G64, c->K64, in ? c->det : nullptr,
+                    in ? c->U64[c->ucur] : nullptr, in ? c->KU64 : nullptr, xnew, in ? c->U64[c->ucur ^ 1] : nullptr,
+                    c->xns_part, c->nanflag);
+                if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, xnew);
+                gmd::launch_max_final(c->stream, c->xns_part, parts, c->nanflag, c->red_host);
+            }
             if (any_peri(c->p)) gmd::launch_set_grid_peri(c->stream, c->geo, Xo);
         }
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->stream));
     } else {
         for (int n = 0; n < 6; ++n) {
             if (n > 0 && (r = fields_per_kernel(c))) return r;
             if ((r = gm_rk_kk(c, n, dt))) return r;
         }
+        if ((r = gm_rk_xnewstar(c, nullptr))) return r;
     }
-    double md = 0;
-    if ((r = gm_rk_xnewstar(c, &md))) return r;
+    const double md = c->red_host[0];
     const int nan = c->red_host[1] != 0;
     h.nan_seen |= nan;
     rec.nan_seen = nan;
