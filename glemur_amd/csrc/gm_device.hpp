@@ -72,14 +72,14 @@ void launch_gradp(hipStream_t s, const Geo &g, const double *X, const double *de
 // B and det of inner points and of every ghost face (the two above in one launch)
 void launch_b_all(hipStream_t s, const Geo &g, const double *X, const double *B0, double *B, double *det);
 // Slope n (0..5) and the stage positions into Xo (X itself, or another array).
-// With cur the current by JStokes is computed on the way (not with jxbAver; Xo
-// is another array) and stored in J if that is given; otherwise J is read.
+// With cur (stages 0..4) the current by JStokes is computed on the way (not
+// with jxbAver; Xo is another array); otherwise J is read.
 // With g.inertia, K holds the position slopes dt u, KU the velocity slopes,
 // and the stage velocity replaces U (padded SoA, like the positions); det is
 // read only then.  Without inertia U, KU and det may be null.
 void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X, double *Xo,
                const double *B, double *J, const double *G, double *K, const double *det, double *U, double *KU, bool cur);
-// The last stage with the current formed and x_new, u_new and the error maxima
+// The last stage with the current formed and stored in J, and x_new, u_new and the error maxima
 // of launch_xnewstar in the same pass; returns the number of partials written.
 int launch_kk_end(hipStream_t s, const Geo &g, const Tableau *tab, double dt, const double *X, double *Xo, const double *B,
                   double *J, const double *G, double *K, const double *det, double *U, double *KU, double *Xnew,

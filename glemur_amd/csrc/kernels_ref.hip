@@ -464,8 +464,9 @@ __global__ void __launch_bounds__(kBlock) k_gradp(Geo g, const double *X, const 
 // copies and their way back cost three further passes (65 x 65 x 193 with
 // inertia: 61 us and 26 us of copies a stage before).
 // CUR: the current by JStokes is computed here from X and B instead of read
-// (a pass of 21 us and 48 bytes a point), stored if J is given; the neighbours
-// of X are read, so the positions go to another array Xo (X itself otherwise).
+// (a pass of 21 us and 48 bytes a point), stored by the last stage only; the
+// neighbours of X are read, so the positions go to another array Xo (X itself
+// otherwise).
 // END (after the last stage): x_new, x_star and u_new of xNewStar as well, as
 // k_xnewstar forms them from the same slopes: that pass reads all twelve again
 // and its output is first copied for the ghost layers, which the candidate's
@@ -523,7 +524,7 @@ __device__ __forceinline__ void kk_point(const Geo &g, const Tableau *__restrict
     ld3(X, g.P, a, x);
 #pragma unroll
     for (int m = 0; m < N; ++m) ld3(K + m * P3, g.P, a, kp[m]);
-    if (CUR && J)
+    if constexpr (END)
         for (int l = 0; l < 3; ++l) J[l * g.P + a] = jv[l];
     if (g.pressure) ld3(G, g.P, a, gp);
     cross3(jv, bv, kv);
@@ -937,8 +938,12 @@ static void launch_kk_n(hipStream_t s, const Geo &g, const Tableau *tab, double 
                         bool cur)
 {
     const dim3 nb(blocks_for(ninner(g))), nt(kBlock);
-    if (cur) hipLaunchKernelGGL((k_kk<N, true>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
-    else hipLaunchKernelGGL((k_kk<N, false>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
+    if constexpr (N < 5)   // the last stage: launch_kk_end
+        if (cur) {
+            hipLaunchKernelGGL((k_kk<N, true>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
+            return;
+        }
+    hipLaunchKernelGGL((k_kk<N, false>), nb, nt, 0, s, g, tab, dt, X, Xo, B, J, G, K, det, U, KU);
 }
 void launch_kk(hipStream_t s, const Geo &g, const Tableau *tab, int n, double dt, const double *X, double *Xo,
                const double *B, double *J, const double *G, double *K, const double *det, double *U, double *KU, bool cur)
