@@ -328,7 +328,7 @@ __device__ inline bf16x8 join(s16x4 a, s16x4 b)
 
 // Input rows of a tile and y: the points, a row of zeros per grid row begun,
 // and one row on either side
-__host__ __device__ inline int wgrad_rows(int nx) { return WT + (WT - 1) / nx + 3; }
+__host__ __device__ constexpr int wgrad_rows(int nx) { return WT + (WT - 1) / nx + 3; }
 
 // floor(v / n) of 0 <= v < 2^16 with inv = 1 / n: v + 1/2 is at least 1/(2n)
 // away from a multiple of n, relative to the quotient more than the rounding
@@ -396,7 +396,10 @@ __device__ inline void bias_part(const WgradArgs &a, bf16_t *st, int chunk, int 
     }
 }
 
-template <int MCO, int NCI>
+// MINNX: the smallest nx the variant takes, which bounds a tile's rows.  A
+// level's nx is 2 or more (a grid of nx = 5 has levels of 5, 3 and 2); rows
+// nobody stages would hold whatever LDS held before.
+template <int MCO, int NCI, int MINNX>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_wgrad(WgradArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];   // [3][NCI][rows][16] input, [MCO][WT][16] gradient, [3][rows] int
@@ -431,7 +434,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k
     bf16_t *xst = Xs + (sc >> 1) * xn + 8 * (sc & 1);
     constexpr int RS = 32 / NCI;                              // rows a wave stages at a time
     // a tile's words on their way to LDS: loaded while the tile before is multiplied
-    constexpr int NX = (WT + (WT - 1) / 5 + 3 + RS - 1) / RS, NG = (WT * 2 * MCO + 191) / 192;   // grids have nx >= 5
+    constexpr int NX = (wgrad_rows(MINNX) + RS - 1) / RS, NG = (WT * 2 * MCO + 191) / 192;
     u32x4 xv[NX], gv[NG];
     int *const tab = reinterpret_cast<int *>(lds + (3 * NCI * xn + MCO * gn)) + ty * rows;   // the wave's
     auto load = [&](int pb) {
@@ -994,7 +997,10 @@ void launch_wgrad_k(hipStream_t s, const WgradArgs &a, int kpad, float *grad, fl
     const int nbias = (a.cout + BG_CH - 1) / BG_CH;
     WgradArgs w = a;
     w.bpart = a.part + (long long)nch * blocks * 27 * MCO * NCI * 256;
-    k_wgrad<MCO, NCI><<<dim3(nch, 3 * blocks + nbias), 192, lds, s>>>(w);
+    // sized for nx = 2 the staging takes two words a lane more than for nx = 4
+    const dim3 grid(nch, 3 * blocks + nbias);
+    if (a.nx < 4) k_wgrad<MCO, NCI, 2><<<grid, 192, lds, s>>>(w);
+    else k_wgrad<MCO, NCI, 4><<<grid, 192, lds, s>>>(w);
     k_wgrad_sum<MCO, NCI><<<dim3(27 * MCO * NCI * 4 + 1, blocks), 256, 0, s>>>(
         w, nch, kpad, grad, nb, bgrad);
 }

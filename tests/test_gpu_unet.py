@@ -92,6 +92,47 @@ def test_gradient_at_box_edges(g, shape):
         off += n
 
 
+def sparse_case(seed, shape):
+    """Parameters and sample whose sums are exact in FP32: four weights that
+    are powers of two an output channel, multiples of 1/8 and 1/16 as
+    features and targets."""
+    import oracle as o
+    rng = np.random.default_rng(seed)
+    params = []
+    for cin, cout in o.UNET_LAYERS:
+        w = np.zeros((cout, 27 * cin))
+        for co in range(cout):
+            w[co, rng.choice(27 * cin, 4, replace=False)] = rng.choice([-0.5, 0.5, 1.0], 4)
+        params += [w.ravel(), rng.choice([0.0, 0.125, 0.25], cout)]
+    feat = rng.integers(-16, 17, shape + (8,)) / 8.0
+    return np.concatenate(params + [np.array([0.5])]), feat, rng.integers(-16, 17, shape + (3,)) / 16.0
+
+
+# Narrow grids: the coarse levels' nx is 2 or 3 and they hold several tiles of
+# points, so a tile of the weight gradient has more rows than on a wide grid.
+# With sums that are exact in FP32 few roundings to bfloat16 can differ from
+# the oracle's (the pool's thirds and the loss's factor: targets moved by 1e-7
+# change the oracle's gradients by at most 5e-5); the weight gradient's FP32
+# sums have at most 100 steps of 2^-23 over terms that cancel to no less than
+# a fiftieth: 6e-4.  Hence 1e-3.
+@pytest.mark.parametrize("shape", [(17, 17, 5), (33, 33, 5), (25, 25, 9), (49, 9, 9), (65, 33, 9)])
+def test_gradient_on_narrow_grids(g, shape):
+    import oracle as o
+    params, feat, target = sparse_case(22, shape)
+    with g.UNet(shape[2], shape[1], shape[0]) as u:
+        u.set_params(params)
+        loss, grad = u.loss_grad(feat, target)
+        loss2, grad2 = u.loss_grad(feat, target)
+    assert loss == loss2 and np.array_equal(grad, grad2)
+    l_r, _, g_r = o.unet_loss(params, feat, target, round_bf16=True)
+    assert abs(loss - l_r) < 1e-3 * l_r
+    off = 0
+    for l, (cin, cout) in enumerate(o.UNET_LAYERS):
+        n = cout * 27 * cin + cout
+        assert relerr(grad[off:off + n], g_r[off:off + n]) < 1e-3, l
+        off += n
+
+
 def relaxed_braid(g, n, steps):
     """A braid on an (n, n, 2n-1) grid relaxed by `steps` attempts (F32K)."""
     p = small_braid(n, n, 2 * n - 1)
