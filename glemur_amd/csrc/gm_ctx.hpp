@@ -114,8 +114,10 @@ struct gm_ctx {
     int TX[7] = {}, TY[7] = {}, tiles_x[7] = {}, tiles_y[7] = {};
     int CZ[7] = {}, nchunks[7] = {}, nblocks[7] = {};
     // stage kernels that compute blocks at once instead of marching their
-    // tile (small grids; off once a caller sets tiles)
+    // tile (small grids; off once a caller sets tiles, and always in the
+    // members of an ensemble, whose launches march)
     bool block[6] = {};
+    bool member = false;
     int BX = 0, BY = 0, BZ = 0;   // the block
     int ncu = 256;
     EvTimer tm;                   // kernel timing (gm_timing_*)

@@ -165,7 +165,7 @@ double rect_lines(int tlx, int tly, int rw, int rh)
 // workgroups per CU, while its loads were issued one plane step ahead; with
 // two steps it is faster on the wide rects: 98 -> 92 us at 129 x 129 x 385.)
 void auto_blocks(gm_ctx *c);
-void auto_tiles(gm_ctx *c, int target, bool member)
+void auto_tiles(gm_ctx *c, int target)
 {
     const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
     const bool lines = c->prec == GM_PREC_F32K;
@@ -186,7 +186,7 @@ void auto_tiles(gm_ctx *c, int target, bool member)
         const int nch = best_chunks(nz, c->tiles_x[k] * c->tiles_y[k], target * stage_blocks_per_cu(c, k));
         set_tile_k(c, k, bx, by, (nz + nch - 1) / nch);
     }
-    if (!member) auto_blocks(c);   // ensemble launches march
+    if (!c->member) auto_blocks(c);   // ensemble launches march
 }
 
 int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -480,7 +480,7 @@ extern "C" int gm_create(const gm_params *pp, int precision, gm_ctx **out)
         hipDeviceProp_t pr;
         c->ncu = hipGetDeviceProperties(&pr, c->device) == hipSuccess ? pr.multiProcessorCount : 256;
     }
-    auto_tiles(c, default_blocks(c), false);
+    auto_tiles(c, default_blocks(c));
     if ((r = ensure_partials(c))) return bail(r);
     if ((r = push_ctl(c))) return bail(r);
     *out = c;
@@ -1213,7 +1213,7 @@ extern "C" int gm_set_tile(gm_ctx *c, int tx, int ty, int cz)
     if (!c) return fail(GM_ERR_ARG, "null context");
     if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
     if (tx <= 0 || ty <= 0) {
-        auto_tiles(c, cz > 0 ? cz : default_blocks(c), false);
+        auto_tiles(c, cz > 0 ? cz : default_blocks(c));
         return ensure_partials(c);
     }
     if ((tx + 4) * (ty + 4) > gmd::fused_max_points(c->prec == GM_PREC_F32K))
@@ -1533,8 +1533,8 @@ int batch_prepare(gm_batch *b)
         K.ctl = c->ctl;
         K.part_delta = c->part_delta;
         K.part_diag = c->part_diag;
-        K.nb_delta = c->nblocks[5];
-        K.nb_diag = c->nblocks[0];
+        K.nb_delta = launch_blocks(c, 5);
+        K.nb_diag = launch_blocks(c, 0);
         K.diag = 1;
         K.nbuf = b->f64 ? 3 : 2;
         K.maxError = c->p.maxError;
@@ -1615,7 +1615,8 @@ extern "C" int gm_batch_create(const gm_params *params, int n, int precision, gm
                                                  "run the per-kernel path"));
         c->zrev = false;   // the members together move several GB per stage
         c->zalt = false;
-        auto_tiles(c, std::max(1, (c->ncu + n - 1) / n), true);
+        c->member = true;
+        auto_tiles(c, std::max(1, (c->ncu + n - 1) / n));
         b->ctlh.push_back(c->ctlh);
     }
     b->press = params[0].pressure ? 1 : 0;

@@ -148,6 +148,36 @@ def test_default_tiles_mix_workgroup_sizes(g):
             assert abs(r.energy - q.energy) <= 1e-12 * abs(q.energy), i
 
 
+@pytest.mark.parametrize("prec", ["F32K", "F64"])
+def test_members_with_automatic_tiles_set_again(g, prec):
+    """set_tile(0, 0, n) on members of a small-grid ensemble picks marching
+    tiles again: the controller joins the partials of the launch that wrote
+    them, so every member still takes its standalone run's attempts (the
+    energy is the same sum in another order)."""
+    pr = getattr(g, "PREC_" + prec)
+    ps = [small_braid(33, 33, 97), small_braid(17, 19, 23)]
+    for p in ps:
+        p.nCycle = 10 ** 6
+    states = [g.init_state(p) for p in ps]
+    with g.Batch(ps, pr) as b:
+        for m, (B0, xb), n in zip(b.members, states, (0, 40)):
+            m.set_tile(0, 0, n)
+            m.upload(B0, xb, 0.0, 0.01)
+        b.run(max_attempts=12, batch=6)
+        got = [(m.time(), m.download(g.FIELD_XB), m.step_log(12)) for m in b.members]
+    for (t, x, log), p, (B0, xb) in zip(got, ps, states):
+        with g.Context(p, pr) as c:
+            c.upload(B0, xb, 0.0, 0.01)
+            c.run(max_attempts=12, batch=6)
+            assert t == c.time() and np.array_equal(x, c.download(g.FIELD_XB))
+            want = c.step_log(12)
+        assert len(log) == len(want) == 12
+        for r, q in zip(log, want):
+            assert (r.maxDelta, r.dt_used, r.accepted, r.ratio, r.ratio_pt, r.jxb_b2, r.jmax) == \
+                   (q.maxDelta, q.dt_used, q.accepted, q.ratio, q.ratio_pt, q.jxb_b2, q.jmax)
+            assert abs(r.energy - q.energy) <= 1e-12 * abs(q.energy)
+
+
 # ------------------------------------------------------------------ FP64
 
 def f64_members(**kw):
