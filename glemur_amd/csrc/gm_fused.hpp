@@ -64,8 +64,8 @@ struct CtlArgs {
     Ctl *mirror;                      // pinned copy of the block after the attempt (may be null)
 };
 
-// Start of a run: n_cycle accepted steps and attempts more from here (<= 0:
-// no limit)
+// Start of a run: n_cycle accepted steps (<= 0: none are left, the run ends
+// with its first attempt) and attempts more from here
 struct ArmArgs {
     Ctl *ctl;
     double stop_ratio, ev_dump, ev_save;

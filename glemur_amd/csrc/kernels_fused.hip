@@ -1281,8 +1281,8 @@ __global__ void k_arm(ArmArgs A)
     h.stop_ratio = A.stop_ratio;
     h.ev_dump = A.ev_dump;
     h.ev_save = A.ev_save;
-    h.n_cycle = A.n_cycle > 0 ? h.n_accept + A.n_cycle : 1LL << 62;
-    h.max_attempt = A.attempts > 0 ? h.n_attempt + A.attempts : 1LL << 62;
+    h.n_cycle = h.n_accept + A.n_cycle;
+    h.max_attempt = h.n_attempt + A.attempts;
 }
 
 // The host's control block and the record of an attempt, by value

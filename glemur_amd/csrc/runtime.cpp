@@ -1086,7 +1086,7 @@ extern "C" int gm_step(gm_ctx *c, gm_step_info *info)
     if (!pk)
         if (int r = check_fused(c)) return r;
     int r;
-    gmd::launch_arm(c->stream, {c->ctl, 0, 0, 0, 0, 0, 0});
+    gmd::launch_arm(c->stream, {c->ctl, 0, 0, 0, 1LL << 62, 1LL << 62, 0});   // one attempt, no limits
     if (pk) {
         if ((r = sync_ctl(c)) || (r = step_per_kernel(c))) return r;
     } else {
