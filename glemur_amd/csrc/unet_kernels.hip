@@ -449,6 +449,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k
             const int p = x + a.nx * (rb + q - 1 + ty - 1 + (tz - 1) * a.ny);
             tab[r] = x < a.nx && y >= 0 && y < a.ny && p >= 0 && p < P ? p : -1;
         }
+        // a lane reads what other lanes of its wave wrote: LDS serves a wave in
+        // order, the fence keeps the compiler from moving the reads up
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         int p[NX];
 #pragma unroll
         for (int u = 0; u < NX; ++u) p[u] = tab[min(sr + u * RS, rows - 1)];
