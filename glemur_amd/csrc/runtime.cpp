@@ -1338,8 +1338,9 @@ constexpr double kTuneKeep = 0.98;
 
 }  // namespace
 
-// Per stage kernel: time `reps` launches of each candidate tile on the
-// current state and keep the fastest (by the keep margin).  The stage
+// Per stage kernel: time `reps` launches of the tile in force and of each
+// candidate tile on the current state and keep the fastest (by the keep
+// margin).  The stage
 // kernels alone write only the slope buffers and the candidate position
 // buffer, so the accepted state, t and dt are unchanged.
 extern "C" int gm_autotune(gm_ctx *c, int reps, double ms_best[6])
@@ -1372,7 +1373,12 @@ extern "C" int gm_autotune(gm_ctx *c, int reps, double ms_best[6])
             ms = t / reps;
             return GM_OK;
         };
-        if (k < 6 && c->block[k] && (rc = timed(block_ms))) break;
+        if (k < 6 && c->block[k]) {
+            if ((rc = timed(block_ms))) break;
+            c->block[k] = false;
+        }
+        // the marching tile in force first: a candidate has to beat it
+        if ((rc = ensure_partials(c)) || (rc = timed(best))) break;
         // per workgroup size: the fewest-points rect and, for F32K, the
         // fewest-lines one
         std::vector<std::pair<int, int>> rects;
@@ -1393,7 +1399,7 @@ extern "C" int gm_autotune(gm_ctx *c, int reps, double ms_best[6])
             const int cols = c->tiles_x[k] * c->tiles_y[k], slots = c->ncu * stage_blocks_per_cu(c, k);
             int cand[3] = {best_chunks(c->p.nz, cols, slots), slots / cols, 2 * slots / cols};
             for (int q = 0; q < 3; ++q) {
-                const int nch = cand[q] = std::max(1, std::min(cand[q], std::max(1, c->p.nz / 8)));
+                const int nch = cand[q] = std::max(1, std::min(cand[q], c->p.nz / 2));   // as best_chunks
                 bool seen = false;
                 for (int r = 0; r < q; ++r) seen |= cand[r] == nch;
                 if (seen) continue;

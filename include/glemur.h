@@ -368,12 +368,12 @@ int gm_get_stage_tile(gm_ctx *ctx, int stage, int *tx, int *ty, int *cz, int *nb
  * (tx+4)(ty+4) must fit the stage kernel's largest workgroup. */
 int gm_set_stage_tile(gm_ctx *ctx, int stage, int tx, int ty, int cz);
 /* Tile autotuner (no reference counterpart): for every stage kernel, times
- * `reps` launches of each candidate rect (the fewest-loads rect for each
- * workgroup size the kernel is built for, with one or two rounds of
- * workgroups over the CUs) on the current state and keeps the fastest (a
- * later candidate must be more than 2% faster to replace an earlier one);
- * ms_best (6 entries, or NULL) receives the kept tiles' mean times.  The
- * accepted state, t and dt are unchanged. */
+ * `reps` launches of the tile in force and of each candidate rect (the
+ * fewest-loads rect for each workgroup size the kernel is built for, with
+ * one or two rounds of workgroups over the CUs) on the current state and
+ * keeps the fastest (a later candidate must be more than 2% faster to
+ * replace an earlier one); ms_best (6 entries, or NULL) receives the kept
+ * tiles' mean times.  The accepted state, t and dt are unchanged. */
 int gm_autotune(gm_ctx *ctx, int reps, double ms_best[6]);
 
 /* ---- files (src/io.cu) ------------------------------------------------ */

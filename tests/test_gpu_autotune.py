@@ -46,6 +46,32 @@ def test_autotune_keeps_state_and_trajectory(g, prec):
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
+def test_autotune_keeps_a_faster_tile_in_force(g):
+    """141 x 141 x 31 with pressure in F32K runs on chunks of six planes by
+    default; tuned, an attempt takes no longer (the keep margin is 2%, the
+    fastest of eight runs of 40 attempts varies by 1 to 2%: 8%).  With no
+    chunk thinner than an eighth of the grid's planes it took 17% longer."""
+    import time
+    p = small_braid(141, 141, 31, pressure=True, beta=0.05)
+    p.nCycle = 10 ** 6
+    B0, xb = g.init_state(p)
+    with g.Context(p, g.PREC_F32K) as c:
+        def fastest():
+            ts = []
+            for _ in range(8):
+                c.upload(B0, xb, 0.0, 1e-3)
+                t0 = time.perf_counter()
+                c.run(max_attempts=40, batch=8)
+                ts.append(time.perf_counter() - t0)
+            return min(ts)
+        fastest()
+        before = fastest()
+        c.autotune(reps=5)
+        after = fastest()
+    print(f"an attempt {before / 40 * 1e6:.1f} us by default, {after / 40 * 1e6:.1f} us tuned")
+    assert after <= 1.08 * before
+
+
 @pytest.mark.parametrize("press", [False, True])
 def test_f32k_workgroup_sizes_give_the_same_trajectory(g, press):
     """F32K stage kernels at every workgroup size they are built for: on a
