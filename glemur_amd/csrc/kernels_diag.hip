@@ -116,7 +116,7 @@ __device__ inline double wave_min(double v)
 // summing their partials serially; what is left is FP64 arithmetic.
 // Partials of a workgroup go to part[q * nb + block], q = energy, |J|max,
 // the four other maxima, convexity, wedge, and the two error sums.
-constexpr int kQ = 10, kRowBlocks = 4096, kEpsRows = 16;
+constexpr int kQ = 10, kRowBlocks = 2048, kEpsRows = 16;
 
 template <class R>
 struct RowArgs {
@@ -126,9 +126,33 @@ struct RowArgs {
     double ar, az, phi1;
     int diag, mesh, errs, eps;
     double *cellVol, *convex, *wedge;
-    int nb, bx, KZ, neps;     // workgroups over points (bx per layer of KZ planes), and of epsilon*
+    int nb, bx, G, KZ, neps;  // workgroups over points (bx per layer of G KZ planes), and of epsilon*
     double *part;
 };
+
+// The columns t, t + bx kB, ... < nx ny and planes [k0, k1) of a thread of
+// workgroup blk.  Where a workgroup has more threads than the grid columns, G
+// groups of them take the planes in turn (2 x 2 x 50000, a row with the mesh and
+// error quantities in FP32: 191 us without, 35 with).
+struct RowPart {
+    int t, k0, k1;
+};
+template <class R>
+__device__ RowPart row_part(const RowArgs<R> &A, int blk)
+{
+    const int layer = blk / A.bx, nxy = A.g.nx * A.g.ny;
+    RowPart p;
+    int sub = 0;
+    p.t = (blk - layer * A.bx) * kB + threadIdx.x;
+    if (A.G > 1) {
+        sub = threadIdx.x / nxy;
+        p.t = sub < A.G ? threadIdx.x - sub * nxy : nxy;
+    }
+    p.k0 = (layer * A.G + sub) * A.KZ;
+    p.k1 = min(p.k0 + A.KZ, A.g.nz);
+    if (p.k0 >= p.k1) p.t = nxy;
+    return p;
+}
 
 template <class R>
 __device__ void eps_star_rows(const RowArgs<R> &A, const R *B, const R *J, int blk)
@@ -172,9 +196,10 @@ template <class R>
 __device__ void errs_block(const RowArgs<R> &A, const R *B, int blk)
 {
     const Geo &g = A.g;
-    const int layer = blk / A.bx, k0 = layer * A.KZ, k1 = min(k0 + A.KZ, g.nz), nxy = g.nx * g.ny;
+    const RowPart part = row_part(A, blk);
+    const int k0 = part.k0, k1 = part.k1, nxy = g.nx * g.ny;
     double e1 = 0, e2 = 0;
-    for (int t = (blk - layer * A.bx) * kB + threadIdx.x; t < nxy; t += A.bx * kB) {
+    for (int t = part.t; t < nxy; t += A.bx * kB) {
         const int j = t / g.nx, i = t - j * g.nx;
         long long a = gidx(g, i + 1, j + 1, k0 + 1);
         const double x = i * g.dx + g.Ox, y = j * g.dy + g.Oy;
@@ -224,11 +249,11 @@ __global__ void __launch_bounds__(kB, sizeof(R) == 8 ? 3 : 4) k_row(RowArgs<R> A
         if (blk >= A.nb) return;
         if (!main || second) return errs_block(A, B, blk);
     }
-    const int layer = blk / A.bx;
     const Geo &g = A.g;
-    const int k0 = layer * A.KZ, k1 = min(k0 + A.KZ, g.nz), nxy = g.nx * g.ny;
+    const RowPart part = row_part(A, blk);
+    const int k0 = part.k0, k1 = part.k1, nxy = g.nx * g.ny;
     double e = 0, jm = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0, cm = 1, wm = 1e300;
-    for (int t = (blk - layer * A.bx) * kB + threadIdx.x; t < nxy; t += A.bx * kB) {
+    for (int t = part.t; t < nxy; t += A.bx * kB) {
         const int j = t / g.nx, i = t - j * g.nx;
         const int bxy = (i == 0) + (j == 0) + (i == g.nx - 1) + (j == g.ny - 1);
         long long a = gidx(g, i + 1, j + 1, k0 + 1);
@@ -331,14 +356,18 @@ int launch_row(hipStream_t s, const Geo &g, const double *x64, const float *xh, 
     if constexpr (sizeof(R) == 8) X.x = x64;
     else X.x = xh;
     RowArgs<R> A{g, X, det, ar, az, phi1, diag, mesh || maps, errs, eps, cellVol, convex, wedge,
-              0, 0, 0, 0, part};
+              0, 0, 0, 0, 0, part};
     // as many planes a thread as leave at most kRowBlocks workgroups: one on
-    // small grids (more workgroups), 7 at 129 x 129 x 385
-    const long long cols = ((long long)g.nx * g.ny + kB - 1) / kB;
+    // small grids (more workgroups), 13 at 129 x 129 x 385.  Twice as many
+    // workgroups keep the kernel that joins their partials busy longer than
+    // they save (a row of 100^3 points in FP32 40 us against 30, 129 x 129 x
+    // 385 67 against 62)
+    const long long nxy = (long long)g.nx * g.ny, cols = (nxy + kB - 1) / kB;
     A.bx = (int)(cols < kRowBlocks ? cols : kRowBlocks);
-    const int layers = kRowBlocks / A.bx;
+    A.G = nxy < kB ? (int)(kB / nxy) : 1;
+    const int layers = kRowBlocks / A.bx * A.G;
     A.KZ = (g.nz + layers - 1) / layers;
-    A.nb = diag || extra ? A.bx * ((g.nz + A.KZ - 1) / A.KZ) : 0;
+    A.nb = diag || extra ? A.bx * ((g.nz + A.G * A.KZ - 1) / (A.G * A.KZ)) : 0;
     A.neps = eps ? (g.nz + kEpsRows - 1) / kEpsRows : 0;
     const bool two = errs && (diag || A.mesh);
     const dim3 grid(A.neps + (two ? 2 * ((A.nb + 7) / 8 * 8) : A.nb));
