@@ -75,8 +75,10 @@ __device__ __forceinline__ void ghost_b(const Geo &g, const GhostPt &G, int face
     else ghost_b_f<2>(g, G, side, xin, B, det);
 }
 
-// floor(v / n) of 0 <= v < 4096, n <= 64 with inv = 1 / n to a few ulp: v + 1/2
-// is 1/(2n) away from a multiple of n, the product's error below 2e-5
+// floor(v / n) of 0 <= v < 2^20, n > 0 with inv = 1 / n to an ulp: (v + 1/2) / n
+// is at least 1/(2n) away from a whole number, and inv's error and the
+// product's rounding move it by at most (v + 1/2) 2^-22 / n, which is less
+// while v + 1/2 < 2^21
 __device__ __forceinline__ int small_div(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
 
 // The points of a block launch a thread computes: output point and face

@@ -888,7 +888,7 @@ k_stage32_batch(const FusedArgs *__restrict__ args, const int *__restrict__ star
 // 8 x 8 x 8), B at the block and its face neighbours (at most NT of them, one a
 // thread).  Every point takes the operations of the march in their order,
 // so the results are its bit for bit; the energy is summed in another order.
-// What bounds it: at 33 x 33 x 97 (225 blocks, one a CU) the chain itself,
+// What bounds it: at 33 x 33 x 97 (252 blocks, one a CU) the chain itself,
 // 4.5 us a stage beside the march's 21 to 27; from a few blocks a CU on the
 // vector instructions (about half of them for halo and face neighbours) and
 // the two blocks a CU that LDS holds: 49 x 49 x 145 stages 1 to 4 26 to 29 ->

@@ -720,10 +720,12 @@ __global__ void __launch_bounds__(NT) k_stage64_batch(const FusedArgs *__restric
 // so the results are the same bit for bit; the energy is summed in another
 // order.  Points beyond a periodic face hold their source's position
 // unshifted and readers shift, as in the march.
-// It needs half the march's registers (122 to 138, no queues along z), so
-// two blocks share a CU.  An attempt at 33 x 33 x 97 285 -> 72 us, at 65 x 65
-// x 193 372 -> 328 us; bound by the FP64 instructions of the block, its ring
-// and its halo there.
+// It needs half the march's registers (no queues along z): without pressure
+// 122 to 126 in stages 1 to 5, so two blocks share a CU; 128 (periodic) and
+// 130 in stage 0, and 136 to 164 with pressure, where a CU holds one (from 129
+// registers on).  An attempt at 33 x 33 x 97 285 -> 72 us, at 65 x 65 x 193
+// 372 -> 324 us; bound by the FP64 instructions of the block, its ring and its
+// halo there.
 template <int NT, int STAGE, bool PRESS, bool PERI>
 __global__ void __launch_bounds__(NT) k_block64(FusedArgs A)
 {

@@ -200,12 +200,22 @@ int launch_blocks(const gm_ctx *c, int k) { return k < 6 && c->block[k] ? num_bl
 // of the march takes 0.75 us (FP32) or 2 us (FP64) however few columns a
 // workgroup holds, so on a small grid a launch lasts its fill of the pipeline;
 // a block costs its halo instead (2.7 to 3 positions and 1.8 B a point).
-// Microseconds an attempt, march -> blocks, F32K and FP64:
+// Microseconds an attempt by stream launches (33 x 33 x 97 as a graph: 45 and
+// 68), march in chunks of eight planes or more -> blocks, F32K and FP64:
 //   33 x 33 x 97     152 -> 51     285 -> 72
 //   49 x 49 x 145    166 -> 93     290 -> 162
-//   61 x 47 x 150    205 -> 160    427 -> 303   (pressure, periodic x and y)
-//   65 x 65 x 193    145 -> 173    372 -> 328   (F32K: chunks of six planes)
+//   61 x 47 x 150    205 -> 143    427 -> 289   (pressure, periodic x and y)
+//   65 x 65 x 193    145 -> 173    372 -> 324   (F32K: chunks of six planes)
 //   81 x 81 x 241    212 -> 289    610 -> 612
+//   600 x 400 x 2    239 -> 168    320 -> 235
+//   300 x 200 x 10   194 -> 147    309 -> 259
+//   129 x 129 x 33   174 -> 142    298 -> 252
+//   100 x 100 x 60   204 -> 174    393 -> 352   (pressure)
+//   2 x 300 x 900    185 -> 157    500 -> 287
+//   2 x 2 x 50000    711 -> 171    3190 -> 306
+// (Chunks of four to six planes come down to the blocks' times near the F32K
+// limit on compact grids, and 4 to 12% below at 129 x 129 x 33 and 100 x 100 x
+// 60, with pressure most.)
 // FP64 stages 1 to 4 alone are still faster at 81 x 81 x 241 (85 to 102 ->
 // 70 to 97 us), stages 0 and 5 not (92 -> 115, 154 -> 163); at 97 x 97 x 289
 // stages 3 and 4 are slower.  Hence the limits, in inner points.

@@ -330,8 +330,9 @@ __device__ inline bf16x8 join(s16x4 a, s16x4 b)
 // and one row on either side
 __host__ __device__ constexpr int wgrad_rows(int nx) { return WT + (WT - 1) / nx + 3; }
 
-// floor(v / n) of 0 <= v < 2^16 with inv = 1 / n: v + 1/2 is at least 1/(2n)
-// away from a multiple of n, relative to the quotient more than the rounding
+// floor(v / n) of 0 <= v < 2^20, n > 0 with inv = 1 / n: (v + 1/2) / n is at
+// least 1/(2n) away from a whole number, the roundings move it by at most
+// (v + 1/2) 2^-22 / n
 __device__ inline int small_div(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
 
 // Bias gradient partials of 4096 points, by workgroups of the weight
