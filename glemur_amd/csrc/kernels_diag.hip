@@ -111,7 +111,7 @@ __device__ inline double wave_min(double v)
 // 8), read once here and three times by a pass per quantity.  A thread
 // marches KZ planes of one column, so its z neighbours stay in registers
 // and the index divisions are done once; the other neighbours hit in cache.
-// 129 x 129 x 385 (FP32, all quantities): 0.19 ms in one launch, 1.9 TB/s,
+// 129 x 129 x 385 (FP32, all quantities): 0.18 ms in one launch, 2.0 TB/s,
 // against 0.6 ms in four launches of 512 workgroups, one wave of them
 // summing their partials serially; what is left is FP64 arithmetic.
 // Partials of a workgroup go to part[q * nb + block], q = energy, |J|max,
